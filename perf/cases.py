@@ -193,6 +193,36 @@ def run(st):
     return C
 
 
+def exact(case, seed):
+    """The product (or the chain of products) of the same inputs in 64 bits, by plain torch; None where whole values come out."""
+    kind = case["kind"]
+    if kind in ("encode", "split_weight", "host_encode"):
+        return None
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(seed)
+    if kind == "stack":  # the layers' weights as decoder_stack draws them
+        h, N = case["hidden"], case["N"]
+        x = torch.randn((N, h), generator=gen, device=dev).half().double()
+        for i in range(case["layers"]):
+            g = torch.Generator(device=dev)
+            g.manual_seed(seed * 64 + i)
+            for M, K, clamp in ((3 * h, h, False), (h, h, False), (4 * h, h, True), (h, 4 * h, False)):
+                W = torch.randn((M, K), generator=g, device=dev).mul_(0.02)
+                W = W.mul_(torch.rand((M, K), generator=g, device=dev) >= case["sparsity"]).half().double()
+                x = x[:, :K] @ W.t()
+                if clamp:
+                    x = x.relu()
+        return x
+    M, N, K, layout = case["M"], case["N"], case["K"], case["layout"]
+    W = _weight(M, K, case["sparsity"], case["skewed"], gen).double()
+    if layout == "row":
+        return W @ torch.randn((K, N), generator=gen, device=dev).half().double()
+    B = torch.randn((N, 3 * K if layout == "strided" else K), generator=gen, device=dev).half()[:, :K].double()
+    C = B @ W.t()
+    return C.relu() if layout == "strided" else C
+
+
 def _csl_bytes(M, K, kept):
     tiles = (M // 128) * (K // 64)
     return 4.0 * M * K * kept + 6.0 * tiles + 4.0 * (tiles + 2)  # words, a tile's padding of 1.5 words, offsets
