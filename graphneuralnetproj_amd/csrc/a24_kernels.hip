@@ -9,8 +9,8 @@
 // accumulator tiles each, fetch their activation fragments from the L2 in operand order, and add
 // up through LDS in wave order at the end (fp32, one rounding to fp16).
 // a24_spmm_shared_b_kernel (the default launch): the waves own rows instead and share each unit's
-// activation tile through LDS.  Also here: the split + pack on the GPU, and the second stream
-// that the two-stream form of the hybrid call uses.
+// activation tile through LDS.  Also here: the second stream that the two-stream form of the
+// hybrid call uses.  (The split + pack on the GPU: a24_pack_device.hip.)
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -845,320 +845,6 @@ extern "C" int a24_launch_spmm(void* stream, const void* packed, const void* B, 
         case 64: return launch_nt<4>(s, packed, B, out, M, N, K, split_k, rb, waves, ldb, ldo, slab);
         default: return static_cast<int>(hipErrorInvalidValue);
     }
-}
-
-// Split and pack on the GPU: the same bits as the host's decompose + pack (a24_pack.cpp), for
-// weights that are already in device memory.  One thread per lane of a record: it reads its row's
-// 4 x 8 columns of the unit, keeps the first two kept values of every group of four
-// (kernel_benchmark/spmm_decompose.h:12-51) in the record and writes the others to the dense
-// residual (when asked for one), zero elsewhere.
-__global__ __launch_bounds__(256) void a24_split_pack_kernel(const uint16_t* __restrict__ A, uint8_t* __restrict__ packed,
-                                                             uint16_t* __restrict__ residual, int K, int units,
-                                                             long records)
-{
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long record = id >> 6;
-    if (record >= records)
-        return;
-    const int L = static_cast<int>(id & 63);
-    // records are numbered ((rb / 8) * units + u) * 8 + rb % 8
-    const long group = record / (static_cast<long>(units) * kGroupBlocks);
-    const int within = static_cast<int>(record - group * units * kGroupBlocks);
-    const int u = within / kGroupBlocks;
-    const long rb = group * kGroupBlocks + within % kGroupBlocks;
-    const size_t row = (size_t)(rb * 16 + (L & 15)) * K + (size_t)u * 128 + (L >> 4) * 8;
-    uint8_t* rec = packed + (size_t)record * kRecordBytes;
-    typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
-    unsigned word = 0;
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-        const u16x8 in = *reinterpret_cast<const u16x8*>(A + row + s * 32);
-        u16x8 rest = {0, 0, 0, 0, 0, 0, 0, 0};
-        unsigned short val[4];
-#pragma unroll
-        for (int half = 0; half < 2; half++) {
-            int pos[2] = {0, 1}, n = 0;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const unsigned short v = in[half * 4 + e];
-                if ((v & 0x7fffu) != 0) {  // compares unequal to zero as a float: NaN counts, -0 does not
-                    if (n < 2)
-                        pos[n] = e;
-                    else
-                        rest[half * 4 + e] = v;
-                    n++;
-                }
-            }
-            unsigned short v0 = 0, v1 = 0;
-            if (n >= 2) {
-                v0 = in[half * 4 + pos[0]];
-                v1 = in[half * 4 + pos[1]];
-            } else if (n == 1) {
-                if (pos[0] == 3) {  // the free slot goes before it
-                    v1 = in[half * 4 + 3];
-                    pos[0] = 2;
-                    pos[1] = 3;
-                } else {
-                    v0 = in[half * 4 + pos[0]];
-                    pos[1] = 3;
-                }
-            } else {
-                pos[0] = 0;
-                pos[1] = 1;
-            }
-            val[half * 2] = v0;
-            val[half * 2 + 1] = v1;
-            word |= static_cast<unsigned>(pos[0]) << (8 * s + 4 * half) | static_cast<unsigned>(pos[1]) << (8 * s + 4 * half + 2);
-        }
-        typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
-        const u16x4 out = {val[0], val[1], val[2], val[3]};
-        *reinterpret_cast<u16x4*>(rec + (s >> 1) * 1024 + L * 16 + (s & 1) * 8) = out;
-        if (residual)
-            *reinterpret_cast<u16x8*>(residual + row + s * 32) = rest;
-    }
-    *reinterpret_cast<unsigned*>(rec + 2048 + L * 4) = word;
-}
-
-// A: row-major M x K fp16 in device memory (M % 16 == 0, K % 128 == 0, checked by the caller);
-// residual may be null.
-extern "C" int a24_launch_split_pack(void* stream, const void* A, void* packed, void* residual, int M, int K)
-{
-    const int units = K / 128;
-    const long records = static_cast<long>(M / 16) * units;
-    const long blocks = (records * 64 + 255) / 256;
-    if (blocks < 1 || blocks > 0x7fffffffL)
-        return static_cast<int>(hipErrorInvalidValue);
-    hipLaunchKernelGGL(a24_split_pack_kernel, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream),
-                       static_cast<const uint16_t*>(A), static_cast<uint8_t*>(packed), static_cast<uint16_t*>(residual), K,
-                       units, records);
-    return static_cast<int>(hipGetLastError());
-}
-
-// The residual lists (a24_format.h) on the GPU, from the dense residual that the split above
-// leaves in device memory: the same words in the same order as the host's pack_residual
-// (a24_pack.cpp).  Three kernels: count per record, scan, emit.  One wave per record: lane L
-// reads columns 32 * (L % 4) .. + 31 of row L / 4, so lane order is the row-major order that the
-// host collects a list in.
-namespace {
-
-constexpr int kMaxListWords = 16 * 128 / 2;  // a residual holds at most two of every four
-
-__device__ __forceinline__ bool residual_kept(unsigned v)
-{
-    return (v & 0x7fffu) != 0;
-}
-
-__device__ __forceinline__ void record_of_list(long list, int units, long& rb, int& u)
-{
-    const long group = list / (static_cast<long>(units) * kGroupBlocks);
-    const int within = static_cast<int>(list - group * units * kGroupBlocks);
-    u = within / kGroupBlocks;
-    rb = group * kGroupBlocks + within % kGroupBlocks;
-}
-
-typedef unsigned short u16x8v __attribute__((ext_vector_type(8)));
-
-__global__ __launch_bounds__(256) void a24_residual_count_kernel(const uint16_t* __restrict__ A2, int K, int units,
-                                                                 long lists, int* __restrict__ offsets)
-{
-    const long list = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (list >= lists)
-        return;
-    const int L = threadIdx.x & 63;
-    long rb;
-    int u;
-    record_of_list(list, units, rb, u);
-    const uint16_t* src = A2 + (size_t)(rb * 16 + (L >> 2)) * K + (size_t)u * 128 + (L & 3) * 32;
-    int n = 0;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const u16x8v v = *reinterpret_cast<const u16x8v*>(src + q * 8);
-#pragma unroll
-        for (int e = 0; e < 8; e++)
-            n += residual_kept(v[e]) ? 1 : 0;
-    }
-    for (int o = 32; o > 0; o >>= 1)
-        n += __shfl_down(n, o);
-    if (L == 0)
-        offsets[list + 1] = n;
-}
-
-// offsets[1..lists] hold the lists' lengths; turn them into running totals (offsets[0] = 0) and
-// report the longest.  One workgroup.  A total beyond what an int holds gives offsets[lists] = -1.
-__global__ __launch_bounds__(1024) void a24_residual_scan_kernel(int* __restrict__ offsets, long lists,
-                                                                 int* __restrict__ longest)
-{
-    __shared__ long long sums[1024];
-    __shared__ int most[1024];
-    const long chunk = (lists + 1023) / 1024;
-    const long lo = threadIdx.x * chunk, hi = lo + chunk < lists ? lo + chunk : lists;
-    long long s = 0;
-    int m = 0;
-    for (long i = lo; i < hi; i++) {
-        const int n = offsets[i + 1];
-        s += n;
-        m = n > m ? n : m;
-    }
-    sums[threadIdx.x] = s;
-    most[threadIdx.x] = m;
-    __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {
-        const long long v = threadIdx.x >= o ? sums[threadIdx.x - o] : 0;
-        const int w = threadIdx.x >= o ? most[threadIdx.x - o] : 0;
-        __syncthreads();
-        sums[threadIdx.x] += v;
-        most[threadIdx.x] = w > most[threadIdx.x] ? w : most[threadIdx.x];
-        __syncthreads();
-    }
-    const bool fits = sums[1023] <= 0x7fffffffLL - 64;
-    long long run = threadIdx.x ? sums[threadIdx.x - 1] : 0;
-    for (long i = lo; i < hi; i++) {
-        run += offsets[i + 1];
-        offsets[i + 1] = fits ? static_cast<int>(run) : (i + 1 == lists ? -1 : 0);
-    }
-    if (threadIdx.x == 0) {
-        offsets[0] = 0;
-        *longest = most[1023];
-    }
-}
-
-// One wave (= one workgroup) per list.
-__global__ __launch_bounds__(64) void a24_residual_emit_kernel(const uint16_t* __restrict__ A2, int K, int units, long lists,
-                                                               const int* __restrict__ offsets, uint32_t* __restrict__ words)
-{
-    __shared__ uint32_t natural[kMaxListWords];  // the list in row-major order, later in its final order
-    __shared__ uint32_t by_bank[kMaxListWords];  // grouped by bank, fullest bank first
-    __shared__ int order[64], count_of[64], start_of[64], used[16], mine[16];
-    const long list = blockIdx.x;
-    const int L = threadIdx.x;
-    long rb;
-    int u;
-    record_of_list(list, units, rb, u);
-    const int row = L >> 2, c0 = (L & 3) * 32;
-    const uint16_t* src = A2 + (size_t)(rb * 16 + row) * K + (size_t)u * 128 + c0;
-    u16x8v v[4];
-    int mine_n = 0;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        v[q] = *reinterpret_cast<const u16x8v*>(src + q * 8);
-#pragma unroll
-        for (int e = 0; e < 8; e++)
-            mine_n += residual_kept(v[q][e]) ? 1 : 0;
-    }
-    int incl = mine_n;  // inclusive scan over the lanes
-    for (int o = 1; o < 64; o <<= 1) {
-        const int t = __shfl_up(incl, o);
-        if (L >= o)
-            incl += t;
-    }
-    const int n = __shfl(incl, 63);
-    const int begin = offsets[list];
-    const int total = offsets[lists];
-    if (total < 0)  // the word count did not fit an int: no offset of this table means anything, nothing is written
-        return;
-    if (list == lists - 1)  // the padding behind the last list
-        words[(size_t)total + L] = 0;
-    if (n == 0 || n > kMaxListWords)  // (more than a residual can hold: not this format's input; nothing is written)
-        return;
-    int at = incl - mine_n;
-    const bool in_order = n <= 64;  // one round: the host leaves such a list as collected
-#pragma unroll
-    for (int q = 0; q < 4; q++)
-#pragma unroll
-        for (int e = 0; e < 8; e++)
-            if (residual_kept(v[q][e])) {
-                const int c = c0 + q * 8 + e;
-                const uint32_t address = row * 256 + ((((c >> 3) ^ row) & 15) << 4) + (c & 7) * 2;
-                const uint32_t w = v[q][e] | address << 16;
-                if (in_order)
-                    words[(size_t)begin + at] = w;
-                else
-                    natural[at] = w;
-                at++;
-            }
-    if (in_order)
-        return;
-    __syncthreads();
-    // lane b looks after bank b: how many words, where they start among the banks sorted by
-    // (count descending, bank ascending), and its words in collected order
-    auto bank_of = [](uint32_t w) { return static_cast<int>(((w >> 16) >> 2) & 63); };
-    int cnt = 0;
-    for (int i = 0; i < n; i++)
-        cnt += bank_of(natural[i]) == L ? 1 : 0;
-    int rank = 0, start = 0;
-    for (int b = 0; b < 64; b++) {
-        const int other = __shfl(cnt, b);
-        const bool before = other > cnt || (other == cnt && b < L);
-        rank += before ? 1 : 0;
-        start += before ? other : 0;
-    }
-    order[rank] = L;
-    count_of[L] = cnt;
-    start_of[L] = start;
-    for (int i = 0, k = start; i < n; i++) {
-        const uint32_t w = natural[i];
-        if (bank_of(w) == L)
-            by_bank[k++] = w;
-    }
-    __syncthreads();
-    // the host's dealing, word by word (a24_pack.cpp: order_by_bank), on one lane
-    if (L == 0) {
-        const int rounds = (n + 63) / 64;
-        for (int r = 0; r < rounds; r++)
-            used[r] = 0;
-        for (int i = 0; i < 64; i++) {
-            const int b = order[i];
-            const int c = count_of[b];
-            if (c == 0)
-                break;
-            for (int r = 0; r < rounds; r++)
-                mine[r] = 0;
-            for (int j = 0; j < c; j++) {
-                int best = -1, best_free = 0;
-                for (int r = 0; r < rounds; r++) {
-                    const int free = (r == rounds - 1 ? n - 64 * (rounds - 1) : 64) - used[r];
-                    if (free > 0 && (best < 0 || mine[r] < mine[best] || (mine[r] == mine[best] && free > best_free))) {
-                        best = r;
-                        best_free = free;
-                    }
-                }
-                natural[best * 64 + used[best]++] = by_bank[start_of[b] + j];
-                mine[best]++;
-            }
-        }
-    }
-    __syncthreads();
-    for (int i = L; i < n; i += 64)
-        words[(size_t)begin + i] = natural[i];
-}
-
-}  // namespace
-
-// A2: row-major M x K fp16 in device memory (M % 128 == 0, K % 128 == 0, checked by the caller).
-// offsets: (M / 16) * (K / 128) + 1 ints; *longest: the longest list's length.
-extern "C" int a24_launch_residual_offsets(void* stream, const void* A2, int M, int K, int* offsets, int* longest)
-{
-    const int units = K / 128;
-    const long lists = static_cast<long>(M / 16) * units;
-    if (lists < 1 || lists > 0x7ffffff0L)
-        return static_cast<int>(hipErrorInvalidValue);
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(a24_residual_count_kernel, dim3((unsigned)((lists + 3) / 4)), dim3(256), 0, s,
-                       static_cast<const uint16_t*>(A2), K, units, lists, offsets);
-    hipLaunchKernelGGL(a24_residual_scan_kernel, dim3(1), dim3(1024), 0, s, offsets, lists, longest);
-    return static_cast<int>(hipGetLastError());
-}
-
-// words: offsets[last] + 64 of them (the last 64 are zeroed).
-extern "C" int a24_launch_residual_words(void* stream, const void* A2, int M, int K, const int* offsets, void* words)
-{
-    const int units = K / 128;
-    const long lists = static_cast<long>(M / 16) * units;
-    if (lists < 1 || lists > 0x7ffffff0L)
-        return static_cast<int>(hipErrorInvalidValue);
-    hipLaunchKernelGGL(a24_residual_emit_kernel, dim3((unsigned)lists), dim3(64), 0, static_cast<hipStream_t>(stream),
-                       static_cast<const uint16_t*>(A2), K, units, lists, offsets, static_cast<uint32_t*>(words));
-    return static_cast<int>(hipGetLastError());
 }
 
 // A second stream per caller stream, so that the residual's Tiled-CSL kernel can run beside the 2:4

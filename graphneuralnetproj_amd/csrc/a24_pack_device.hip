@@ -1,0 +1,437 @@
+// A weight that is in device memory becomes 2:4 records, a dense residual and the residual's lists
+// of words (layouts: a24_format.h), with the same bits as the host functions in a24_pack.cpp.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "offset_scan.h"
+
+namespace {
+constexpr int kRecordBytes = 2304;
+constexpr int kGroupBlocks = 8;  // records of eight row blocks are stored together, unit by unit
+}  // namespace
+
+// Split and pack on the GPU: the same bits as the host's decompose + pack (a24_pack.cpp), for
+// weights that are already in device memory.  One thread per lane of a record: it reads its row's
+// 4 x 8 columns of the unit, keeps the first two kept values of every group of four
+// (kernel_benchmark/spmm_decompose.h:12-51) in the record and writes the others to the dense
+// residual (when asked for one), zero elsewhere.
+__global__ __launch_bounds__(256) void a24_split_pack_kernel(const uint16_t* __restrict__ A, uint8_t* __restrict__ packed,
+                                                             uint16_t* __restrict__ residual, int K, int units,
+                                                             long records)
+{
+    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long record = id >> 6;
+    if (record >= records)
+        return;
+    const int L = static_cast<int>(id & 63);
+    // records are numbered ((rb / 8) * units + u) * 8 + rb % 8
+    const long group = record / (static_cast<long>(units) * kGroupBlocks);
+    const int within = static_cast<int>(record - group * units * kGroupBlocks);
+    const int u = within / kGroupBlocks;
+    const long rb = group * kGroupBlocks + within % kGroupBlocks;
+    const size_t row = (size_t)(rb * 16 + (L & 15)) * K + (size_t)u * 128 + (L >> 4) * 8;
+    uint8_t* rec = packed + (size_t)record * kRecordBytes;
+    typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
+    unsigned word = 0;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const u16x8 in = *reinterpret_cast<const u16x8*>(A + row + s * 32);
+        u16x8 rest = {0, 0, 0, 0, 0, 0, 0, 0};
+        unsigned short val[4];
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+            int pos[2] = {0, 1}, n = 0;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const unsigned short v = in[half * 4 + e];
+                if ((v & 0x7fffu) != 0) {  // compares unequal to zero as a float: NaN counts, -0 does not
+                    if (n < 2)
+                        pos[n] = e;
+                    else
+                        rest[half * 4 + e] = v;
+                    n++;
+                }
+            }
+            unsigned short v0 = 0, v1 = 0;
+            if (n >= 2) {
+                v0 = in[half * 4 + pos[0]];
+                v1 = in[half * 4 + pos[1]];
+            } else if (n == 1) {
+                if (pos[0] == 3) {  // the free slot goes before it
+                    v1 = in[half * 4 + 3];
+                    pos[0] = 2;
+                    pos[1] = 3;
+                } else {
+                    v0 = in[half * 4 + pos[0]];
+                    pos[1] = 3;
+                }
+            } else {
+                pos[0] = 0;
+                pos[1] = 1;
+            }
+            val[half * 2] = v0;
+            val[half * 2 + 1] = v1;
+            word |= static_cast<unsigned>(pos[0]) << (8 * s + 4 * half) | static_cast<unsigned>(pos[1]) << (8 * s + 4 * half + 2);
+        }
+        typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
+        const u16x4 out = {val[0], val[1], val[2], val[3]};
+        *reinterpret_cast<u16x4*>(rec + (s >> 1) * 1024 + L * 16 + (s & 1) * 8) = out;
+        if (residual)
+            *reinterpret_cast<u16x8*>(residual + row + s * 32) = rest;
+    }
+    *reinterpret_cast<unsigned*>(rec + 2048 + L * 4) = word;
+}
+
+// A: row-major M x K fp16 in device memory (M % 16 == 0, K % 128 == 0, checked by the caller);
+// residual may be null.
+extern "C" int a24_launch_split_pack(void* stream, const void* A, void* packed, void* residual, int M, int K)
+{
+    const int units = K / 128;
+    const long records = static_cast<long>(M / 16) * units;
+    const long blocks = (records * 64 + 255) / 256;
+    if (blocks < 1 || blocks > 0x7fffffffL)
+        return static_cast<int>(hipErrorInvalidValue);
+    hipLaunchKernelGGL(a24_split_pack_kernel, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const uint16_t*>(A), static_cast<uint8_t*>(packed), static_cast<uint16_t*>(residual), K,
+                       units, records);
+    return static_cast<int>(hipGetLastError());
+}
+
+// The residual lists on the GPU, from the dense residual that the split above leaves in device
+// memory: the same words in the same order as the host's pack_residual (a24_pack.cpp).  Three
+// kernels: count per list, scan, emit.
+namespace {
+
+constexpr int kMaxListWords = 16 * 128 / 2;  // a residual holds at most two of every four
+
+__device__ __forceinline__ bool residual_kept(unsigned v)
+{
+    return (v & 0x7fffu) != 0;
+}
+
+// Words per list into offsets[list + 1].  Bound by HBM (the residual is read once).  A wave takes the
+// 16 rows of up to four consecutive units: sixteen loads of one contiguous KiB each, all in flight
+// together.  (One list per wave, 64 bytes per lane: a load instruction touched 32 half lines and a
+// 21504 x 7168 residual of 308 MB took 105 us; now 73.)  Workgroups run from the matrix's end to its
+// start, and the emit kernel from start to end: each begins with what the kernel before it left in
+// the last-level cache.
+__global__ __launch_bounds__(256) void a24_residual_count_kernel(const uint16_t* __restrict__ A2, int K, int units,
+                                                                 unsigned tasks, int* __restrict__ offsets)
+{
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    const unsigned task = (gridDim.x - 1 - blockIdx.x) * 4 + (threadIdx.x >> 6);
+    if (task >= tasks)
+        return;
+    const int L = threadIdx.x & 63;
+    const unsigned spans = (units + 3) / 4;
+    const unsigned rb = task / spans;
+    const int u = static_cast<int>(task % spans) * 4 + (L >> 4);
+    int n = 0;
+    if (u < units) {
+        const uint16_t* src = A2 + (size_t)rb * 16 * K + (size_t)u * 128 + (L & 15) * 8;
+        u32x4 v[16];
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+            v[r] = *reinterpret_cast<const u32x4*>(src + (size_t)r * K);
+        u16x2 c = {0, 0};
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const u16x2 mag = __builtin_bit_cast(u16x2, v[r][i] & 0x7fff7fffu);
+                c += __builtin_elementwise_min(mag, u16x2{1, 1});
+            }
+        n = c[0] + c[1];
+    }
+    for (int o = 8; o > 0; o >>= 1)
+        n += __shfl_xor(n, o);
+    if ((L & 15) == 0 && u < units)
+        offsets[((size_t)(rb / kGroupBlocks) * units + u) * kGroupBlocks + rb % kGroupBlocks + 1] = n;
+}
+
+// offsets[1..lists] hold the lists' lengths; turn them into running totals (offsets[0] = 0) and
+// report the longest.  One workgroup.  A total beyond what an int holds gives offsets[lists] = -1.
+__global__ __launch_bounds__(offscan::kThreads) void a24_residual_scan_kernel(int* __restrict__ offsets, long lists,
+                                                                              int* __restrict__ longest)
+{
+    int most;
+    const long long total = offscan::scan_in_place(offsets + 1, lists, most);
+    const bool fits = total <= 0x7fffffffLL - 64;
+    if (!fits) {
+        __syncthreads();
+        offscan::clear_counts(offsets + 1, lists);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        if (!fits)
+            offsets[lists] = -1;
+        offsets[0] = 0;
+        *longest = most;
+    }
+}
+
+// The words.  Bound by instruction issue and by the dealing below; the residual is read once.
+//
+// In a list's order (a24_pack.cpp: order_by_bank) the words of one LDS bank are neighbours: banks by
+// (count descending, number ascending), a bank's words as collected.  A bank's words come from 16
+// known column pairs, one per row (row r: pair bank ^ (r << 2)), so lane b of a list's wave reads
+// bank b's 32 candidates itself, a whole 256-byte row per load, and knows its count, its place
+// among the banks (six ballots) and its words without any exchange.  Where a word goes is then
+// the result of dealing the banks' words to the rounds one by one, each word depending on the one
+// before; it depends on the counts alone, so one LANE deals for one list: 32 lists of a workgroup
+// side by side (one lane of one wave dealing for the wave's only list took 1150 us on the
+// 21504 x 7168 residual of a 60 % sparse weight; now 138).  A list of at most 64 words stays in
+// row-major order, as the host leaves it.
+//
+// So many workgroups per compute unit as the dealing waves need to hide each other: 256 threads, 18.5
+// KiB of LDS, 64 registers (lists beyond four rounds spill a few), the residual read a second time for
+// the writing (from the last-level cache) instead of kept in registers.  (Eight waves with 51 KiB, registers kept, words placed as 16-bit numbers: 211 us.
+// Dealing by laps, every round with room one word in the order of its room, four keys sorted per lap:
+// 302 us instead of 211, the lanes diverge.)
+constexpr int kEmitWaves = 4, kEmitLists = 32, kListsPerWave = kEmitLists / kEmitWaves;
+constexpr int kPlaces = 8192;  // bytes: 32 lists of 256 words (an ordinary residual has up to 200) are dealt in one pass
+
+// A word of the bank-sorted sequence goes to the round that has the fewest words of its bank, then
+// the most room, then the lowest number: the largest of keys (63 - words of the bank, room - 1, last -
+// round), zero for a full round.  For a list of at most four rounds the lower two fields are one
+// byte, the word's place in code; for longer lists the place is written as two bytes.
+__device__ __forceinline__ int place_bytes(int n)
+{
+    return n <= 256 ? n : 2 * n;
+}
+__device__ __forceinline__ int place_of(const uint8_t* places, int p, int n)
+{
+    if (n > 256)
+        return places[p] | places[p + n] << 8;
+    const int code = places[p];
+    const int end = 256 - 64 * (code & 3);  // 64 * (round + 1)
+    return (end < n ? end : n) - 1 - (code >> 2);
+}
+
+// Deals one list of n words, 64 < n <= 64 * R, whose banks hold counts[0] >= counts[1] >= ... words.
+template<int R>
+__device__ __forceinline__ void deal(const unsigned* counts, int n, uint8_t* places)
+{
+    constexpr int kRoundBits = R <= 4 ? 2 : 4, kLast = (1 << kRoundBits) - 1;
+    constexpr unsigned kRoom = 1u << kRoundBits, kOne = 64u << kRoundBits;  // units of the two upper fields
+    unsigned key[R];
+    const int rounds = (n + 63) >> 6;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int room = r < rounds - 1 ? 64 : (r == rounds - 1 ? n - 64 * (rounds - 1) : 0);
+        key[r] = room > 0 ? 63 * kOne + (room - 1) * kRoom + (kLast - r) : 0u;
+    }
+    unsigned four = counts[0];
+    for (int k = 0; k < 16 && four != 0; k++) {
+        const unsigned next = k < 15 ? counts[k + 1] : 0u;
+        for (; four != 0; four >>= 8) {  // (largest first: once a byte is zero all that follow are)
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                key[r] = key[r] ? (key[r] & (kOne - 1)) | 63 * kOne : 0u;
+            for (int c = four & 0xffu; c > 0; c--, places++) {
+                unsigned best = key[0];
+#pragma unroll
+                for (int r = 1; r < R; r++)
+                    best = key[r] > best ? key[r] : best;
+                const unsigned room = best & (kOne - kRoom);  // minus one
+                if constexpr (R <= 4) {
+                    *places = static_cast<uint8_t>(best);
+                } else {
+                    const int end = 1024 - 64 * static_cast<int>(best & kLast);
+                    const int place = (end < n ? end : n) - 1 - static_cast<int>(room / kRoom);
+                    places[0] = static_cast<uint8_t>(place);
+                    places[n] = static_cast<uint8_t>(place >> 8);
+                }
+                const unsigned then = room == 0 ? 0u : best - kOne - kRoom;
+#pragma unroll
+                for (int r = 0; r < R; r++)
+                    key[r] = key[r] == best ? then : key[r];
+            }
+        }
+        four = next;
+    }
+}
+
+__global__ __launch_bounds__(kEmitWaves * 64, 8) void a24_residual_emit_kernel(const uint16_t* __restrict__ A2, int K, int units,
+                                                                               long lists, const int* __restrict__ offsets,
+                                                                               uint32_t* __restrict__ words)
+{
+    __shared__ unsigned images[kEmitWaves][8 * 64];  // per wave: half of a list's block, [row][bank] column pairs
+    __shared__ unsigned sorted[kEmitLists][17];      // counts of a list's banks, one byte each, largest first
+    __shared__ int length[kEmitLists];
+    __shared__ uint8_t places[kPlaces];
+    const int L = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int total = offsets[lists];
+    if (total < 0)  // the word count did not fit an int: no offset of this table means anything, nothing is written
+        return;
+    if (blockIdx.x == 0 && w == 0)  // the padding behind the last list
+        words[(size_t)total + L] = 0;
+    unsigned* const image = images[w];
+
+    // wave w takes the workgroup's lists w, w + 4, ...
+    auto list_of = [&](int i) { return (long)blockIdx.x * kEmitLists + i * kEmitWaves + w; };
+    auto load_list = [&](long list, unsigned (&pairs)[16]) {
+        const unsigned unit_row = static_cast<unsigned>(list / kGroupBlocks);  // (128-row group, unit)
+        const unsigned group = unit_row / units, u = unit_row % units;
+        size_t block = ((size_t)group * kGroupBlocks + list % kGroupBlocks) * 16 * K + (size_t)u * 128;
+        int lane = L;
+        // (opaque: else the compiler issues the loads of all lists ahead of the first one's use, 300 registers)
+        asm volatile("" : "+s"(block), "+v"(lane)::"memory");
+        const uint16_t* src = A2 + block;
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+            pairs[r] = *reinterpret_cast<const unsigned*>(src + (size_t)r * K + 2 * (lane ^ (r << 2)));
+    };
+    unsigned kept[kListsPerWave];  // bit 2 r + h: element h of row r's pair
+    int start[kListsPerWave];      // where the bank's words begin in the bank-sorted sequence
+
+    // 1. counts of the banks, their order; lists of one round are written at once
+#pragma unroll
+    for (int i = 0; i < kListsPerWave; i++) {
+        const long list = list_of(i);
+        const int li = i * kEmitWaves + w;
+        kept[i] = 0;
+        start[i] = 0;
+        if (list >= lists) {
+            if (L == 0)
+                length[li] = 0;
+            continue;
+        }
+        unsigned pairs[16];
+        load_list(list, pairs);
+        unsigned mask = 0;
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+            mask |= (residual_kept(pairs[r]) ? 1u << (2 * r) : 0u) | (residual_kept(pairs[r] >> 16) ? 2u << (2 * r) : 0u);
+        kept[i] = mask;
+        const int count = __popc(mask);
+        // the banks with more words, and those with as many and a lower number, bit by bit
+        uint64_t more = 0, equal = ~0ull, planes[6];
+        int n = 0;
+#pragma unroll
+        for (int bit = 5; bit >= 0; bit--) {
+            const bool set = (count >> bit) & 1;
+            planes[bit] = __ballot(set);
+            n += __popcll(planes[bit]) << bit;
+            more |= set ? 0ull : equal & planes[bit];
+            equal &= set ? planes[bit] : ~planes[bit];
+        }
+        const uint64_t before = more | (equal & ((1ull << L) - 1));
+        int s = 0;
+#pragma unroll
+        for (int bit = 0; bit < 6; bit++)
+            s += __popcll(before & planes[bit]) << bit;
+        start[i] = s;
+        reinterpret_cast<uint8_t*>(sorted[li])[__popcll(before)] = static_cast<uint8_t>(count);
+        // (a block with more kept values than a residual can hold is not this format's input: nothing is written)
+        const bool dealt = n > 64 && n <= kMaxListWords;
+        if (L == 0)
+            length[li] = dealt ? n : 0;
+        if (n > 0 && n <= 64) {  // in row-major order
+            int at = offsets[list];
+#pragma unroll
+            for (int half = 0; half < 2; half++) {
+#pragma unroll
+                for (int r = 0; r < 8; r++)
+                    image[r * 64 + L] = pairs[half * 8 + r];
+                asm volatile("" ::: "memory");  // other lanes' words are read below
+                for (int r8 = 0; r8 < 8; r8++) {
+                    const int r = half * 8 + r8;
+                    const unsigned pair = image[r8 * 64 + (L ^ (r << 2))];  // columns 2 L and 2 L + 1
+                    const bool lo = residual_kept(pair), hi = residual_kept(pair >> 16);
+                    const uint64_t los = __ballot(lo), his = __ballot(hi), below = (1ull << L) - 1;
+                    const int place = at + __popcll(los & below) + __popcll(his & below);
+                    const unsigned address = r * 256 + (((L >> 2) ^ r) << 4) + (L & 3) * 4;
+                    if (lo)
+                        words[(size_t)place] = (pair & 0xffffu) | address << 16;
+                    if (hi)
+                        words[(size_t)place + (lo ? 1 : 0)] = pair >> 16 | (address + 2) << 16;
+                    at += __popcll(los) + __popcll(his);
+                }
+                asm volatile("" ::: "memory");
+            }
+        }
+    }
+    __syncthreads();
+
+    // 2. deal as many of the lists as there is room for (all of them, but for very dense ones), 3. write them
+    const int mine = L < kEmitLists ? length[L] : 0;
+    const int through = offscan::wave_inclusive_sum(mine > 0 ? place_bytes(mine) : 0);  // room for lists 0 .. L
+    for (int first = 0, dealt = 0; first < kEmitLists;) {
+        const uint64_t fit = __ballot(L < kEmitLists && through - dealt <= kPlaces);  // 0 .. last - 1: totals only grow
+        const int last = __popcll(fit);
+        const int at = through - place_bytes(mine) - dealt;
+        if (w == 0 && L >= first && L < last && mine > 0) {
+            if (mine > 256)  // (lane by lane: the form of a list's places goes by its own length)
+                deal<16>(sorted[L], mine, places + at);
+            else if (__any(mine > 192))
+                deal<4>(sorted[L], mine, places + at);
+            else
+                deal<3>(sorted[L], mine, places + at);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kListsPerWave; i++) {
+            const int li = i * kEmitWaves + w;
+            const int n = __builtin_amdgcn_readlane(mine, li);
+            if (li < first || li >= last || n == 0)
+                continue;
+            unsigned pairs[16];
+            load_list(list_of(i), pairs);
+            const uint8_t* const list_places = places + __builtin_amdgcn_readlane(at, li);
+            uint32_t* const out = words + (size_t)offsets[list_of(i)];
+            int p = start[i];
+#pragma unroll
+            for (int half = 0; half < 2; half++) {
+#pragma unroll
+                for (int r = 0; r < 8; r++)
+                    image[r * 64 + L] = pairs[half * 8 + r];
+                asm volatile("" ::: "memory");
+                for (unsigned mask = kept[i] >> (16 * half) & 0xffffu; mask; mask &= mask - 1, p++) {
+                    const int e = __ffs(static_cast<int>(mask)) - 1;
+                    const unsigned address = (e >> 1) * 256 + L * 4 + (e & 1) * 2;  // in the half image as in the kernel's own
+                    const unsigned value = *reinterpret_cast<const unsigned short*>(reinterpret_cast<const uint8_t*>(image) + address);
+                    out[place_of(list_places, p, n)] = value | (address + half * 2048) << 16;
+                }
+                asm volatile("" ::: "memory");
+            }
+        }
+        first = last;
+        if (first < kEmitLists) {
+            dealt = __builtin_amdgcn_readlane(through, first - 1);
+            __syncthreads();  // the places are dealt afresh
+        }
+    }
+}
+
+}  // namespace
+
+// A2: row-major M x K fp16 in device memory (M % 128 == 0, K % 128 == 0, checked by the caller).
+// offsets: (M / 16) * (K / 128) + 1 ints; *longest: the longest list's length.
+extern "C" int a24_launch_residual_offsets(void* stream, const void* A2, int M, int K, int* offsets, int* longest)
+{
+    const int units = K / 128;
+    const long lists = static_cast<long>(M / 16) * units;
+    if (lists < 1 || lists > 0x7ffffff0L)
+        return static_cast<int>(hipErrorInvalidValue);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const long tasks = static_cast<long>(M / 16) * ((units + 3) / 4);
+    hipLaunchKernelGGL(a24_residual_count_kernel, dim3((unsigned)((tasks + 3) / 4)), dim3(256), 0, s,
+                       static_cast<const uint16_t*>(A2), K, units, (unsigned)tasks, offsets);
+    hipLaunchKernelGGL(a24_residual_scan_kernel, dim3(1), dim3(offscan::kThreads), 0, s, offsets, lists, longest);
+    return static_cast<int>(hipGetLastError());
+}
+
+// words: offsets[last] + 64 of them (the last 64 are zeroed).
+extern "C" int a24_launch_residual_words(void* stream, const void* A2, int M, int K, const int* offsets, void* words)
+{
+    const int units = K / 128;
+    const long lists = static_cast<long>(M / 16) * units;
+    if (lists < 1 || lists > 0x7ffffff0L)
+        return static_cast<int>(hipErrorInvalidValue);
+    hipLaunchKernelGGL(a24_residual_emit_kernel, dim3((unsigned)((lists + kEmitLists - 1) / kEmitLists)), dim3(kEmitWaves * 64), 0,
+                       static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(A2), K, units, lists, offsets,
+                       static_cast<uint32_t*>(words));
+    return static_cast<int>(hipGetLastError());
+}

@@ -857,3 +857,21 @@ def test_fused_row_skewed_weight_full_size(spmm, oracle):
     two = run_hybrid(spmm, packed, items, offsets, B, M, N, K, s, spmm.SpMM_SuggestSplitK(M, N, K))
     diff = np.abs(C.astype(np.float32) - two.astype(np.float32))
     assert np.isfinite(C).all() and (diff <= 2e-2 + 2e-2 * np.abs(two.astype(np.float32))).all()
+
+
+@pytest.mark.parametrize("M,K,sparsity", [(8320, 4096, 0.6), (128, 384, 0.55), (1024, 896, 0.25), (256, 512, 0.85)])
+def test_device_residual_lists_edges(spmm, oracle, M, K, sparsity):
+    """Residual lists where the GPU's packer changes its way: more lists than one step of the scan takes
+    (16640), units that leave a rest of four and workgroups with a rest of 32 lists, lists beyond four
+    rounds of 64 words and more words than are dealt in one pass, lists of one round beside empty ones."""
+    torch = _torch()
+    A = spmm.synth_weights(M, K, sparsity, False, seed=M + K)
+    _, A2 = oracle.decompose(A)
+    want_words, want_offs, want_longest = spmm.HeteroSparse_PackA2(A2)
+    d_A2 = torch.from_numpy(A2.view(np.int16).copy()).to("cuda:0").view(torch.float16)
+    print(f"[gpu case] device residual lists M={M} K={K} sparsity={sparsity}", flush=True)
+    words, offs, longest = spmm.pack_residual_on_device(d_A2)
+    torch.cuda.synchronize()
+    assert longest == want_longest
+    assert np.array_equal(offs.cpu().numpy(), want_offs)
+    assert np.array_equal(words.cpu().numpy().view(np.uint32), want_words)
