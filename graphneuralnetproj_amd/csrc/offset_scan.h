@@ -1,10 +1,12 @@
 // Running totals of per-tile or per-list counts in device memory, in place, by one workgroup.
+// Shared by the Tiled-CSL encoder and the residual packer.
 //
 // Bound by the latency of its few trips to memory, not by bandwidth: 75264 counts are 0.3 MB.  A
 // workgroup takes 16384 counts per step, 16 bytes per lane and load with whole lines per wave, the
 // next step's loads in flight while this one adds; lane sums go through DPP, wave sums through LDS
 // with one barrier per step.  (One chunk of consecutive counts per thread, read twice, had every
-// load of a wave touch 64 lines: 133 us for 75264 counts, now 10.)
+// load of a wave touch 64 lines: 133 us for 75264 counts, now 10;
+// 38 us for 25088, now 7.)
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -11,197 +11,270 @@
 //   * the pop order is "level = tallest stack down to 1, banks in id order, every bank at
 //     least that tall" (the largest stack with the lowest id wins each arg-max,
 //     csrc/SpMM_API.cu:223-234), and the emission order (:379-424) is index arithmetic on it.
-// So every element computes its own final position.  Three kernels: count per tile, scan,
+// So every element computes its own place in the pop order.  Three kernels: count per tile, scan,
 // emit.  No counterpart in the reference, which encodes on one host thread.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
+#include "offset_scan.h"
+
 namespace {
 
-constexpr int kTileRows = 128, kTileCols = 64, kBanks = 32, kThreads = 256;
-constexpr int kRowsPerThread = kTileRows / (kThreads / kBanks);  // 16
-constexpr int kMaxLevel = 2 * kTileRows + 4;                      // 256 per bank + up to 3 pads, rounded up
+constexpr int kTileRows = 128, kTileCols = 64, kBanks = 32, kThreads = 256, kWaves = kThreads / 64;
+constexpr int kRowGroups = kThreads / kBanks, kRowsPerThread = kTileRows / kRowGroups;  // 8, 16
+constexpr int kMaxLevel = 2 * kTileRows + 4;  // 256 per bank + up to 3 pads, rounded up
 
-// csrc/SpMM_API.cu:262: kept when fabs(float(v)) > 0, i.e. not +-0 and not NaN
-__device__ __forceinline__ bool kept(uint32_t h)
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+// 1 in each half that holds a kept value (csrc/SpMM_API.cu:262: fabs(float(v)) > 0, i.e. not +-0 and
+// not NaN), else 0.
+__device__ __forceinline__ u16x2 kept_halves(uint32_t pair)
 {
-    const uint32_t mag = h & 0x7fffu;
-    return mag != 0 && mag <= 0x7c00u;
+    const u16x2 mag = __builtin_bit_cast(u16x2, pair & 0x7fff7fffu);
+    const u16x2 nan = (mag + u16x2{0x3ff, 0x3ff}) >> u16x2{15, 15};  // past 0x7c00
+    return __builtin_elementwise_min(mag, u16x2{1, 1}) - nan;
 }
 
-// The pair of adjacent columns that row m gives to bank b, as one 32-bit load.
-__device__ __forceinline__ uint32_t load_pair(const uint16_t* tile, int ld, int m, int b)
-{
-    const int x = b ^ ((m & 7) << 2);  // the unswizzled column pair
-    return *reinterpret_cast<const uint32_t*>(tile + (size_t)m * ld + 2 * x);
-}
-
+// Vectors per tile into offsets[tile + 1].  Bound by HBM (the matrix is read once): a wave reads 32
+// rows of up to eight consecutive tiles, a contiguous KiB per load, all in flight.  (Four bytes per
+// lane, one tile per workgroup: 86 us for 411 MB, now 74.)  Workgroups go from the matrix's
+// start to its end, the emit kernel's from end to start: it begins with what is left in the
+// last-level cache.
+constexpr int kCountTiles = 8;
 __global__ __launch_bounds__(kThreads) void tcsl_count_tiles(const uint16_t* __restrict__ A, int K, int tiles_k,
                                                             int* __restrict__ offsets)
 {
-    const int t = blockIdx.x;
-    const uint16_t* tile = A + (size_t)(t / tiles_k) * kTileRows * K + (size_t)(t % tiles_k) * kTileCols;
-    const int b = threadIdx.x & 31, rg = threadIdx.x >> 5;
-    int c = 0;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    __shared__ int part[kWaves][kCountTiles];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int spans = (tiles_k + kCountTiles - 1) / kCountTiles;
+    const int row_tile = blockIdx.x / spans, first = (blockIdx.x % spans) * kCountTiles;
+    int n = 0;
+    if (first + (lane >> 3) < tiles_k) {
+        constexpr int kRows = kTileRows / kWaves;
+        const uint16_t* src = A + ((size_t)row_tile * kTileRows + wave * kRows) * K + (size_t)first * kTileCols + lane * 8;
+        u32x4 v[kRows];
 #pragma unroll
-    for (int i = 0; i < kRowsPerThread; i++) {
-        const uint32_t p = load_pair(tile, K, rg * kRowsPerThread + i, b);
-        c += kept(p & 0xffffu) + kept(p >> 16);
+        for (int r = 0; r < kRows; r++)
+            v[r] = *reinterpret_cast<const u32x4*>(src + (size_t)r * K);
+        u16x2 c = {0, 0};
+#pragma unroll
+        for (int r = 0; r < kRows; r++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                c += kept_halves(v[r][i]);
+        n = c[0] + c[1];
     }
-    __shared__ int part[kThreads / 64];
-    for (int o = 32; o > 0; o >>= 1)
-        c += __shfl_down(c, o);
-    if ((threadIdx.x & 63) == 0)
-        part[threadIdx.x >> 6] = c;
+    for (int o = 4; o > 0; o >>= 1)
+        n += __shfl_xor(n, o);
+    if ((lane & 7) == 0)
+        part[wave][lane >> 3] = n;
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < kCountTiles && first + (int)threadIdx.x < tiles_k) {
         int nz = 0;
-        for (int i = 0; i < kThreads / 64; i++)
-            nz += part[i];
-        offsets[t + 1] = (nz + 3) / 4;  // vectors of four words, zero padded (:289)
+        for (int w = 0; w < kWaves; w++)
+            nz += part[w][threadIdx.x];
+        offsets[(size_t)row_tile * tiles_k + first + threadIdx.x + 1] = (nz + 3) / 4;  // vectors of four words, zero padded (:289)
     }
 }
 
 // offsets[1..tiles] hold per-tile vector counts; turn them into the running total
 // (offsets[0] = 0, offsets[tiles + 1] = total, :426-435).  One workgroup.  If the total does
 // not fit an int, offsets[tiles + 1] is set to -1.
-__global__ __launch_bounds__(1024) void tcsl_scan_offsets(int* __restrict__ offsets, long tiles)
+__global__ __launch_bounds__(offscan::kThreads) void tcsl_scan_offsets(int* __restrict__ offsets, long tiles)
 {
-    __shared__ long long sums[1024];
-    const long chunk = (tiles + 1023) / 1024;
-    const long lo = threadIdx.x * chunk, hi = lo + chunk < tiles ? lo + chunk : tiles;
-    long long s = 0;
-    for (long i = lo; i < hi; i++)
-        s += offsets[i + 1];
-    sums[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {  // inclusive scan of the chunk sums
-        const long long v = threadIdx.x >= o ? sums[threadIdx.x - o] : 0;
-        __syncthreads();
-        sums[threadIdx.x] += v;
-        __syncthreads();
-    }
-    long long run = threadIdx.x ? sums[threadIdx.x - 1] : 0;
-    const bool fits = sums[1023] <= 0x7fffffffLL;
-    for (long i = lo; i < hi; i++) {
-        run += offsets[i + 1];
-        offsets[i + 1] = fits ? static_cast<int>(run) : 0;
-    }
+    int most;
+    const long long total = offscan::scan_in_place(offsets + 1, tiles, most);
+    const bool fits = total <= 0x7fffffffLL;
+    if (!fits)
+        offscan::clear_counts(offsets + 1, tiles);
     if (threadIdx.x == 0) {
         offsets[0] = 0;
-        offsets[tiles + 1] = fits ? static_cast<int>(sums[1023]) : -1;
+        offsets[tiles + 1] = fits ? static_cast<int>(total) : -1;
     }
 }
 
-__global__ __launch_bounds__(kThreads) void tcsl_emit_tiles(const uint16_t* __restrict__ A, int K, int tiles_k,
-                                                           const int* __restrict__ offsets,
-                                                           uint32_t* __restrict__ items)
+// Smallest and largest value of lanes 0 .. 31, whose copies lanes 32 .. 63 hold.
+template<typename Op>
+__device__ __forceinline__ int half_wave_reduce(int x, int neutral, Op op)
 {
-    __shared__ uint32_t bank[kBanks][kMaxLevel];      // the per-bank lists ("stacks" of the reference)
-    __shared__ int grp_count[kThreads / kBanks][kBanks];
-    __shared__ int grp_zero[kThreads / kBanks][kBanks];
-    __shared__ int size[kBanks];
-    __shared__ uint32_t level_mask[kMaxLevel + 2];    // banks at least l tall
-    __shared__ int level_first[kMaxLevel + 2];        // pops made before level l starts
-    __shared__ int total_words;
+    x = op(x, __builtin_amdgcn_update_dpp(neutral, x, 0x111, 0xf, 0xf, false));  // row_shr 1, 2, 4, 8: within 16 lanes
+    x = op(x, __builtin_amdgcn_update_dpp(neutral, x, 0x112, 0xf, 0xf, false));
+    x = op(x, __builtin_amdgcn_update_dpp(neutral, x, 0x114, 0xf, 0xf, false));
+    x = op(x, __builtin_amdgcn_update_dpp(neutral, x, 0x118, 0xf, 0xf, false));
+    x = op(x, __builtin_amdgcn_update_dpp(neutral, x, 0x142, 0xa, 0xf, false));  // lane 15 to lanes 16 .. 31
+    return __builtin_amdgcn_readlane(x, 31);
+}
 
-    const int t = blockIdx.x;
+// The packed words of one tile, by one workgroup; thread (rg, b) owns the sixteen column pairs that
+// rows 16 rg .. +15 give to bank b, and keeps them in registers.  Bound by instruction issue (32
+// candidates per thread, a fifth of them kept at 80 % sparsity) beside the read of the matrix and
+// the write of the words.
+//   * An element's place in its bank's list is a prefix count; its place in the pop order is the
+//     number of pops before its level plus the number of lower banks as tall, both from one LDS
+//     read of the level's entry (mask of banks, pops before).  The four waves fill that table level by
+//     level from ballots on the banks' sizes, each its quarter of the levels.
+//   * Words go into LDS in pop order and leave it in the order of emission (:379-424), which is plain
+//     arithmetic on the output position: four conflict-free reads and one 16-byte store per vector.
+//   * 4096 words of LDS for the sequence, so that seven workgroups share a compute unit; a tile beyond
+//     that (50 % dense) takes another pass over the registers for every 3968 words.
+// (Bank lists staged in LDS, level sums by one thread over 260 levels, words stored one by one:
+// 303 us for a 28672 x 7168 weight at 80 %, now 130, 4.4 TB/s.)
+constexpr int kSeqWords = 4096, kPassWords = kSeqWords - 128;  // the first pass takes the tail's up to 124 pops as well
+
+__global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* __restrict__ A, int K, int tiles_k,
+                                                              const int* __restrict__ offsets, uint32_t* __restrict__ items)
+{
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    __shared__ uint32_t seq[kSeqWords + 64];   // pops first .. first + kSeqWords - 1; then where words of other passes go
+    __shared__ u32x2 levels[kMaxLevel + 1];    // level l: banks at least l tall, pops made before the level starts
+    __shared__ int grp_count[kRowGroups][kBanks];
+    __shared__ int grp_zero[kRowGroups][kBanks];
+
+    const int t = gridDim.x - 1 - blockIdx.x;
     const int words = (offsets[t + 1] - offsets[t]) * 4;
     if (words == 0)
         return;  // an all-zero tile emits nothing (uniform for the workgroup)
     const uint16_t* tile = A + (size_t)(t / tiles_k) * kTileRows * K + (size_t)(t % tiles_k) * kTileCols;
-    uint32_t* out = items + (size_t)offsets[t] * 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int b = threadIdx.x & 31, rg = threadIdx.x >> 5;
 
-    // 1. this thread's 16 rows of bank b: count the kept elements, note the first zero position
+    // 1. this thread's 16 rows of bank b: mark the kept elements, note the first other position.
+    //    Row m gives bank b the pair of adjacent columns whose swizzled positions are 2 b, 2 b + 1.
+    const uint16_t* const own_rows = tile + (size_t)(rg * kRowsPerThread) * K;
     uint32_t pairs[kRowsPerThread];
-    int c = 0, zero = -1;
 #pragma unroll
     for (int i = 0; i < kRowsPerThread; i++) {
-        const int m = rg * kRowsPerThread + i;
-        pairs[i] = load_pair(tile, K, m, b);
-        const bool k0 = kept(pairs[i] & 0xffffu), k1 = kept(pairs[i] >> 16);
-        c += k0 + k1;
-        if (zero < 0 && !k0)
-            zero = m * kTileCols + 2 * b;       // position = row * 64 + swizzled column (:330-339)
-        if (zero < 0 && !k1)
-            zero = m * kTileCols + 2 * b + 1;
+        const int x = b ^ ((i & 7) << 2);
+        pairs[i] = *reinterpret_cast<const uint32_t*>(own_rows + (size_t)i * K + 2 * x);
     }
-    grp_count[rg][b] = c;
-    grp_zero[rg][b] = zero;
-    __syncthreads();
-
-    // 2. place in the bank's list = kept elements of the bank in earlier rows; write the words
-    int rank = 0;
-    for (int g = 0; g < rg; g++)
-        rank += grp_count[g][b];
+    uint32_t kept = 0;  // bit i + 16 h: element h of row i
 #pragma unroll
-    for (int i = 0; i < kRowsPerThread; i++) {
-        const int m = rg * kRowsPerThread + i;
-        const uint32_t lo = pairs[i] & 0xffffu, hi = pairs[i] >> 16;
-        if (kept(lo))
-            bank[b][rank++] = lo | (uint32_t)(m * kTileCols + 2 * b) << 16;
-        if (kept(hi))
-            bank[b][rank++] = hi | (uint32_t)(m * kTileCols + 2 * b + 1) << 16;
-    }
-    if (rg == kThreads / kBanks - 1)
-        size[b] = rank;
+    for (int i = 0; i < kRowsPerThread; i++)
+        kept |= __builtin_bit_cast(uint32_t, kept_halves(pairs[i])) << i;
+    const int own = __popc(kept);
+    const uint32_t gone = ~kept;  // the first position in row order: the lower row, then the lower element
+    const int z0 = __ffs(static_cast<int>(gone & 0xffffu)) - 1, z1 = __ffs(static_cast<int>(gone >> 16)) - 1;
+    const int z = z0 >= 0 && (z1 < 0 || z0 <= z1) ? 2 * z0 : (z1 < 0 ? -1 : 2 * z1 + 1);
+    const int corner = rg * kRowsPerThread * kTileCols + 2 * b;  // position = row * 64 + swizzled column (:330-339)
+    grp_count[rg][b] = own;
+    grp_zero[rg][b] = z < 0 ? -1 : corner + (z >> 1) * kTileCols + (z & 1);
     __syncthreads();
 
-    // 3. zero padding to a multiple of four, each pad on the currently smallest bank (lowest id
-    //    on ties), pointing at that bank's first zero position (:352-365)
-    if (threadIdx.x == 0) {
-        int count = 0;
-        for (int i = 0; i < kBanks; i++)
-            count += size[i];
-        const int pad = (4 - count % 4) % 4;
-        for (int p = 0; p < pad; p++) {
-            int s = 0;
-            for (int i = 1; i < kBanks; i++)
-                if (size[i] < size[s])
-                    s = i;
-            int z = -1;
-            for (int g = 0; g < kThreads / kBanks && z < 0; g++)
-                z = grp_zero[g][s];
-            bank[s][size[s]++] = (uint32_t)z << 16;
-        }
-        total_words = count + pad;
+    // 2. the bank's size, and this thread's first place in its list
+    int size = 0, rank = 0;
+#pragma unroll
+    for (int g = 0; g < kRowGroups; g++) {
+        const int c = grp_count[g][b];
+        rank += g < rg ? c : 0;
+        size += c;
     }
-    __syncthreads();
-
-    // 4. pop order: level = tallest down to 1, banks by id.  level_first[l] = pops before level l.
-    for (int l = threadIdx.x + 1; l <= kMaxLevel; l += kThreads) {
-        uint32_t mask = 0;
-        for (int i = 0; i < kBanks; i++)
-            mask |= (uint32_t)(size[i] >= l) << i;
-        level_mask[l] = mask;
+    // 3. zero padding to a multiple of four, each pad on the currently smallest bank (lowest id on
+    //    ties), pointing at that bank's first zero position (:352-365).  Every wave works it out.
+    const int real = size;  // of the bank, without pads
+    const int count = __builtin_amdgcn_readlane(offscan::wave_inclusive_sum(lane < kBanks ? size : 0), 63);
+    for (int pad = (4 - count % 4) % 4; pad > 0; pad--) {
+        const int low = half_wave_reduce(size << 5 | b, 0x7fffffff, [](int x, int y) { return x < y ? x : y; });
+        size += (low & 31) == b ? 1 : 0;
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int run = 0;
-        for (int l = kMaxLevel; l >= 1; l--) {
-            level_first[l] = run;
-            run += __popc(level_mask[l]);
+    // 4. pop order: level = tallest down to 1, banks by id
+    const int top = half_wave_reduce(size, 0, [](int x, int y) { return x > y ? x : y; });
+    const int share = (top + kWaves - 1) / kWaves;
+    const int lo = 1 + wave * share, hi = lo + share - 1 < top ? lo + share - 1 : top;
+    if (lo <= hi) {
+        const int above = size - hi;
+        int pops = __builtin_amdgcn_readlane(offscan::wave_inclusive_sum(lane < kBanks && above > 0 ? above : 0), 63);
+        for (int l = hi; l >= lo; l--) {
+            const uint32_t mask = static_cast<uint32_t>(__ballot(size >= l));
+            if (lane == 0)
+                levels[l] = u32x2{mask, static_cast<uint32_t>(pops)};
+            pops += __popc(mask);
         }
     }
     __syncthreads();
 
-    // 5. emission (:379-424): V vectors = R groups of 32 lanes + rem lanes.  The first 4*rem pops
+    // 5. emission (:379-424): V vectors = R groups of 32 lanes + rem lanes.  The first 4 * rem pops
     //    fill the tail (lane = pop % rem, slot 3 - pop / rem), the rest the main part (lane =
-    //    pop' % 32, arrival kk = pop' / 32 written at reverse position 4R-1-kk).
-    const int vecs = total_words / 4, R = vecs / 32, rem = vecs % 32;
-    for (int j = rg; j < size[b]; j += kThreads / kBanks) {
-        const int l = j + 1;
-        const int pop = level_first[l] + __popc(level_mask[l] & ((1u << b) - 1u));
-        int idx;
-        if (pop < 4 * rem) {
-            idx = R * 128 + (pop % rem) * 4 + (3 - pop / rem);
-        } else {
-            const int q = pop - 4 * rem, kk = q >> 5, lane = q & 31;
-            const int pos = 4 * R - 1 - kk;  // = 4 * r + v
-            idx = ((pos >> 2) * 32 + lane) * 4 + (pos & 3);
+    //    pop' % 32, arrival kk = pop' / 32 written at reverse position 4 R - 1 - kk).
+    const uint32_t below = (1u << b) - 1u;
+    const int vecs = words / 4, R = vecs / 32, rem = vecs % 32;
+    u32x4* const out = reinterpret_cast<u32x4*>(items) + offsets[t];
+    const int dump = kSeqWords + lane;
+    // The words of pops first .. last - 1 into the sequence.  Level entries are read sixteen at a time,
+    // ahead of the writes that depend on them: one by one, every element pays a trip to LDS.
+    auto place_words = [&](int first, int last, auto all) __attribute__((always_inline)) {
+        auto slot = [&](u32x2 e, bool used) {
+            const int pop = static_cast<int>(e[1]) + __popc(e[0] & below);
+            if constexpr (decltype(all)::value)  // the tile's words fit one pass
+                return used ? pop : dump;
+            return used && pop >= first && pop < last ? pop - first : dump;
+        };
+        int level = rank, at = corner;
+        uint32_t live = kept;
+        // (opaque: or the compiler prepares all 32 words and places ahead of both ways, and spills)
+        asm volatile("" : "+v"(level), "+v"(at), "+v"(live));
+#pragma unroll
+        for (int i0 = 0; i0 < kRowsPerThread; i0 += 8) {
+            u32x2 e[16];
+#pragma unroll
+            for (int j = 0; j < 16; j++) {
+                level += (live >> (i0 + j / 2 + 16 * (j & 1))) & 1;
+                e[j] = levels[level];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < 16; j++) {
+                const uint32_t pair = pairs[i0 + j / 2], position = at + (i0 + j / 2) * kTileCols + (j & 1);
+                seq[slot(e[j], (live >> (i0 + j / 2 + 16 * (j & 1))) & 1)] = (j & 1 ? pair >> 16 : pair & 0xffffu) | position << 16;
+            }
         }
-        out[idx] = bank[b][j];
+        if (rg == 0 && size > real) {  // the pads, behind the bank's last element
+            int p = -1;
+            for (int g = 0; g < kRowGroups && p < 0; g++)
+                p = grp_zero[g][b];
+            for (int l = real + 1; l <= size; l++)
+                seq[slot(levels[l], true)] = static_cast<uint32_t>(p) << 16;
+        }
+    };
+    // groups of 32 vectors out of the sequence, whose word `from` is the first of their 128 pops
+    auto write_groups = [&](int from, int done, int groups) __attribute__((always_inline)) {
+        for (int i = threadIdx.x; i < groups * 32; i += kThreads) {
+            const int g = i >> 5, at = from + g * 128 + (i & 31);  // pops 128 g + 32 (3 - s) + lane
+            u32x4 v;
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+                v[s] = seq[at + (3 - s) * 32];
+            out[(R - 1 - done - g) * 32 + (i & 31)] = v;
+        }
+    };
+    auto write_tail = [&]() __attribute__((always_inline)) {
+        if ((int)threadIdx.x < rem) {
+            u32x4 v;
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+                v[s] = seq[(3 - s) * rem + threadIdx.x];
+            out[R * 32 + threadIdx.x] = v;
+        }
+    };
+    if (words <= kPassWords) {
+        place_words(0, words, std::true_type{});
+        __syncthreads();
+        write_tail();
+        write_groups(4 * rem, 0, R);
+        return;
+    }
+    for (int first = 0, last = 4 * rem + kPassWords; first < words; first = last, last += kPassWords) {
+        place_words(first, last, std::false_type{});
+        __syncthreads();
+        const int from = first == 0 ? 4 * rem : 0;
+        const int done = (first + from - 4 * rem) / 128;  // groups of earlier passes
+        if (first == 0)
+            write_tail();
+        write_groups(from, done, R - done < kPassWords / 128 ? R - done : kPassWords / 128);
+        __syncthreads();  // the sequence is written afresh
     }
 }
 
@@ -214,9 +287,10 @@ extern "C" int tcsl_launch_encode_offsets(void* stream, const void* A, int M, in
     if (tiles < 1 || tiles > 0x7fffffffL)
         return static_cast<int>(hipErrorInvalidValue);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(tcsl_count_tiles, dim3((unsigned)tiles), dim3(kThreads), 0, s, static_cast<const uint16_t*>(A), K,
+    const long spans = (tiles_k + kCountTiles - 1) / kCountTiles * (M / kTileRows);
+    hipLaunchKernelGGL(tcsl_count_tiles, dim3((unsigned)spans), dim3(kThreads), 0, s, static_cast<const uint16_t*>(A), K,
                        (int)tiles_k, offsets);
-    hipLaunchKernelGGL(tcsl_scan_offsets, dim3(1), dim3(1024), 0, s, offsets, tiles);
+    hipLaunchKernelGGL(tcsl_scan_offsets, dim3(1), dim3(offscan::kThreads), 0, s, offsets, tiles);
     return static_cast<int>(hipGetLastError());
 }
 

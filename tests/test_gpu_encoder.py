@@ -102,6 +102,13 @@ def test_device_encoder_matches_oracle(spmm, oracle, M, K, sparsity, skew):
     _compare(spmm, oracle, spmm.synth_weights(M, K, sparsity, skew, seed=M + K))
 
 
+@pytest.mark.parametrize("M,K,sparsity", [(128, 64, 0.516), (256, 64 * 9, 0.515), (128, 64 * 8, 0.03), (256, 64 * 17, 0.27)])
+def test_device_encoder_edges(spmm, oracle, M, K, sparsity):
+    """Tiles around the 3968 words that the GPU encoder emits in one pass (48.4 % dense) and beyond, in two
+    and in three; spans of eight tiles, whole and with a rest of one; pads of every number."""
+    _compare(spmm, oracle, spmm.synth_weights(M, K, sparsity, False, seed=M + K))
+
+
 def test_device_encoder_special_tiles(spmm, oracle):
     """All-zero tiles, a fully dense tile, single elements, and the values the reference treats specially."""
     rng = np.random.default_rng(7)
