@@ -189,8 +189,13 @@ __global__ __launch_bounds__(offscan::kThreads) void a24_residual_scan_kernel(in
 // the writing (from the last-level cache) instead of kept in registers.  (Eight waves with 51 KiB, registers kept, words placed as 16-bit numbers: 211 us.
 // Dealing by laps, every round with room one word in the order of its room, four keys sorted per lap:
 // 302 us instead of 211, the lanes diverge.)
-constexpr int kEmitWaves = 4, kEmitLists = 32, kListsPerWave = kEmitLists / kEmitWaves;
-constexpr int kPlaces = 8192;  // bytes: 32 lists of 256 words (an ordinary residual has up to 200) are dealt in one pass
+constexpr int kEmitWaves = 4;
+// Lists per workgroup: 32 where that makes a chip full of workgroups (eight per compute unit), else
+// eight: the lists of a wave follow one another, so few lists are better spread over more waves
+// (whole calls at 50 / 70 / 95 % sparsity, 2048 x 4096 = 4096 lists: 72 / 56 / 47 us, with 32 a group
+// 91 / 75 / 59; 16384 lists are the 2048 groups of eight that run at once).
+constexpr int kManyLists = 32, kFewLists = 8;
+constexpr long kManyFrom = 16384;
 
 // A word of the bank-sorted sequence goes to the round that has the fewest words of its bank, then
 // the most room, then the lowest number: the largest of keys (63 - words of the bank, room - 1, last -
@@ -253,10 +258,14 @@ __device__ __forceinline__ void deal(const unsigned* counts, int n, uint8_t* pla
     }
 }
 
+template<int kEmitLists>
 __global__ __launch_bounds__(kEmitWaves * 64, 8) void a24_residual_emit_kernel(const uint16_t* __restrict__ A2, int K, int units,
                                                                                long lists, const int* __restrict__ offsets,
                                                                                uint32_t* __restrict__ words)
 {
+    constexpr int kListsPerWave = kEmitLists / kEmitWaves;
+    constexpr int kPlaces = kEmitLists * 256;  // bytes: lists of 256 words (an ordinary residual has up to 200) are dealt in one pass
+    static_assert(kPlaces >= 2 * kMaxListWords, "the longest list has to fit");
     __shared__ unsigned images[kEmitWaves][8 * 64];  // per wave: half of a list's block, [row][bank] column pairs
     __shared__ unsigned sorted[kEmitLists][17];      // counts of a list's banks, one byte each, largest first
     __shared__ int length[kEmitLists];
@@ -336,9 +345,14 @@ __global__ __launch_bounds__(kEmitWaves * 64, 8) void a24_residual_emit_kernel(c
                 for (int r = 0; r < 8; r++)
                     image[r * 64 + L] = pairs[half * 8 + r];
                 asm volatile("" ::: "memory");  // other lanes' words are read below
+                unsigned natural[8];  // columns 2 L and 2 L + 1
+#pragma unroll
+                for (int r8 = 0; r8 < 8; r8++)
+                    natural[r8] = image[r8 * 64 + (L ^ ((half * 8 + r8) << 2))];
+#pragma unroll
                 for (int r8 = 0; r8 < 8; r8++) {
                     const int r = half * 8 + r8;
-                    const unsigned pair = image[r8 * 64 + (L ^ (r << 2))];  // columns 2 L and 2 L + 1
+                    const unsigned pair = natural[r8];
                     const bool lo = residual_kept(pair), hi = residual_kept(pair >> 16);
                     const uint64_t los = __ballot(lo), his = __ballot(hi), below = (1ull << L) - 1;
                     const int place = at + __popcll(los & below) + __popcll(his & below);
@@ -430,8 +444,14 @@ extern "C" int a24_launch_residual_words(void* stream, const void* A2, int M, in
     const long lists = static_cast<long>(M / 16) * units;
     if (lists < 1 || lists > 0x7ffffff0L)
         return static_cast<int>(hipErrorInvalidValue);
-    hipLaunchKernelGGL(a24_residual_emit_kernel, dim3((unsigned)((lists + kEmitLists - 1) / kEmitLists)), dim3(kEmitWaves * 64), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(A2), K, units, lists, offsets,
-                       static_cast<uint32_t*>(words));
+    auto launch = [&](auto* kernel, int per_group) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((lists + per_group - 1) / per_group)), dim3(kEmitWaves * 64), 0,
+                           static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(A2), K, units, lists, offsets,
+                           static_cast<uint32_t*>(words));
+    };
+    if (lists >= kManyFrom)
+        launch(a24_residual_emit_kernel<kManyLists>, kManyLists);
+    else
+        launch(a24_residual_emit_kernel<kFewLists>, kFewLists);
     return static_cast<int>(hipGetLastError());
 }
