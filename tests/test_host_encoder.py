@@ -266,3 +266,22 @@ def test_where_the_slabs_are_added_up(spmm):
     for M, N, K, S in ((1000, 16, 1024, 2), (1024, 12, 1024, 2), (1024, 16, 1000, 2), (1024, 16, 1024, 0)):
         with pytest.raises(spmm.SpMMError):
             spmm.SpMM_PlanReductionInLaunch(M, N, K, S)
+
+
+@pytest.mark.parametrize("M,K,sparsity", [(128, 64, 0.9), (256, 64 * 17, 0.5), (1024, 4096, 0.5), (128, 64 * 33, 0.02)])
+def test_encoder_pieces_and_memory(spmm, oracle, M, K, sparsity):
+    """Spans of 16 tiles with a rest, results below and above the size that asks for huge pages, nearly
+    dense tiles; and the words stay readable through a view after the array itself is gone."""
+    import gc
+
+    A = spmm.synth_weights(M, K, sparsity, False, seed=M + K)
+    want, want_offsets = oracle.encode(A)
+    items, offsets = spmm.InitSparseMatrixA_API(A)
+    assert np.array_equal(offsets, want_offsets) and np.array_equal(items, want)
+    assert items.dtype == np.uint32 and items.flags.writeable and items.flags.c_contiguous
+    tail = items[len(items) // 2:]
+    del items
+    gc.collect()
+    for _ in range(3):  # would take the memory over
+        spmm.InitSparseMatrixA_API(A)
+    assert np.array_equal(tail, want[len(want) // 2:])
