@@ -10,12 +10,15 @@ namespace tcsl {
 // separate_reduction (mode 1, Split_K > 1): the slabs of partial sums are added up by the reduction
 //         kernel instead of by the last workgroup of each tile row inside the launch (mode 0 always
 //         uses the reduction kernel).
+// paired (mode 0, 2 waves, 64 tokens): both waves work on every tile of one tile row, with 32 tokens each;
+//         only the planner makes such a plan.
 struct LaunchPlan {
     int mode;
     int waves;
     int stage_b;
     unsigned lds_bytes;
     bool separate_reduction = false;
+    bool paired = false;
 };
 
 // True (and lds_bytes filled in) when the kernels can run this shape.

@@ -873,6 +873,260 @@ __global__ __launch_bounds__(MAXW* kWave) void tcsl_spmm_kernel(const int* __res
                          arrivals + blockIdx.x, reinterpret_cast<unsigned int*>(lds), W * kWave, ROWMAJ);
 }
 
+// 64 tokens, two waves to a work unit: both work on every tile of the unit's run, each scatters half of
+// the tile's words into one image that both then multiply, with 32 tokens of activations each.
+//
+// What bounds 64 tokens in the kernel above is the chain of one wave: a tile is 64 MFMAs (1024 cycles)
+// behind some 72 LDS instructions, in about 3000 cycles, and its 128 accumulator registers leave room
+// for one wave per SIMD.  Half the tokens halve a wave's accumulators, MFMAs, activation fragments and
+// scatter; a pair takes 1780 cycles for a tile where it has a compute unit to itself, and three pairs fit
+// one.  The image is read twice for it (256 of about 500 LDS cycles per tile), so this wins where there is
+// little work per compute unit and the chain is what counts, and ties where the chip is full:
+// 512 x 704 12.2 -> 9.6 us, 1024 x 2240 12.2 -> 10.2, 3072 x 2368 14.5 -> 12.1, 47232 x 1024 33.6 -> 27.9,
+// 49152 x 12288 125 -> 119, but 28672 x 7168 49 against 55 at best (the planner's rule: launch_plan.cpp).
+// (32 tokens, 16 for each wave, lost 2 % in the mean over the same sizes and up to 23 %.)
+//
+// Three images per pair, one barrier per tile.  Before tile t's barrier a wave has scattered its half
+// of t into image t % 3 (and waits for its LDS operations); behind it, it reads tile t and clears its
+// half of tile t - 1's image, which nobody reads any more (every wave's reads of t - 1 came back before
+// the barrier; whole lines: 8 writes, where undoing the scatter takes 13 and 32 registers).  Image t % 3 is written again for tile t + 3, behind the barrier of t + 2; its clearing
+// lies between the barriers of t + 1 and t + 2.  The clearing of the last tile but one is left out: the
+// waves take the two images that the last tile does not use for their output.
+//
+// Loads, segments and the asynchronous-load rule as above, with half as many vectors per lane in a ring
+// of three slots (two slots covered too little of the memory's latency: 28672 x 7168 in one batch 101 us, three 87);
+// the second half begins at a multiple of 32 vectors, the groups that the encoder spreads over the banks.  Dynamic LDS: three tiles.  grid (tile rows, Split_K), 128 threads.
+constexpr int kPairImages = 3, kPairRing = 3;
+__global__ __launch_bounds__(2 * kWave, 2) void tcsl_spmm_pair_kernel(const int* __restrict__ offsets,
+                                                                      const u32x4* __restrict__ items,
+                                                                      const _Float16* __restrict__ B,
+                                                                      _Float16* __restrict__ out, int K, int avg, int ldb, int M,
+                                                                      int ldo, int relu)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    constexpr int NB = 2, NTOK = 32 * NB, BL = 2 * NB, D = kPairRing;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int rt = blockIdx.x, batch = blockIdx.y;
+    const int nkb = K / kTileCols;
+    int kb0 = batch * avg;
+    kb0 = kb0 < nkb ? kb0 : nkb;
+    int kb1 = kb0 + avg;
+    kb1 = kb1 < nkb ? kb1 : nkb;
+    const int ntile = kb1 - kb0;
+    const int* const toff = offsets + (size_t)rt * nkb + kb0;
+    const int wreg = toff[lane <= ntile ? lane : ntile];  // lane l: first vector of tile l
+    for (int i = threadIdx.x * 16; i < kPairImages * kTileBytes; i += 2 * kWave * 16)
+        *reinterpret_cast<u32x4*>(lds + i) = u32x4{0u, 0u, 0u, 0u};
+    __syncthreads();
+
+    auto tile_range = [&](int i, int& begin, int& end) __attribute__((always_inline)) {  // 0 <= i < ntile
+        begin = __builtin_amdgcn_readlane(wreg, i);
+        end = __builtin_amdgcn_readlane(wreg, i + 1);
+    };
+
+    f32x4 acc[NB][8];
+#pragma unroll
+    for (int c = 0; c < NB; c++)
+#pragma unroll
+        for (int r = 0; r < 8; r++)
+            acc[c][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int l15 = lane & 15, q = lane >> 4;
+    int a_off[2];
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+        a_off[s] = l15 * 128 + (((s * 4 + q) ^ (lane & 7)) << 4);
+    const _Float16* bptr[NB];
+#pragma unroll
+    for (int c = 0; c < NB; c++)
+        bptr[c] = B + (size_t)(wave * (16 * NB) + c * 16 + l15) * ldb + (size_t)kb0 * kTileCols + q * 8;
+    const int voff_lo = lane * 16, voff_hi = lane * 16 + 4096;
+    uint32_t vtwo = 2;
+    asm volatile("" : "+v"(vtwo));
+    const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
+    int image = 0;  // byte offset of the current tile's image
+
+    auto stream_run = [&](auto vpl_c) __attribute__((always_inline)) {
+        constexpr int VPL = decltype(vpl_c)::value;
+        constexpr int L = VPL + BL;
+        constexpr int kSeg = VPL * kWave;
+        struct Seg {
+            int tile;     // index within the unit; ntile = past the end
+            int begin;    // first vector, absolute
+            int n;        // vectors in this segment
+            bool last;    // last segment of this wave's half of the tile
+        };
+        struct Cur {
+            int tile, off;
+        };
+        auto make_seg = [&](Cur c, Seg& s, Cur& nxt) __attribute__((always_inline)) {
+            if (c.tile >= ntile) {
+                s = Seg{ntile, 0, 0, true};
+                nxt = c;
+                return;
+            }
+            int b, e;
+            tile_range(c.tile, b, e);
+            const int n = e - b, cut = (n / 2 + 16) & ~31, middle = b + (cut < n ? cut : n);
+            b = wave ? middle : b;
+            e = wave ? e : middle;
+            const int rest = e - b - c.off;
+            s.tile = c.tile;
+            s.begin = b + c.off;
+            s.n = rest < kSeg ? rest : kSeg;
+            s.last = rest <= kSeg;
+            nxt = s.last ? Cur{c.tile + 1, 0} : Cur{c.tile, c.off + kSeg};
+        };
+
+        u32x4 regs[D][VPL];
+        half8 bfrag[D][BL];
+        Seg held[D] = {};
+        int old_image = 0;  // the tile before's
+
+        auto issue = [&](int slot, const Seg& s) __attribute__((always_inline)) {
+            const bool live = s.tile < ntile;
+            const uint64_t base = reinterpret_cast<uint64_t>(items + s.begin);
+            i32x4 rs = {(int)(uint32_t)base, (int)((uint32_t)(base >> 32) & 0xffff), live ? s.n * 16 : 0, 0x00020000};
+            const int bt = live ? s.tile : ntile - 1;
+#pragma unroll
+            for (int cb = 0; cb < NB; cb++)
+#pragma unroll
+                for (int k = 0; k < 2; k++)
+                    bfrag[slot][cb * 2 + k] = load_activations(bptr[cb] + bt * kTileCols + k * 32);
+            static_for<VPL>([&](auto uc) {
+                constexpr int u = decltype(uc)::value;
+                if constexpr (u < 4)
+                    regs[slot][u] = load_words<u * 1024>(rs, voff_lo);
+                else
+                    regs[slot][u] = load_words<(u - 4) * 1024>(rs, voff_hi);
+            });
+        };
+        auto land = [&](int slot, auto younger) __attribute__((always_inline)) {
+            wait_loads<decltype(younger)::value>();
+            static_for<VPL>([&](auto uc) { pin(regs[slot][decltype(uc)::value]); });
+#pragma unroll
+            for (int h = 0; h < BL; h++)
+                settle(bfrag[slot][h]);
+        };
+        // op(u) for every vector u of this lane's that a segment of n vectors holds (see the kernel above)
+        auto by_chunks = [&](int n, auto&& op) __attribute__((always_inline)) {
+            const int full = n >> 6;
+            const bool in_part = (full << 6) + lane < n;
+            bool done = false;
+            static_for<VPL + 1>([&](auto pc) {
+                constexpr int P = decltype(pc)::value;
+                if (!done && full == P) {
+                    static_for<P>([&](auto uc) { op(uc); });
+                    if constexpr (P < VPL) {
+                        if (in_part)
+                            op(pc);
+                    }
+                    done = true;
+                }
+            });
+        };
+        auto consume = [&](auto slot_c, const Seg& s, auto younger) __attribute__((always_inline)) {
+            constexpr int slot = decltype(slot_c)::value;
+            land(slot, younger);
+            if (s.tile >= ntile)
+                return;
+            uint32_t vbase = lds_base + image;
+            asm volatile("" : "+v"(vbase));
+            by_chunks(s.n, [&](auto uc) {
+                constexpr int u = decltype(uc)::value;
+                uint32_t address[4];
+                scatter_words_keep(regs[slot][u], vbase, vtwo, address);
+            });
+            if (!s.last)
+                return;  // more segments of this half follow
+            // One barrier per tile, on both waves: an empty half has its one empty segment.
+            asm volatile("s_waitcnt lgkmcnt(0)\n s_barrier" ::: "memory");
+            const uint8_t* const tile = lds + image;
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                half8 afrag[8];
+#pragma unroll
+                for (int r = 0; r < 8; r++)
+                    afrag[r] = *reinterpret_cast<const half8*>(tile + a_off[k] + r * 2048);
+                __builtin_amdgcn_sched_barrier(0);
+                if (k == 1 && s.tile > 0 && s.tile < ntile - 1) {  // behind this tile's reads, beside its MFMAs
+                    uint8_t* const half = lds + old_image + wave * (kTileBytes / 2) + lane * 16;
+#pragma unroll
+                    for (int i = 0; i < kTileBytes / 2 / (kWave * 16); i++)
+                        *reinterpret_cast<u32x4*>(half + i * kWave * 16) = u32x4{0u, 0u, 0u, 0u};
+                }
+#pragma unroll
+                for (int r = 0; r < 8; r++)
+#pragma unroll
+                    for (int cb = 0; cb < NB; cb++)
+                        acc[cb][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag[r], bfrag[slot][cb * 2 + k], acc[cb][r], 0, 0, 0);
+            }
+            old_image = image;
+            image = image == (kPairImages - 1) * kTileBytes ? 0 : image + kTileBytes;
+        };
+
+        Cur ci{0, 0};
+        static_for<D>([&](auto sc) {
+            constexpr int s = decltype(sc)::value;
+            Cur nx;
+            make_seg(ci, held[s], nx);
+            ci = nx;
+            issue(s, held[s]);
+        });
+        for (;;) {
+            static_for<D>([&](auto sc) {
+                constexpr int s = decltype(sc)::value;
+                consume(sc, held[s], std::integral_constant<int, (D - 1) * L>{});
+                Cur nx;
+                make_seg(ci, held[s], nx);
+                ci = nx;
+                issue(s, held[s]);
+            });
+            if (held[0].tile >= ntile)
+                break;
+        }
+        static_for<D>([&](auto sc) { land(decltype(sc)::value, std::integral_constant<int, 0>{}); });
+    };
+    if (ntile > 0) {
+        const int segments = segment_choice(__builtin_amdgcn_readlane(wreg, ntile) - __builtin_amdgcn_readlane(wreg, 0), ntile);
+        if (segments == 3)
+            stream_run(std::integral_constant<int, kVecPerLaneLong / 2>{});
+        else if (segments == 1)
+            stream_run(std::integral_constant<int, kVecPerLaneShort / 2>{});
+        else if (segments == 0)
+            stream_run(std::integral_constant<int, kVecPerLaneTiny / 2>{});
+        else
+            stream_run(std::integral_constant<int, kVecPerLane / 2>{});
+    }
+
+    // The output through an image that the last tile did not use (see above), 16 tokens at a time; `image`
+    // is the one behind the last tile's.
+    int mine = image + wave * kTileBytes;
+    mine = mine >= kPairImages * kTileBytes ? mine - kPairImages * kTileBytes : mine;
+    uint8_t* const stage = lds + mine;
+    _Float16* const oslab = out + (size_t)batch * M * NTOK + (size_t)rt * kTileRows;
+    constexpr int kTokStride = 272;
+#pragma unroll
+    for (int c = 0; c < NB; c++) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            half4 h;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                h[i] = static_cast<_Float16>(relu ? fmaxf(acc[c][r][i], 0.f) : acc[c][r][i]);
+            *reinterpret_cast<half4*>(stage + l15 * kTokStride + (r * 16 + q * 4) * 2) = h;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int e = i * kWave + lane, tok = e >> 4, part = e & 15;
+            const half8 v = *reinterpret_cast<const half8*>(stage + tok * kTokStride + part * 16);
+            *reinterpret_cast<half8*>(oslab + (size_t)(wave * (16 * NB) + c * 16 + tok) * ldo + part * 8) = v;
+        }
+    }
+}
+
 // C[n][m] = fp16(sum over slabs of float(W[s][n][m])) (csrc/Reduction_Kernel.cuh:36-46), 8 elements
 // per thread; rows8 = vector length / 8, ldc = elements between two vectors of C (slabs are
 // dense).  The slab loads of a thread are independent; they are issued eight at a time so
@@ -991,6 +1245,18 @@ int launch_spmm(hipStream_t stream, const void* items, const int* offsets, const
     return static_cast<int>(hipGetLastError());
 }
 
+int launch_pair(hipStream_t stream, const void* items, const int* offsets, const void* B, void* out, int M, int K, int split_k,
+                int ldb, int ldo, int relu)
+{
+    const int tiles = (K / kTileCols - 1) / split_k + 1;
+    if (split_k > 65535 || tiles >= kWave)  // (the offsets of a batch sit in one register, a lane each)
+        return static_cast<int>(hipErrorInvalidValue);
+    hipLaunchKernelGGL(tcsl_spmm_pair_kernel, dim3(M / kTileRows, split_k), dim3(2 * kWave), kPairImages * kTileBytes, stream,
+                       offsets, static_cast<const u32x4*>(items), static_cast<const _Float16*>(B), static_cast<_Float16*>(out), K,
+                       tiles, ldb, M, ldo, relu);
+    return static_cast<int>(hipGetLastError());
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -1000,7 +1266,8 @@ int launch_spmm(hipStream_t stream, const void* items, const int* offsets, const
 // mode 0: the W waves of a workgroup take W consecutive tile rows of one batch; with stage_b = 1
 //         (N <= 16) they share the batch's activation slice, staged once in LDS; with stage_b = 2
 //         (N = 32: 4 or 8 waves, N = 64: 4 waves) they walk the batch in step and share each
-//         activation tile through LDS;
+//         activation tile through LDS; with stage_b = 3 (N = 64, two waves) both work on one tile row,
+//         with half of the tokens each;
 // mode 1: the W waves of a workgroup split the batch of one tile row among themselves and
 //         add their results up in LDS (stage_b must be 0).
 // row_major: B is [K][N] and the output [M][N] instead of [N][K] and [N][M] (stage_b must be 0).
@@ -1025,6 +1292,11 @@ extern "C" int tcsl_launch_spmm(void* stream, const void* items, const int* offs
         return static_cast<int>(hipErrorInvalidValue);
     if (stage_b == 2 && (mode == 1 || row_major || !((N == 32 && (waves == 4 || waves == 8)) || (N == 64 && waves == 4))))
         return static_cast<int>(hipErrorInvalidValue);
+    if (stage_b == 3) {
+        if (mode != 0 || row_major || N != 64 || waves != 2 || fuse_page >= 0)
+            return static_cast<int>(hipErrorInvalidValue);
+        return launch_pair(s, items, offsets, B, out, M, K, split_k, ldb, ldo, relu);
+    }
     if (stage_b < 0 || stage_b > 2)
         return static_cast<int>(hipErrorInvalidValue);
     unsigned int* arrivals = nullptr;

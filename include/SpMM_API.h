@@ -256,7 +256,9 @@ SPMM_EXPORT int SpMM_SuggestSplitK_Bytes(int M_Global, int N_Global, int K_Globa
  *   Mode 0  the Waves waves of a workgroup take consecutive 128-row tile rows of one
  *           split-K batch (StageB = 1, up to 16 tokens: they share the batch's activation slice,
  *           staged once in LDS; StageB = 2, 32 tokens with 4 or 8 waves and 64 tokens with 4:
- *           they walk the batch in step and share each 64-column activation tile through LDS);
+ *           they walk the batch in step and share each 64-column activation tile through LDS;
+ *           LdsBytes = 49152 with two waves and 64 tokens: both work on every tile of one tile row,
+ *           with half of the tokens each, a launch shape of the planner's own);
  *   Mode 1  the Waves waves of a workgroup split the batch of one tile row among
  *           themselves and add their accumulators up in LDS.
  * Any output pointer may be NULL.  EstimatedUs is the cost model's figure for the whole

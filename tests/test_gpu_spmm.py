@@ -1006,3 +1006,42 @@ def test_shared_activation_tiles_rejects_other_shapes(spmm):
     for (N, mode, waves, row_major) in [(16, 0, 4, 0), (32, 0, 2, 0), (64, 0, 2, 0), (32, 1, 4, 0), (64, 0, 4, 1), (8, 0, 8, 0)]:
         with pytest.raises(spmm.SpMMError):
             spmm.SpMM_SplitK_API_Planned(None, z, z, z, z, 1024, N, 1024, z, 1, mode, waves, 2, row_major)
+
+
+@pytest.mark.parametrize("M,K,split_k,sparsity,flags", [
+    (128, 64, 1, 0.8, 0),          # one tile
+    (256, 64 * 2, 2, 0.8, 1),      # two batches of one tile, clamped by the reduction
+    (384, 64 * 6, 1, 0.5, 1),      # denser than one segment of a wave's half, clamped by the kernel
+    (512, 64 * 11, 4, 0.8, 0),     # batches of 3, 3, 3, 2
+    (512, 64 * 12, 2, 0.0, 0),     # dense: five segments of ten vectors a lane and more
+    (640, 64 * 5, 1, 0.97, 0),     # tiles of a few vectors: the second wave's half is empty
+    (1024, 64 * 6, 1, 0.999, 0),   # empty tiles
+    (128 * 65, 64 * 27, 5, 0.9, 1),   # two units on some compute units, batches of 6, 6, 6, 6, 3
+    (128 * 257, 64 * 27, 1, 0.85, 0),
+    (128 * 256, 64 * 6, 1, 0.7, 0),
+])
+def test_two_waves_per_unit_at_64_tokens(spmm, oracle, M, K, split_k, sparsity, flags):
+    """The launch shape whose two waves share every tile at 64 tokens, on strided operands: the planner takes
+    it here; its images rotate over three, its last two tiles are not cleared."""
+    torch = _torch()
+    N = 64
+    p = spmm.SpMM_PlanLaunch(M, N, K, split_k)
+    assert (p["mode"], p["waves"], p["stage_b"], p["lds_bytes"]) == (0, 2, 0, 49152)
+    A, B, items, offsets = make_case(spmm, M, K, N, sparsity, seed=M + K + split_k)
+    dev = torch.device("cuda:0")
+    ldb, ldc = K + 8, M + 16
+    wide = np.zeros((N, ldb), dtype=np.float16)
+    wide[:, :K] = B
+    d_items = torch.from_numpy(items.view(np.int32).copy()).to(dev)
+    d_offs = torch.from_numpy(offsets.copy()).to(dev)
+    d_B = torch.from_numpy(wide.view(np.int16).copy()).to(dev)
+    d_C = torch.full((N, ldc), float("nan"), dtype=torch.float16, device=dev)
+    d_W = torch.full((split_k, N, M), float("nan"), dtype=torch.float16, device=dev)
+    print(f"[gpu case] pairs M={M} K={K} split_k={split_k} sparsity={sparsity} flags={flags}", flush=True)
+    for _ in range(3):
+        spmm.SpMM_SplitK_API_Strided(torch.cuda.current_stream(), d_items, d_offs, d_B, ldb, d_C, ldc, M, N, K, d_W, split_k, flags)
+    torch.cuda.synchronize()
+    ref = oracle.gemm_f32(A, B)
+    C = d_C.cpu().numpy()
+    assert_close(C[:, :M], np.maximum(ref, 0) if flags & 1 else ref)
+    assert np.isnan(C[:, M:]).all()
