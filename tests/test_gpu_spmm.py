@@ -1045,3 +1045,33 @@ def test_two_waves_per_unit_at_64_tokens(spmm, oracle, M, K, split_k, sparsity, 
     C = d_C.cpu().numpy()
     assert_close(C[:, :M], np.maximum(ref, 0) if flags & 1 else ref)
     assert np.isnan(C[:, M:]).all()
+
+
+@pytest.mark.parametrize("split_k", [2, 3, 5, 6, 7, 9, 13, 17, 23, 25, 31, 32, 33, 40])
+@pytest.mark.parametrize("flags", [2, 3])
+def test_reduction_kernel_adds_any_number_of_slabs(spmm, split_k, flags):
+    """The reduction kernel's sums bit for bit: slabs of partial sums that the main kernel left, added in slab
+    order in 32 bits and rounded once, with and without the clamp, below, at and beyond the numbers of
+    slabs that it loads at once."""
+    torch = _torch()
+    M, K, N = 384, 64 * 40 * split_k, 16
+    if split_k > 8:
+        K = 64 * split_k
+    A, B, items, offsets = make_case(spmm, M, K, N, 0.9, seed=split_k)
+    dev = torch.device("cuda:0")
+    d_items = torch.from_numpy(items.view(np.int32).copy()).to(dev)
+    d_offs = torch.from_numpy(offsets.copy()).to(dev)
+    d_B = torch.from_numpy(np.ascontiguousarray(B).view(np.int16).copy()).to(dev)
+    d_C = torch.full((N, M + 8), float("nan"), dtype=torch.float16, device=dev)
+    d_W = torch.full((split_k, N, M), float("nan"), dtype=torch.float16, device=dev)
+    print(f"[gpu case] reduction of {split_k} slabs flags={flags}", flush=True)
+    spmm.SpMM_SplitK_API_Strided(torch.cuda.current_stream(), d_items, d_offs, d_B, K, d_C, M + 8, M, N, K, d_W, split_k, flags)
+    torch.cuda.synchronize()
+    want = torch.zeros((N, M), dtype=torch.float32)
+    for slab in d_W.cpu():
+        want += slab.float()
+    if flags & 1:
+        want.clamp_(min=0)
+    got = d_C.cpu()
+    assert torch.isfinite(want).all() and torch.equal(got[:, :M], want.half())
+    assert torch.isnan(got[:, M:].float()).all()
