@@ -210,7 +210,7 @@ double plan_cost_us(int M, int N, int K, int split_k, const LaunchPlan& p, doubl
     return total;
 }
 
-LaunchPlan plan_launch(int M, int N, int K, int split_k, bool row_major, double* cost_us, double tile_bytes)
+LaunchPlan plan_launch(int M, int N, int K, int split_k, bool row_major, double* cost_us, double tile_bytes, bool allow_pair)
 {
     // a measured optimum with this Split_K: of the weight's own density if the caller gave it, else of any
     if (const Tuned* t = find_tuned(M, N, K, split_k, tile_bytes > 0.0 ? density_table(tile_bytes) : -1)) {
@@ -262,7 +262,7 @@ LaunchPlan plan_launch(int M, int N, int K, int split_k, bool row_major, double*
     // Split_K: faster by 5 to 22 % and 0 to 30 % there (means 12 and 9 %); slower from seven to eleven tiles on
     // with one unit (0.97, then 0.92 to 0.55), and with more than two units (0.95).  The estimate stays
     // that of the shape that this replaces: it is what a Split_K is chosen by.
-    if (N == 64 && !row_major) {
+    if (N == 64 && !row_major && allow_pair) {
         const long units = static_cast<long>(M / kTileRows) * split_k;
         const long tiles = (K / kTileCols - 1) / split_k + 1;
         if (units <= kCUs ? tiles <= 6 : units <= 2 * kCUs && tiles <= 27) {

@@ -32,7 +32,9 @@ double plan_cost_us(int M, int N, int K, int split_k, const LaunchPlan& p, doubl
 
 // Best plan for a given Split_K; *cost_us (optional) receives its estimate.
 // row_major: B is [K][N] and C [M][N]; such calls cannot stage the activation slice.
-LaunchPlan plan_launch(int M, int N, int K, int split_k, bool row_major, double* cost_us, double tile_bytes = 0.0);
+// allow_pair: the plan may be a paired one.
+LaunchPlan plan_launch(int M, int N, int K, int split_k, bool row_major, double* cost_us, double tile_bytes = 0.0,
+                       bool allow_pair = true);
 
 // Best Split_K in 1..32 (with its plan) for the shape.
 int suggest_split_k(int M, int N, int K, LaunchPlan* plan, double tile_bytes = 0.0);

@@ -95,21 +95,21 @@ namespace {
 
 // Plans are a pure function of the shape; the last few are remembered per thread so that a
 // decode loop cycling over a handful of layer shapes never re-runs the model.
-tcsl::LaunchPlan cached_plan(int M, int N, int K, int Split_K, bool row_major)
+tcsl::LaunchPlan cached_plan(int M, int N, int K, int Split_K, bool row_major, bool allow_pair)
 {
     struct Entry {
         int M, N, K, S;
-        bool row_major;
+        bool row_major, allow_pair;
         tcsl::LaunchPlan plan;
     };
     constexpr int kEntries = 16;
     thread_local Entry cache[kEntries] = {};
     thread_local int next = 0;
     for (const Entry& e : cache)
-        if (e.M == M && e.N == N && e.K == K && e.S == Split_K && e.row_major == row_major)
+        if (e.M == M && e.N == N && e.K == K && e.S == Split_K && e.row_major == row_major && e.allow_pair == allow_pair)
             return e.plan;
-    const tcsl::LaunchPlan p = tcsl::plan_launch(M, N, K, Split_K, row_major, nullptr);
-    cache[next] = Entry{M, N, K, Split_K, row_major, p};
+    const tcsl::LaunchPlan p = tcsl::plan_launch(M, N, K, Split_K, row_major, nullptr, 0.0, allow_pair);
+    cache[next] = Entry{M, N, K, Split_K, row_major, allow_pair, p};
     next = (next + 1) % kEntries;
     return p;
 }
@@ -158,7 +158,9 @@ int launch_main(void* stream, const void* Compressed_A, const int* TileOffsets, 
                 int K, int Split_K, const CallOptions& o, int ldb, int ldo, bool relu, void* fused_out, long ldc,
                 bool* fused)
 {
-    const tcsl::LaunchPlan p = o.forced ? *o.forced : cached_plan(M, N, K, Split_K, o.row_major);
+    // (where this launch's sum would take an earlier launch's slabs along, a shape that leaves the sum to
+    // the reduction kernel costs a launch more than its own gain)
+    const tcsl::LaunchPlan p = o.forced ? *o.forced : cached_plan(M, N, K, Split_K, o.row_major, o.extra_slabs == 0);
     int page = -1;
     // Only the layout whose workgroup owns a single tile row fuses the reduction: its last arriver
     // adds up 128 rows.  In the row-sharing layout one workgroup would be left with W x 128 rows of
