@@ -176,6 +176,8 @@ __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* _
     //    ties), pointing at that bank's first zero position (:352-365).  Every wave works it out.
     const int real = size;  // of the bank, without pads
     const int count = __builtin_amdgcn_readlane(offscan::wave_inclusive_sum(lane < kBanks ? size : 0), 63);
+    if ((count + 3) / 4 * 4 != words)
+        return;  // these are not this tile's offsets (every wave sees the same count)
     for (int pad = (4 - count % 4) % 4; pad > 0; pad--) {
         const int low = half_wave_reduce(size << 5 | b, 0x7fffffff, [](int x, int y) { return x < y ? x : y; });
         size += (low & 31) == b ? 1 : 0;
