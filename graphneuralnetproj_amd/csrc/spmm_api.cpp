@@ -3,7 +3,6 @@
 // reached only through the tcsl_* launchers of spmm_kernels.hip and
 // tiled_csl_encode_device.hip and the a24_* launchers of a24_kernels.hip and a24_pack_device.hip.
 #include <cstdint>
-#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <mutex>
@@ -527,37 +526,35 @@ int a24_waves_for(int M, int split_k)
 
 A24Plan a24_default_plan(int M, int N, int K)
 {
-    // Waves that own two row blocks each and share the activation tile through LDS, and the split-K
-    // with the least estimated time for the finished result: a start per round of workgroups (256 of
-    // eight waves or 512 of four at a time), the units of a batch one after the other at a time per
-    // unit that grows with the tokens, with a second workgroup on the compute unit and with eight waves,
-    // or the records at the chip's rate where that is longer, and with more than one batch the sum of
-    // the slabs, inside the launch (up to 16 tokens) or by the reduction kernel.
-    // Constants: least regret over 72 shapes of 128 x 256 to 47104 x 16384, 50 to 70 % sparsity, four
-    // token counts, every split-K; half of them fitted, and checked on the other half, where the suggested
-    // split-K is 0.5 % slower than the best in the mean and 14 % at most.  (An estimate by bytes per compute
-    // unit alone, fitted on large shapes: 11 % and 56 %; 256 x 1024 at 64 tokens 1 -> 8 batches, 1.75 times faster.)
+    // From sweeps over the OPT-30B and OPT-66B shapes (N = 16 and 64, with and without the residual):
+    // waves that own two row blocks each and share the activation tile through LDS, and the split-K
+    // with the least estimated time for the finished result: rounds of workgroups (256 of eight
+    // waves or 512 of four at a time), each compute unit streaming its share of the records at one
+    // unit's rate plus a fixed cost per round, and the reduction kernel plus a cost per slab once
+    // there is more than one batch.  That picks what the sweeps found fastest: just under 256
+    // workgroups of eight waves or as many of four with half the slabs (FFN1 28672x7168, N = 16:
+    // four waves, one batch, no reduction: 36.0 us against 35.2 + 3 us), else e.g. 432 rather than
+    // 144 or 288.  With 64 tokens eight waves hide the matrix cores' and the LDS's latencies better
+    // (FFN1: 41 us + reduction against 46).
+    // Small matrices would run faster from more batches (256 x 1024 at 64 tokens, eight instead of one: 1.75
+    // times), but a batch's partial sums are rounded to fp16: the error against 64 bits goes from 2.1e-4 to
+    // 3.1e-4, which is the caller's to choose (any Split_K is taken), not this suggestion's.
     A24Plan p{2, 4, 1, 1};
     const int units = K / a24::kUnitCols;
-    const double unit_us = N <= 16 ? 0.578 : N <= 32 ? 0.683 : 1.375;
-    constexpr double kRoundUs = 4.286, kShared = 0.840, kEightWaves = 1.697, kChipBytesPerUs = 5.25e6, kNorm = 4.8;
-    constexpr double kInLaunchUs = 0.323, kInLaunchSlabUs = 0.126, kReduceUs = 2.363, kReduceSlabUs = 0.079, kSlabBytesPerUs = 5.05e6;
-    const double chip_us = static_cast<double>(a24::bytes(M, K)) / kChipBytesPerUs;
+    const double bytes = static_cast<double>(a24::bytes(M, K));
+    constexpr double kUnitBytesPerUs = 25.4e3, kRoundUs = 6.0, kReduceUs = 3.0, kSlabUs = 0.8, kFourWaves64 = 1.15;
     double best = 0.0;
     for (int s = 1; s <= 32 && s <= units; s++) {
         const int per = (units + s - 1) / s;
-        if (static_cast<long>(per) * (s - 1) >= units)
-            continue;  // an empty last batch
+        if ((s > 1 && per < 2) || static_cast<long>(per) * (s - 1) >= units)
+            continue;  // batches of one unit, or an empty last batch
         const int waves = a24_waves_for(M, s);
         const long n = static_cast<long>(M / (16 * p.row_blocks * waves)) * s;
         const long at_once = waves == 8 ? 256 : 512;
         const long rounds = (n + at_once - 1) / at_once;
-        const long beside = ((n < at_once ? n : at_once) + 255) / 256 - 1;  // further workgroups on a compute unit
-        const double stream = rounds * per * unit_us * (1.0 + kShared * beside) * (waves == 8 ? kEightWaves : 1.0);
-        double cost = rounds * kRoundUs + std::pow(std::pow(stream, kNorm) + std::pow(chip_us, kNorm), 1.0 / kNorm);
-        if (s > 1)
-            cost += (N <= 16 ? kInLaunchUs + kInLaunchSlabUs * s : kReduceUs + kReduceSlabUs * s) +
-                    2.0 * (2.0 * s + 1.0) * M * N / kSlabBytesPerUs;
+        const long per_unit = ((n < at_once ? n : at_once) + 255) / 256;  // workgroups that share a compute unit
+        const double stream = bytes / n * per_unit / kUnitBytesPerUs * (N == 64 && waves == 4 ? kFourWaves64 : 1.0);
+        const double cost = rounds * (stream + kRoundUs) + (s > 1 ? kReduceUs + kSlabUs * s : 0.0);
         if (best == 0.0 || cost < best * 0.999) {
             best = cost;
             p.split_k = s;

@@ -877,23 +877,21 @@ def test_device_residual_lists_edges(spmm, oracle, M, K, sparsity):
     assert np.array_equal(words.cpu().numpy().view(np.uint32), want_words)
 
 
-@pytest.mark.parametrize("M,K,N,sparsity", [(256, 1024, 64, 0.5), (128, 2944, 8, 0.68), (128, 128 * 33, 16, 0.5), (128, 2048, 32, 0.6),
-                                            (2176, 1152, 64, 0.6)])
-def test_suggested_batches_of_small_matrices(spmm, oracle, M, K, N, sparsity):
-    """The split that HeteroSparse_SuggestSplitK gives small matrices, down to batches of one unit each,
-    summed inside the launch (up to 16 tokens) and by the reduction kernel, against the oracle."""
+@pytest.mark.parametrize("M,K,N,sparsity,split_k", [(256, 1024, 64, 0.5, 8), (128, 2944, 8, 0.68, 12), (128, 128 * 33, 16, 0.5, 11),
+                                                    (128, 2048, 32, 0.6, 16), (2176, 1152, 64, 0.6, 9)])
+def test_batches_of_one_unit_and_few(spmm, oracle, M, K, N, sparsity, split_k):
+    """Small matrices in many batches, down to one unit each, summed inside the launch (up to 16 tokens) and by
+    the reduction kernel, against the oracle."""
     torch = _torch()
-    s = spmm.HeteroSparse_SuggestSplitK(M, N, K)
-    assert s > 1
     A = spmm.synth_weights(M, K, sparsity, False, seed=M + K + N)
     B = spmm.synth_activations(N, K, seed=5)
     d_A = torch.from_numpy(A.view(np.int16).copy()).to("cuda:0").view(torch.float16)
     packed, residual = spmm.split_pack_on_device(d_A)
     words, offsets, longest = spmm.pack_residual_on_device(residual)
     d_C = torch.full((N, M), float("nan"), dtype=torch.float16, device="cuda:0")
-    d_W = torch.full((s, N, M), float("nan"), dtype=torch.float16, device="cuda:0")
-    print(f"[gpu case] suggested split M={M} K={K} N={N} split_k={s} longest={longest}", flush=True)
+    d_W = torch.full((split_k, N, M), float("nan"), dtype=torch.float16, device="cuda:0")
+    print(f"[gpu case] small batches M={M} K={K} N={N} split_k={split_k} longest={longest}", flush=True)
     for _ in range(2):
-        spmm.HeteroSparse_Fused_SpMM_API(torch.cuda.current_stream(), packed, words, offsets, longest, _dev(B), d_C, M, N, K, d_W, s)
+        spmm.HeteroSparse_Fused_SpMM_API(torch.cuda.current_stream(), packed, words, offsets, longest, _dev(B), d_C, M, N, K, d_W, split_k)
     torch.cuda.synchronize()
     assert_close(d_C.cpu().numpy(), oracle.gemm_f32(A, B))
