@@ -1127,47 +1127,51 @@ __global__ __launch_bounds__(2 * kWave, 2) void tcsl_spmm_pair_kernel(const int*
     }
 }
 
+// sum += slabs s .. s + COUNT - 1, in slab order.  TOGETHER: every load is issued before the first one is waited
+// for; else the compiler has eight or so in flight, and adds up what has come meanwhile.
+template<int COUNT, bool TOGETHER>
+__device__ __forceinline__ void add_slabs(float (&sum)[8], const _Float16* w0, long mn, int s)
+{
+    half8 w[COUNT];
+#pragma unroll
+    for (int u = 0; u < COUNT; u++)
+        w[u] = __builtin_nontemporal_load(reinterpret_cast<const half8*>(w0 + (size_t)(s + u) * mn));
+    if constexpr (TOGETHER)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < COUNT; u++)
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            sum[j] += static_cast<float>(w[u][j]);
+}
+
 // C[n][m] = fp16(sum over slabs of float(W[s][n][m])) (csrc/Reduction_Kernel.cuh:36-46), 8 elements
 // per thread; rows8 = vector length / 8, ldc = elements between two vectors of C (slabs are
-// dense).  Latency bound (a few MB in all): the loads of FLIGHT slabs are in flight together, the last
-// slab's repeated where there are fewer, and are added in slab order, as the reference does.  The launch
-// takes the smallest FLIGHT of 2, 3, 4, 6, 8, 12, 16, 24, 32 that holds all slabs, so nearly every call pays
-// one trip to memory.  (Eight at a time and the rest one after the other, a trip each: whole calls on
-// 1408 x 5824 at 32 tokens and 90 % sparsity with 23 slabs 11.1 us, now 9.5; 2048 x 2048 at 16 tokens
-// with seven 9.5, now 8.3.)
-template<int FLIGHT>
+// dense).  Slabs are added in their order, as the reference does: CHUNK at a time, then REST at a time,
+// then one by one.
+// A small output is bound by the trips to memory: CHUNK = 16 and the rest in one trip, every load of a trip in
+// flight together, none without a use.  A large one is bound by bandwidth, and many loads a lane cost
+// occupancy: CHUNK = 8.  The launch has the rule.  Whole calls: 1408 x 64 tokens with 23 slabs, eight at a time and
+// the rest one by one 14.3 us, now 12.3; 7168 x 16 tokens with seven 9.2, now 7.5; 12288 x 32 tokens with 17
+// 11.7, now 11.6 (24 loads, the last slab's repeated: 12.7); 49152 x 64 tokens with 25 96.8 (32 loads: 108).
+template<int CHUNK, int REST>
 __global__ __launch_bounds__(64) void tcsl_reduce_kernel(_Float16* __restrict__ C, const _Float16* __restrict__ W,
                                                         long mn8, long mn, int rows8, long ldc, int split_k, int relu)
 {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= mn8)
         return;
+    constexpr bool TOGETHER = CHUNK > 8;
     const _Float16* w0 = W + i * 8;
     float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < split_k; s += FLIGHT) {
-        half8 w[FLIGHT];
-        if (s + FLIGHT <= split_k) {
-#pragma unroll
-            for (int u = 0; u < FLIGHT; u++)
-                w[u] = __builtin_nontemporal_load(reinterpret_cast<const half8*>(w0 + (size_t)(s + u) * mn));
-        } else {
-#pragma unroll
-            for (int u = 0; u < FLIGHT; u++)
-                w[u] = __builtin_nontemporal_load(
-                    reinterpret_cast<const half8*>(w0 + (size_t)(s + u < split_k ? s + u : split_k - 1) * mn));
-            __builtin_amdgcn_sched_barrier(0);
-            // (a sum that began at +0 is never -0: adding +0 to it changes nothing)
-#pragma unroll
-            for (int u = 1; u < FLIGHT; u++) {
-                const u32x4 keep = s + u < split_k ? u32x4{~0u, ~0u, ~0u, ~0u} : u32x4{0u, 0u, 0u, 0u};
-                w[u] = __builtin_bit_cast(half8, __builtin_bit_cast(u32x4, w[u]) & keep);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < FLIGHT; u++)
-#pragma unroll
-            for (int j = 0; j < 8; j++)
-                sum[j] += static_cast<float>(w[u][j]);
+    int s = 0;
+    for (; s + CHUNK <= split_k; s += CHUNK)
+        add_slabs<CHUNK, TOGETHER>(sum, w0, mn, s);
+    if constexpr (REST > 0) {  // the launch's REST is split_k % CHUNK
+        add_slabs<REST, TOGETHER>(sum, w0, mn, s);
+    } else {
+        for (; s < split_k; s++)
+            add_slabs<1, TOGETHER>(sum, w0, mn, s);
     }
     half8 o;
 #pragma unroll
@@ -1175,6 +1179,14 @@ __global__ __launch_bounds__(64) void tcsl_reduce_kernel(_Float16* __restrict__ 
         o[j] = static_cast<_Float16>(relu ? fmaxf(sum[j], 0.f) : sum[j]);
     const long n = i / rows8, m8 = i - n * rows8;
     *reinterpret_cast<half8*>(C + n * ldc + m8 * 8) = o;
+}
+
+// The kernel that adds REST = rest of CHUNK slabs in one trip (rest = 0: whatever is left, one by one).
+template<int CHUNK, int... REST>
+auto* reduce_kernel(int rest, std::integer_sequence<int, REST...>)
+{
+    static decltype(&tcsl_reduce_kernel<CHUNK, 0>) const table[] = {tcsl_reduce_kernel<CHUNK, REST>...};
+    return table[rest];
 }
 
 // Plain streaming copy, used only to calibrate hardware counters against a
@@ -1358,15 +1370,12 @@ extern "C" int tcsl_launch_reduce(void* stream, void* C, const void* W, long row
     const long blocks = (mn8 + 63) / 64;
     if (blocks < 1 || blocks > 0x7fffffffL || rows / 8 > 0x7fffffffL)
         return static_cast<int>(hipErrorInvalidValue);
-    auto* const kernel = split_k <= 2    ? tcsl_reduce_kernel<2>
-                         : split_k <= 3  ? tcsl_reduce_kernel<3>
-                         : split_k <= 4  ? tcsl_reduce_kernel<4>
-                         : split_k <= 6  ? tcsl_reduce_kernel<6>
-                         : split_k <= 8  ? tcsl_reduce_kernel<8>
-                         : split_k <= 12 ? tcsl_reduce_kernel<12>
-                         : split_k <= 16 ? tcsl_reduce_kernel<16>
-                         : split_k <= 24 ? tcsl_reduce_kernel<24>
-                                         : tcsl_reduce_kernel<32>;
+    // One wave to a workgroup.  Up to 1024 (four to a compute unit) 16 slabs a trip are no slower at any number of
+    // slabs from 2 to 32 (896 waves: 15 slabs 17.5 -> 15.9 us, 25 slabs 24.7 -> 24.5); beyond, eight (1536
+    // waves, 16 slabs: 19.4 us, in one trip 19.8; 6144 waves, 13 slabs: 52.9, 54.1).  There a rest behind 16 slabs
+    // goes one by one: in one trip it measured 1 % slower at 3584 waves.
+    auto* const kernel = blocks <= 1024 ? reduce_kernel<16>(split_k % 16, std::make_integer_sequence<int, 16>{})
+                                        : reduce_kernel<8>(split_k < 16 ? split_k % 8 : 0, std::make_integer_sequence<int, 8>{});
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(64), 0, static_cast<hipStream_t>(stream),
                        static_cast<_Float16*>(C), static_cast<const _Float16*>(W), mn8, mn, static_cast<int>(rows / 8),
                        ldc, split_k, relu);

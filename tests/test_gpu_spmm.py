@@ -1075,3 +1075,28 @@ def test_reduction_kernel_adds_any_number_of_slabs(spmm, split_k, flags):
     got = d_C.cpu()
     assert torch.isfinite(want).all() and torch.equal(got[:, :M], want.half())
     assert torch.isnan(got[:, M:].float()).all()
+
+
+@pytest.mark.parametrize("split_k", [2, 5, 8, 9, 15, 16, 17, 23, 24])
+def test_reduction_kernel_adds_slabs_of_large_outputs(spmm, split_k):
+    """The reduction kernel on an output beyond the 1024 workgroups (of 64 x 8 values) up to which 16 slabs are
+    loaded at once, bit for bit, on strided C: fewer than eight slabs, eights with a rest in one trip, and
+    from 16 on one by one."""
+    torch = _torch()
+    M, K, N = 128 * 65, 64 * split_k, 64
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(split_k)
+    W = torch.randn((M, K), generator=gen, device=dev).mul_(torch.rand((M, K), generator=gen, device=dev) < 0.05).half()
+    items, offs = spmm.encode_on_device(W)
+    d_B = torch.randn((N, K), generator=gen, device=dev).half()
+    d_C = torch.full((N, M + 8), float("nan"), dtype=torch.float16, device=dev)
+    d_W = torch.full((split_k, N, M), float("nan"), dtype=torch.float16, device=dev)
+    print(f"[gpu case] reduction of {split_k} large slabs", flush=True)
+    spmm.SpMM_SplitK_API_Strided(torch.cuda.current_stream(), items, offs, d_B, K, d_C, M + 8, M, N, K, d_W, split_k, 2)
+    torch.cuda.synchronize()
+    want = torch.zeros((N, M), dtype=torch.float32)
+    for slab in d_W.cpu():
+        want += slab.float()
+    got = d_C.cpu()
+    assert torch.isfinite(want).all() and torch.equal(got[:, :M], want.half())
+    assert torch.isnan(got[:, M:].float()).all()
