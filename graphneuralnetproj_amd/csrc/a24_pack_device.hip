@@ -333,12 +333,13 @@ __global__ __launch_bounds__(kEmitWaves * 64, 8) void a24_residual_emit_kernel(c
             s += __popcll(before & planes[bit]) << bit;
         start[i] = s;
         reinterpret_cast<uint8_t*>(sorted[li])[__popcll(before)] = static_cast<uint8_t>(count);
-        // (a block with more kept values than a residual can hold is not this format's input: nothing is written)
-        const bool dealt = n > 64 && n <= kMaxListWords;
+        // (a block with more kept values than a residual can hold is not this format's input: nothing is written,
+        // nor where the offsets are not those of this matrix: the words would land in other lists' room or behind all)
+        int at = offsets[list];
+        const bool fits = n <= kMaxListWords && n == offsets[list + 1] - at;
         if (L == 0)
-            length[li] = dealt ? n : 0;
-        if (n > 0 && n <= 64) {  // in row-major order
-            int at = offsets[list];
+            length[li] = fits && n > 64 ? n : 0;
+        if (fits && n > 0 && n <= 64) {  // in row-major order
 #pragma unroll
             for (int half = 0; half < 2; half++) {
 #pragma unroll

@@ -436,7 +436,8 @@ SPMM_EXPORT int HeteroSparse_A1_Partials(void* stream, const void* Packed_A1, co
  * Both only enqueue kernels on `stream`; read T and the longest list back (after synchronising) to
  * size the second buffer, or allocate the worst case M*K/2 + 64 words up front.  A2_d must be a
  * residual: at most two kept values in every group of four, hence at most 1024 per 16 x 128 block
- * (a block that holds more gets no words; *LongestList_d shows it).  With T = -1 the second
+ * (a block that holds more gets no words; *LongestList_d shows it), and neither does a block whose number of
+ * kept values is not what Offsets_d has room for (offsets of another matrix).  With T = -1 the second
  * step writes nothing at all: check T before trusting Words_d.  Return a hipError_t value;
  * hipErrorInvalidValue for M % 128, K % 128 or null pointers.
  */

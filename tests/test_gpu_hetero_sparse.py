@@ -895,3 +895,43 @@ def test_batches_of_one_unit_and_few(spmm, oracle, M, K, N, sparsity, split_k):
         spmm.HeteroSparse_Fused_SpMM_API(torch.cuda.current_stream(), packed, words, offsets, longest, _dev(B), d_C, M, N, K, d_W, split_k)
     torch.cuda.synchronize()
     assert_close(d_C.cpu().numpy(), oracle.gemm_f32(A, B))
+
+
+@pytest.mark.parametrize("M,K", [(256, 1280), (4096, 8320)])  # lists for the kernel of eight a workgroup, and of 32
+def test_device_residual_lists_with_offsets_of_another_matrix(spmm, M, K):
+    """The second step of the packing, given offsets of a matrix that has fewer words in some blocks and more in
+    others: blocks whose counts agree get their words, the room of all others and what lies behind the last
+    list stay as they were."""
+    import ctypes
+
+    torch = _torch()
+    dev = torch.device("cuda:0")
+    A = torch.from_numpy(spmm.synth_weights(M, K, 0.6, False, seed=3).view(np.int16).copy()).to(dev).view(torch.float16)
+    _, A2 = spmm.split_pack_on_device(A)
+    words, offsets, _ = spmm.pack_residual_on_device(A2)
+    other = A2.clone()
+    block = torch.zeros((M // 16, K // 128), dtype=torch.bool, device=dev)
+    block.view(-1)[::3] = True    # emptied
+    grown = torch.zeros_like(block)
+    grown.view(-1)[1::3] = True   # two of every four everywhere: the longest list
+    spread = lambda m: m.repeat_interleave(16, 0).repeat_interleave(128, 1)  # noqa: E731
+    other[spread(block)] = 0
+    two = torch.tensor([1.0, 2.0, 0.0, 0.0], dtype=torch.float16, device=dev).repeat(K // 4).expand(M, K)
+    other = torch.where(spread(grown), two, other).contiguous()
+    total = int(offsets[-1].item())
+    mark = 0x5A5A5A5A
+    out = torch.full((total + 64 + 8192,), mark, dtype=torch.int32, device=dev)
+    lib = spmm.load_library()
+    print(f"[gpu case] residual words with foreign offsets M={M} K={K}", flush=True)
+    rc = lib.HeteroSparse_DevicePackA2_Words(ctypes.c_void_p(torch.cuda.current_stream().cuda_stream or None),
+                                             ctypes.c_void_p(other.data_ptr()), M, K, ctypes.c_void_p(offsets.data_ptr()),
+                                             ctypes.c_void_p(out.data_ptr()))
+    assert rc == 0
+    torch.cuda.synchronize()
+    # lists are numbered ((rb / 8) * units + u) * 8 + rb % 8
+    order = lambda m: m.view(M // 128, 8, K // 128).transpose(1, 2).reshape(-1)  # noqa: E731
+    same = (~order(block | grown)).cpu().numpy()
+    o, want, got = offsets.cpu().numpy(), words.cpu().numpy(), out.cpu().numpy()
+    keep = np.repeat(same, np.diff(o))
+    assert np.array_equal(got[:total], np.where(keep, want[:total], mark))
+    assert (got[total:total + 64] == 0).all() and (got[total + 64:] == mark).all()
