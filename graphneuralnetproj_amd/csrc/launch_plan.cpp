@@ -258,14 +258,15 @@ LaunchPlan plan_launch(int M, int N, int K, int split_k, bool row_major, double*
     if (cost_us)
         *cost_us = best_cost;
     // 64 tokens: two waves to a work unit where a compute unit has one unit of up to six tiles, or two
-    // of up to 27.  Measured on 56 shapes of 128 x 256 to 47104 x 16384 at 65 to 92 % sparsity, every
-    // Split_K: faster by 5 to 22 % and 0 to 30 % there (means 12 and 9 %); slower from seven to eleven tiles on
-    // with one unit (0.97, then 0.92 to 0.55), and with more than two units (0.95).  The estimate stays
-    // that of the shape that this replaces: it is what a Split_K is chosen by.
+    // of three to 27.  Measured on 612 calls there, 128 x 64 to 47104 x 1728 and Split_K 1 to 32 at 60 to 95 % sparsity,
+    // against the shape that the model picks: 1.006 to 1.54 times as fast (mean 1.24) with one unit, 1.004 to 1.41
+    // (1.12) with two.  Slower from seven to eleven tiles on with one unit (0.97, then 0.92 to 0.55), with two
+    // units of one or two tiles (0.92 to 1.1: 47104 x 64 6.5 us, 7.1 in pairs), and with more than two units
+    // (0.95).  The estimate stays that of the shape that this replaces: it is what a Split_K is chosen by.
     if (N == 64 && !row_major && allow_pair) {
         const long units = static_cast<long>(M / kTileRows) * split_k;
         const long tiles = (K / kTileCols - 1) / split_k + 1;
-        if (units <= kCUs ? tiles <= 6 : units <= 2 * kCUs && tiles <= 27) {
+        if (units <= kCUs ? tiles <= 6 : units <= 2 * kCUs && tiles >= 3 && tiles <= 27) {
             LaunchPlan pair{0, 2, 0, static_cast<unsigned>(3 * kTileLds)};
             pair.paired = true;
             return pair;

@@ -185,6 +185,20 @@ def test_planner_gives_runnable_plans(spmm):
         spmm.SpMM_PlanLaunch(1024, 12, 1024, 1)
 
 
+def test_planner_pairs_waves_only_where_that_is_faster(spmm):
+    """64 tokens: two waves share a unit's tiles with up to 256 units of up to six tiles or up to 512 of three to 27;
+    batches of one or two tiles on more than 256 units ran slower in pairs (47104 x 64 6.5 -> 7.1 us)."""
+    def paired(M, K, S):
+        p = spmm.SpMM_PlanLaunch(M, 64, K, S)
+        return (p["mode"], p["waves"], p["lds_bytes"]) == (0, 2, 3 * 16384)
+
+    for M, K, S in [(47104, 64, 1), (47104, 128, 1), (8192, 512, 8), (8192, 1024, 8), (4096, 1024, 16), (32896, 64 * 2, 1),
+                    (512, 64 * 7, 1), (128 * 513, 64 * 3, 1), (128 * 257, 64 * 28, 1)]:
+        assert not paired(M, K, S), (M, K, S)
+    for M, K, S in [(128, 64, 1), (32768, 64, 1), (32768, 384, 1), (32896, 192, 1), (128 * 512, 64 * 27, 1), (8192, 64 * 24, 8)]:
+        assert paired(M, K, S), (M, K, S)
+
+
 def test_planner_uses_every_compute_unit_on_the_headline_shapes(spmm):
     # one round of workgroups, at least 200 of them, for the big OPT layers at N = 16
     for (M, K) in [(28672, 7168), (7168, 28672), (36864, 9216), (9216, 36864)]:
