@@ -135,6 +135,10 @@ bool complete_plan(int N, int K, int split_k, bool row_major, LaunchPlan& p)
             if (row_major || !((N == 32 && (p.waves == 4 || p.waves == 8)) || (N == 64 && p.waves == 4)))
                 return false;
             lds += 2L * N * 128;
+        } else if (p.stage_b == 3) {  // two waves on every tile, three images; a batch's offsets sit in one register
+            if (row_major || N != 64 || p.waves != 2 || tiles > 63)
+                return false;
+            lds = 3 * kTileLds;
         } else if (p.stage_b != 0) {
             return false;
         }
@@ -266,11 +270,10 @@ LaunchPlan plan_launch(int M, int N, int K, int split_k, bool row_major, double*
     if (N == 64 && !row_major && allow_pair) {
         const long units = static_cast<long>(M / kTileRows) * split_k;
         const long tiles = (K / kTileCols - 1) / split_k + 1;
-        if (units <= kCUs ? tiles <= 6 : units <= 2 * kCUs && tiles >= 3 && tiles <= 27) {
-            LaunchPlan pair{0, 2, 0, static_cast<unsigned>(3 * kTileLds)};
-            pair.paired = true;
+        LaunchPlan pair{0, 2, 3, 0};
+        if ((units <= kCUs ? tiles <= 6 : units <= 2 * kCUs && tiles >= 3 && tiles <= 27) &&
+            complete_plan(N, K, split_k, row_major, pair))
             return pair;
-        }
     }
     return best;
 }

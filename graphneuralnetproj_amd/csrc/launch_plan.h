@@ -10,15 +10,13 @@ namespace tcsl {
 // separate_reduction (mode 1, Split_K > 1): the slabs of partial sums are added up by the reduction
 //         kernel instead of by the last workgroup of each tile row inside the launch (mode 0 always
 //         uses the reduction kernel).
-// paired (mode 0, 2 waves, 64 tokens): both waves work on every tile of one tile row, with 32 tokens each;
-//         only the planner makes such a plan.
+// stage_b = 3 (mode 0, 2 waves, 64 tokens): both waves work on every tile of one tile row, with 32 tokens each.
 struct LaunchPlan {
     int mode;
     int waves;
     int stage_b;
     unsigned lds_bytes;
     bool separate_reduction = false;
-    bool paired = false;
 };
 
 // True (and lds_bytes filled in) when the kernels can run this shape.
@@ -32,7 +30,7 @@ double plan_cost_us(int M, int N, int K, int split_k, const LaunchPlan& p, doubl
 
 // Best plan for a given Split_K; *cost_us (optional) receives its estimate.
 // row_major: B is [K][N] and C [M][N]; such calls cannot stage the activation slice.
-// allow_pair: the plan may be a paired one.
+// allow_pair: the plan may have stage_b = 3.
 LaunchPlan plan_launch(int M, int N, int K, int split_k, bool row_major, double* cost_us, double tile_bytes = 0.0,
                        bool allow_pair = true);
 

@@ -189,7 +189,7 @@ int launch_main(void* stream, const void* Compressed_A, const int* TileOffsets, 
             dense_waves = p.waves;
         }
     }
-    int rc = tcsl_launch_spmm(stream, Compressed_A, TileOffsets, B, out, M, N, K, Split_K, run.mode, run.waves, run.paired ? 3 : run.stage_b,
+    int rc = tcsl_launch_spmm(stream, Compressed_A, TileOffsets, B, out, M, N, K, Split_K, run.mode, run.waves, run.stage_b,
                               o.row_major ? 1 : 0, run.lds_bytes, ldb, ldo,
                               (relu && (Split_K == 1 || page >= 0) ? 1 : 0)  // slabs of partial sums are never clamped
                                   | (page >= 0 ? o.extra_slabs << 8 : 0),
@@ -305,7 +305,7 @@ extern "C" int SpMM_PlanLaunch(int M, int N, int K, int Split_K, int* Mode, int*
     if (Waves)
         *Waves = p.waves;
     if (StageB)
-        *StageB = p.stage_b;
+        *StageB = p.stage_b == 3 ? 0 : p.stage_b;  // (told apart by LdsBytes)
     if (LdsBytes)
         *LdsBytes = static_cast<int>(p.lds_bytes);
     if (EstimatedUs)

@@ -257,12 +257,13 @@ SPMM_EXPORT int SpMM_SuggestSplitK_Bytes(int M_Global, int N_Global, int K_Globa
  *           split-K batch (StageB = 1, up to 16 tokens: they share the batch's activation slice,
  *           staged once in LDS; StageB = 2, 32 tokens with 4 or 8 waves and 64 tokens with 4:
  *           they walk the batch in step and share each 64-column activation tile through LDS;
- *           LdsBytes = 49152 with two waves and 64 tokens: both work on every tile of one tile row,
- *           with half of the tokens each, a launch shape of the planner's own);
+ *           64 tokens with two waves and LdsBytes = 49152: both work on every tile of one tile row,
+ *           with half of the tokens each; StageB is 0 here, and 3 for SpMM_SplitK_API_Planned);
  *   Mode 1  the Waves waves of a workgroup split the batch of one tile row among
  *           themselves and add their accumulators up in LDS.
  * Any output pointer may be NULL.  EstimatedUs is the cost model's figure for the whole
- * call.  Returns 0, or -1 for a shape the kernels do not take.  The reference has one
+ * call (in the last shape of Mode 0 that of the shape which the planner would take otherwise).
+ * Returns 0, or -1 for a shape the kernels do not take.  The reference has one
  * fixed block shape (csrc/SpMM_API.cu:25-71) and nothing like this.
  */
 SPMM_EXPORT int SpMM_PlanLaunch(int M_Global, int N_Global, int K_Global, int Split_K, int* Mode, int* Waves, int* StageB,
@@ -283,8 +284,8 @@ SPMM_EXPORT int SpMM_PlanReductionInLaunch(int M_Global, int N_Global, int K_Glo
  * SpMM_SplitK_API with the launch shape given by the caller instead of the planner
  * (for tuning a table of plans on the target machine, and for tests).  Returns
  * hipErrorInvalidValue when the shape does not fit (Waves above 8, or 4 for N = 64;
- * StageB with Mode 1 or RowMajor, StageB = 1 with N > 16, StageB = 2 outside the shapes above;
- * more than 160 KiB of LDS).  RowMajor != 0 selects
+ * StageB with Mode 1 or RowMajor, StageB = 1 with N > 16, StageB = 2 outside the shapes above, StageB = 3
+ * with other than two waves, 64 tokens and batches of up to 63 tiles; more than 160 KiB of LDS).  RowMajor != 0 selects
  * the operand layout of SpMM_SplitK_API_RowMajor; Flags as for SpMM_SplitK_API_Strided.  No
  * counterpart in the reference.
  */

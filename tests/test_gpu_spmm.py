@@ -1047,6 +1047,44 @@ def test_two_waves_per_unit_at_64_tokens(spmm, oracle, M, K, split_k, sparsity, 
     assert np.isnan(C[:, M:]).all()
 
 
+@pytest.mark.parametrize("M,K,split_k,sparsity,flags", [(512, 64 * 11, 4, 0.8, 0), (384, 64 * 6, 1, 0.6, 1),   # the planner's
+                                                        (512, 64 * 63, 1, 0.8, 0), (256, 64 * 83, 2, 0.9, 1),  # longer batches
+                                                        (128 * 515, 64 * 2, 1, 0.7, 0)])                       # more units
+def test_paired_launch_on_request(spmm, oracle, M, K, split_k, sparsity, flags):
+    """SpMM_SplitK_API_Planned launches the shape whose two waves share every tile as StageB = 3: the planner's own calls bit
+    for bit, and beyond its rule, up to 63 tiles a batch, against the oracle; other forms are refused."""
+    torch = _torch()
+    N, dev = 64, torch.device("cuda:0")
+    A, B, items, offsets = make_case(spmm, M, K, N, sparsity, seed=M + K)
+    d_items = torch.from_numpy(items.view(np.int32).copy()).to(dev)
+    d_offs = torch.from_numpy(offsets.copy()).to(dev)
+    d_B = torch.from_numpy(np.ascontiguousarray(B).view(np.int16).copy()).to(dev).view(torch.float16)
+    d_W = torch.full((split_k, N, M), float("nan"), dtype=torch.float16, device=dev)
+
+    def call(*plan):
+        C = torch.full((N, M), float("nan"), dtype=torch.float16, device=dev)
+        print(f"[gpu case] paired on request M={M} K={K} split_k={split_k} plan={plan}", flush=True)
+        if plan:
+            spmm.SpMM_SplitK_API_Planned(torch.cuda.current_stream(), d_items, d_offs, d_B, C, M, N, K, d_W, split_k, *plan, flags)
+        else:
+            spmm.SpMM_SplitK_API_Strided(torch.cuda.current_stream(), d_items, d_offs, d_B, K, C, M, M, N, K, d_W, split_k, flags)
+        torch.cuda.synchronize()
+        return C.cpu().numpy()
+
+    C = call(0, 2, 3, 0)
+    ref = oracle.gemm_f32(A, B)
+    assert_close(C, np.maximum(ref, 0) if flags & 1 else ref)
+    if spmm.SpMM_PlanLaunch(M, N, K, split_k)["paired"]:
+        assert np.array_equal(C.view(np.uint16), call().view(np.uint16))
+    for plan in ((0, 1, 3, 0), (0, 4, 3, 0), (1, 2, 3, 0), (0, 2, 3, 1), (0, 2, 4, 0)):
+        with pytest.raises(spmm.SpMMError):
+            call(*plan)
+    with pytest.raises(spmm.SpMMError):  # 64 tiles a batch
+        spmm.SpMM_SplitK_API_Planned(None, d_items, d_offs, d_B, d_B, 128, N, 64 * 64, d_W, 1, 0, 2, 3)
+    with pytest.raises(spmm.SpMMError):
+        spmm.SpMM_SplitK_API_Planned(None, d_items, d_offs, d_B, d_B, 128, 32, 64, d_W, 1, 0, 2, 3)
+
+
 @pytest.mark.parametrize("split_k", [2, 3, 5, 6, 7, 9, 13, 17, 23, 25, 31, 32, 33, 40])
 @pytest.mark.parametrize("flags", [2, 3])
 def test_reduction_kernel_adds_any_number_of_slabs(spmm, split_k, flags):

@@ -299,3 +299,18 @@ def test_encoder_pieces_and_memory(spmm, oracle, M, K, sparsity):
     for _ in range(3):  # would take the memory over
         spmm.InitSparseMatrixA_API(A)
     assert np.array_equal(tail, want[len(want) // 2:])
+
+
+def test_tuner_writes_no_row_that_would_keep_the_planner_from_pairs(spmm):
+    """The tuner times the paired launch at 64 tokens; where it wins, its line is a remark if the planner pairs there by
+    itself (a row would be found before the planner's rule), else the row of the next plan."""
+    from graphneuralnetproj_amd import tune_plans
+
+    for only in (None, [2]):
+        assert (2, 0, 2, tune_plans.PAIRED) in tune_plans.candidate_plans(64, 16, only)
+        assert all(p[1:] != (0, 2, tune_plans.PAIRED) for p in tune_plans.candidate_plans(32, 16, only))
+    assert spmm.SpMM_PlanLaunch(512, 64, 1024, 4)["paired"] and not spmm.SpMM_PlanLaunch(28672, 64, 7168, 1)["paired"]
+    results = [(9.5, (4, 0, 2, tune_plans.PAIRED)), (12.0, (4, 1, 4, 0))]
+    assert tune_plans.best_row(512, 1024, 64, results).lstrip().startswith("//")
+    results = [(50.0, (1, 0, 2, tune_plans.PAIRED)), (55.0, (1, 0, 4, 2))]
+    assert tune_plans.best_row(28672, 7168, 64, results).lstrip().startswith("{28672, 7168, 64, 1, 0, 4, 2},")
