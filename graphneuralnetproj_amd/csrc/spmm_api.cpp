@@ -58,6 +58,12 @@ extern "C" int InitSparseMatrixA_API_NoReorder(const uint16_t* A_h, int M, int N
     return tcsl::encode_noreorder(A_h, M, K, Compressed_A, TileOffsets);
 }
 
+extern "C" int SpMM_EncodeInto(const uint16_t* A_h, int M, int K, int Reorder, void* (*Allocate)(void* User, size_t Bytes),
+                               void* User, int* TileOffsets)
+{
+    return tcsl::encode_into(A_h, M, K, Reorder != 0, Allocate, User, TileOffsets);
+}
+
 extern "C" int GenSparseMatrixBinFile(char* DenseMatrixFileName, int M, int K, char* NZWeightsFileName,
                                       char* TileOffsetsFileName, char* OutputSizesFileName)
 {

@@ -14,7 +14,7 @@
 //     two passes (count -> prefix sum -> encode) spread over a small thread pool
 //     by tile row.  The reference is single threaded.
 //
-// Plain C++: no HIP here.
+// Plain C++ and SSE2 (part of every x86-64, the only hosts this card has): no HIP here.
 #include <emmintrin.h>
 #include <sys/mman.h>
 
@@ -87,19 +87,21 @@ int count_tile(const uint16_t* tile, int ld)
 
 constexpr int kChunkTiles = 16;  // tiles of a tile row that one thread encodes at a time
 
-// Room for n words, to be given back with free().  Large rooms are aligned to huge pages and the
-// system is asked for them: the first touch of 41 MB in 4 KiB pages costs 10000 faults.
-uint32_t* alloc_words(size_t n)
+// Room for the words of a caller that takes it as it comes, to be given back with free(); *user, a void*, is
+// the room.  Large rooms are aligned to huge pages and the system is asked for them: the first touch of
+// 41 MB in 4 KiB pages costs 10000 faults.
+void* allocate_words(void* user, size_t bytes)
 {
     constexpr size_t kHuge = size_t(2) << 20;
-    const size_t bytes = n * sizeof(uint32_t);
-    if (bytes < 2 * kHuge)
-        return static_cast<uint32_t*>(std::malloc(bytes));
-    const size_t whole = (bytes + kHuge - 1) / kHuge * kHuge;
-    void* p = std::aligned_alloc(kHuge, whole);
-    if (p)
-        (void)madvise(p, whole, MADV_HUGEPAGE);  // a hint: refused, nothing is lost
-    return static_cast<uint32_t*>(p);
+    void** const room = static_cast<void**>(user);
+    if (bytes < 2 * kHuge) {
+        *room = std::malloc(bytes ? bytes : 1);
+    } else if (posix_memalign(room, kHuge, bytes) == 0) {
+        (void)madvise(*room, bytes / kHuge * kHuge, MADV_HUGEPAGE);  // a hint: refused, nothing is lost
+    } else {
+        *room = nullptr;
+    }
+    return *room;
 }
 
 struct TileScratch {
@@ -126,7 +128,7 @@ int first_zero_of(const TileScratch& ws, int b)
 // Bound by the instructions per kept element (two: into its bank's list, and out of it), so rows are
 // tested 16 elements at a time and only set bits are visited, and the emission order's groups of
 // 32 x 4 words are transposed 4 x 4 words at a time.  (7168 x 7168 at 80 % on 16 threads, the whole call
-// from Python with no copy of the words: 2.8 ms; element by element, in two sets of threads, with
+// from Python with no copy of the words: 3.1 ms; element by element, in two sets of threads, with
 // the copy: 15.1.)
 int emit_tile(const uint16_t* tile, int ld, uint32_t* dst, TileScratch& ws)
 {
@@ -224,7 +226,32 @@ int emit_tile_noreorder(const uint16_t* tile, int ld, uint32_t* dst, int pads)
     return w;
 }
 
-int encode_impl(const uint16_t* A, int M, int K, uint32_t** items_out, int** offsets_out, bool reorder);
+bool bad_shape(int M, int K)
+{
+    return M <= 0 || K <= 0 || M % kTileRows != 0 || K % kTileCols != 0;
+}
+
+int encode_impl(const uint16_t* A, int M, int K, uint32_t** items_out, int** offsets_out, bool reorder)
+{
+    if (!A || !items_out || !offsets_out)
+        return kErrNullPointer;
+    if (bad_shape(M, K))
+        return kErrBadShape;
+    const size_t entries = static_cast<size_t>(M / kTileRows) * (K / kTileCols) + kOffsetPadding;
+    int* const offs = static_cast<int*>(std::malloc(entries * sizeof(int)));
+    if (!offs)
+        return kErrNoMemory;
+    void* items = nullptr;
+    const int rc = encode_into(A, M, K, reorder, allocate_words, &items, offs);
+    if (rc < 0) {
+        std::free(items);
+        std::free(offs);
+        return rc;
+    }
+    *items_out = static_cast<uint32_t*>(items);
+    *offsets_out = offs;
+    return rc;
+}
 
 }  // namespace
 
@@ -238,29 +265,23 @@ int encode_noreorder(const uint16_t* A, int M, int K, uint32_t** items_out, int*
     return encode_impl(A, M, K, items_out, offsets_out, false);
 }
 
-namespace {
-
-int encode_impl(const uint16_t* A, int M, int K, uint32_t** items_out, int** offsets_out, bool reorder)
+int encode_into(const uint16_t* A, int M, int K, bool reorder, void* (*allocate)(void* user, size_t bytes), void* user, int* offs)
 {
-    if (!A || !items_out || !offsets_out)
+    if (!A || !allocate || !offs)
         return kErrNullPointer;
-    if (M <= 0 || K <= 0 || M % kTileRows != 0 || K % kTileCols != 0)
+    if (bad_shape(M, K))
         return kErrBadShape;
     const int tr = M / kTileRows, tc = K / kTileCols;
     const long ntiles = static_cast<long>(tr) * tc;
 
-    int* offs = static_cast<int*>(std::malloc((ntiles + kOffsetPadding) * sizeof(int)));
-    if (!offs)
-        return kErrNoMemory;
-
     // One set of threads for both passes (making threads costs about as much as counting a few tile
-    // rows): counts, a meeting at which the last one to arrive adds them up and allocates, words.
+    // rows): counts, a meeting at which the caller's thread adds them up and asks for the room, words.
     uint32_t* items = nullptr;
     int rc = 0;
     std::atomic<bool> ok{true};
     std::atomic<long> next_row{0}, next_chunk{0};
     std::mutex mu;
-    std::condition_variable met;
+    std::condition_variable all_in, met;
     const long chunks_per_row = (tc + kChunkTiles - 1) / kChunkTiles, chunks = tr * chunks_per_row;
     const int threads = pool_size(chunks);
     int started = threads, arrived = 0;
@@ -278,11 +299,11 @@ int encode_impl(const uint16_t* A, int M, int K, uint32_t** items_out, int** off
             offs[t + 1] = static_cast<int>(total_vecs);
         }
         offs[ntiles + 1] = static_cast<int>(total_vecs);  // trailing empty tile (:433-435)
-        items = alloc_words(std::max<size_t>(total_vecs * kVec, 1));
+        items = static_cast<uint32_t*>(allocate(user, static_cast<size_t>(total_vecs) * kVec * sizeof(uint32_t)));
         if (!items)
             rc = kErrNoMemory;
     };
-    auto work = [&]() {
+    auto work = [&](bool caller) {
         // pass 1: padded word count of every tile, stored in offs[t + 1]; whole rows, in memory order
         for (long i; (i = next_row.fetch_add(1)) < tr;) {
             int* const counts = offs + i * tc + 1;
@@ -297,10 +318,14 @@ int encode_impl(const uint16_t* A, int M, int K, uint32_t** items_out, int** off
         }
         {
             std::unique_lock<std::mutex> lock(mu);
-            if (++arrived == started) {
+            arrived++;
+            if (caller) {
+                all_in.wait(lock, [&] { return arrived == started; });
                 add_up();
                 met.notify_all();
             } else {
+                if (arrived == started)
+                    all_in.notify_one();
                 met.wait(lock, [&] { return ready; });
             }
             if (rc != 0)
@@ -336,33 +361,24 @@ int encode_impl(const uint16_t* A, int M, int K, uint32_t** items_out, int** off
     try {
         pool.reserve(threads - 1);
         for (int t = 1; t < threads; t++)
-            pool.emplace_back(work);
+            pool.emplace_back(work, false);
     } catch (...) {  // fewer threads than wanted: go on with those that there are
         std::lock_guard<std::mutex> lock(mu);
         started = static_cast<int>(pool.size()) + 1;
     }
-    work();
+    work(true);
     for (auto& th : pool)
         th.join();
     if (rc == 0 && !ok)
         rc = kErrNoMemory;
-    if (rc != 0) {
-        std::free(items);
-        std::free(offs);
-        return rc;
-    }
-    *items_out = items;
-    *offsets_out = offs;
-    return static_cast<int>(ntiles + kOffsetPadding);
+    return rc != 0 ? rc : static_cast<int>(ntiles + kOffsetPadding);
 }
-
-}  // namespace
 
 int encode_file(const char* dense, int M, int K, const char* nz_path, const char* off_path, const char* sizes_path)
 {
     if (!dense || !nz_path || !off_path || !sizes_path)
         return kErrNullPointer;
-    if (M <= 0 || K <= 0 || M % kTileRows != 0 || K % kTileCols != 0)
+    if (bad_shape(M, K))
         return kErrBadShape;
     const size_t bytes = static_cast<size_t>(M) * K * sizeof(uint16_t);
     std::vector<uint16_t> host(static_cast<size_t>(M) * K);

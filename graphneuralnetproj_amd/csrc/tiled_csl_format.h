@@ -29,6 +29,10 @@ inline uint32_t pack_item(uint16_t value_bits, int position)
 
 int encode(const uint16_t* A, int M, int K, uint32_t** items_out, int** offsets_out);
 int encode_noreorder(const uint16_t* A, int M, int K, uint32_t** items_out, int** offsets_out);
+// The same into room of the caller's: offsets has (M / 128) * (K / 64) + 2 ints, allocate(user, bytes) is called once,
+// on the caller's thread, when the words' size is known (nullptr: kErrNoMemory).  Nothing is freed here.
+int encode_into(const uint16_t* A, int M, int K, bool reorder, void* (*allocate)(void* user, size_t bytes), void* user,
+                int* offsets);
 int encode_file(const char* dense, int M, int K, const char* nz_path, const char* off_path, const char* sizes_path);
 
 // Deterministic synthetic inputs (counter based, identical on every host).

@@ -16,7 +16,6 @@ Reference interfaces mirrored (paths relative to the reference checkout):
 import ctypes
 import os
 import subprocess
-import weakref
 
 import numpy as np
 
@@ -27,10 +26,12 @@ _LIB_PATH = os.environ.get("SPMM_LIB_PATH") or os.path.join(_PKG, "lib", "libSpM
 _u16p = ctypes.POINTER(ctypes.c_uint16)
 _u32p = ctypes.POINTER(ctypes.c_uint32)
 _i32p = ctypes.POINTER(ctypes.c_int)
+_ALLOCATE = ctypes.CFUNCTYPE(ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t)
 
 EXPORTED_SYMBOLS = (
     "InitSparseMatrixA_API",
     "InitSparseMatrixA_API_NoReorder",
+    "SpMM_EncodeInto",
     "SpMM_SplitK_API",
     "SpMM_SplitK_API_StaticWorkspace",
     "GenSparseMatrixBinFile",
@@ -120,6 +121,8 @@ def load_library():
                                           ctypes.POINTER(_i32p)]
     lib.InitSparseMatrixA_API_NoReorder.restype = ctypes.c_int
     lib.InitSparseMatrixA_API_NoReorder.argtypes = lib.InitSparseMatrixA_API.argtypes
+    lib.SpMM_EncodeInto.restype = ctypes.c_int
+    lib.SpMM_EncodeInto.argtypes = [_u16p, ctypes.c_int, ctypes.c_int, ctypes.c_int, _ALLOCATE, ctypes.c_void_p, _i32p]
     lib.SpMM_SplitK_API.restype = ctypes.c_int
     lib.SpMM_SplitK_API.argtypes = [ctypes.c_void_p] * 6 + [ctypes.c_int] * 3 + [ctypes.c_void_p, ctypes.c_int]
     lib.SpMM_SplitK_API_StaticWorkspace.restype = ctypes.c_int
@@ -245,22 +248,25 @@ def InitSparseMatrixA_API(A_h, M=None, N=0, K=None, _entry="InitSparseMatrixA_AP
     if a.size != M * K:
         raise ValueError(f"A_h has {a.size} elements, expected {M}*{K}")
     lib = load_library()
-    items, offs = _u32p(), _i32p()
-    n = getattr(lib, _entry)(a.ctypes.data_as(_u16p), M, N, K, ctypes.byref(items), ctypes.byref(offs))
+    if M <= 0 or K <= 0 or M % 128 or K % 64:
+        raise SpMMError(_entry, -1)
+    offsets = np.empty((M // 128) * (K // 64) + 2, dtype=np.int32)
+    words = []
+
+    # The words go straight into an array that owns them (a copy out of the library's memory, 41 MB on one
+    # thread for 7168 x 7168 at 80 % sparsity, took longer than the encoding).
+    def allocate(_, size):
+        try:
+            words.append(np.empty(size // 4, dtype=np.uint32))
+        except MemoryError:
+            return None
+        return words[0].ctypes.data
+
+    n = lib.SpMM_EncodeInto(a.ctypes.data_as(_u16p), M, K, _entry == "InitSparseMatrixA_API", _ALLOCATE(allocate), None,
+                            offsets.ctypes.data_as(_i32p))
     if n < 0:
         raise SpMMError(_entry, n)
-    offsets = np.ctypeslib.as_array(offs, shape=(n,)).astype(np.int32, copy=True)
-    lib.SpMM_FreeHost(offs)
-    nwords = int(offsets[-1]) * 4
-    if not nwords:
-        lib.SpMM_FreeHost(items)
-        return np.zeros(0, dtype=np.uint32), offsets
-    # The array is the library's own memory, given back when the last view of it is gone (a copy of
-    # 7168 x 7168 at 80 % sparsity, 41 MB on one thread, took longer than the encoding).
-    address = ctypes.cast(items, ctypes.c_void_p).value
-    owner = (ctypes.c_uint32 * nwords).from_address(address)
-    weakref.finalize(owner, lib.SpMM_FreeHost, ctypes.c_void_p(address)).atexit = False
-    return np.frombuffer(owner, dtype=np.uint32), offsets
+    return words.pop(), offsets
 
 
 def _ptr(x):

@@ -62,6 +62,16 @@ SPMM_EXPORT int InitSparseMatrixA_API_NoReorder(const uint16_t* A_h, int M, int 
                                                 int** TileOffsets);
 
 /*
+ * Both encoders (Reorder != 0: InitSparseMatrixA_API, 0: InitSparseMatrixA_API_NoReorder) into memory of the caller's, for
+ * callers whose arrays own what they hold.  TileOffsets has (M/128)*(K/64) + 2 ints.  Allocate(User, Bytes) is
+ * called once, on the calling thread, when the words' size is known (Bytes may be 0), and returns room for them,
+ * 4-byte aligned, or NULL (-2).  Returns as the encoders do; on an error what Allocate gave is still the caller's.  The reference
+ * only returns memory of its own.
+ */
+SPMM_EXPORT int SpMM_EncodeInto(const uint16_t* A_h, int M, int K, int Reorder, void* (*Allocate)(void* User, size_t Bytes),
+                                void* User, int* TileOffsets);
+
+/*
  * The product C = A * B on the GPU.  Stands in for
  *   cudaError_t SpMM_SplitK_API(cudaStream_t stream, const half* A, const uint4* Compressed_A,
  *                               const int* TileOffsets, const half* B, half* C,

@@ -314,3 +314,28 @@ def test_tuner_writes_no_row_that_would_keep_the_planner_from_pairs(spmm):
     assert tune_plans.best_row(512, 1024, 64, results).lstrip().startswith("//")
     results = [(50.0, (1, 0, 2, tune_plans.PAIRED)), (55.0, (1, 0, 4, 2))]
     assert tune_plans.best_row(28672, 7168, 64, results).lstrip().startswith("{28672, 7168, 64, 1, 0, 4, 2},")
+
+
+@pytest.mark.parametrize("entry", ["InitSparseMatrixA_API", "InitSparseMatrixA_API_NoReorder"])
+def test_encoded_arrays_own_their_memory(spmm, entry):
+    """Both arrays are the caller's own, resizable in place, also the empty one of an all-zero matrix; and the C
+    function's memory is the same words, given back with free()."""
+    import ctypes
+
+    A = spmm.synth_weights(1024, 2048, 0.5, False, seed=4)  # 4 MB of words: huge pages are asked for
+    for dense in (A, np.zeros((128, 64), dtype=np.float16)):
+        items, offsets = getattr(spmm, entry)(dense)
+        assert items.flags.owndata and offsets.flags.owndata and items.base is None
+        assert items.dtype == np.uint32 and items.size == 4 * offsets[-1]
+        head = items[:8].copy()
+        items.resize(items.size + 8, refcheck=False)
+        assert np.array_equal(items[:head.size], head) and (items[-8:] == 0).all()
+    lib = spmm.load_library()
+    items, offsets = getattr(spmm, entry)(A)
+    w, o = ctypes.POINTER(ctypes.c_uint32)(), ctypes.POINTER(ctypes.c_int)()
+    bits = A.view(np.uint16)
+    n = getattr(lib, entry)(bits.ctypes.data_as(ctypes.POINTER(ctypes.c_uint16)), 1024, 0, 2048, ctypes.byref(w), ctypes.byref(o))
+    assert n == offsets.size and np.array_equal(np.ctypeslib.as_array(o, shape=(n,)), offsets)
+    assert np.array_equal(np.ctypeslib.as_array(w, shape=items.shape), items)
+    lib.SpMM_FreeHost(w)
+    lib.SpMM_FreeHost(o)
