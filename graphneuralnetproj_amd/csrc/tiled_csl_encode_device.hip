@@ -27,6 +27,10 @@ constexpr int kRowGroups = kThreads / kBanks, kRowsPerThread = kTileRows / kRowG
 constexpr int kMaxLevel = 2 * kTileRows + 4;  // 256 per bank + up to 3 pads, rounded up
 
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+// The matrix and the words may lie at any element: callers' views begin anywhere (the loads and stores are as wide all the same).
+typedef uint32_t pair_any __attribute__((aligned(2)));
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x4_word __attribute__((ext_vector_type(4), aligned(4)));
 
 // 1 in each half that holds a kept value (csrc/SpMM_API.cu:262: fabs(float(v)) > 0, i.e. not +-0 and
 // not NaN), else 0.
@@ -46,7 +50,6 @@ constexpr int kCountTiles = 8;
 __global__ __launch_bounds__(kThreads) void tcsl_count_tiles(const uint16_t* __restrict__ A, int K, int tiles_k,
                                                             int* __restrict__ offsets)
 {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     __shared__ int part[kWaves][kCountTiles];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int spans = (tiles_k + kCountTiles - 1) / kCountTiles;
@@ -55,10 +58,10 @@ __global__ __launch_bounds__(kThreads) void tcsl_count_tiles(const uint16_t* __r
     if (first + (lane >> 3) < tiles_k) {
         constexpr int kRows = kTileRows / kWaves;
         const uint16_t* src = A + ((size_t)row_tile * kTileRows + wave * kRows) * K + (size_t)first * kTileCols + lane * 8;
-        u32x4 v[kRows];
+        u32x4_any v[kRows];
 #pragma unroll
         for (int r = 0; r < kRows; r++)
-            v[r] = *reinterpret_cast<const u32x4*>(src + (size_t)r * K);
+            v[r] = *reinterpret_cast<const u32x4_any*>(src + (size_t)r * K);
         u16x2 c = {0, 0};
 #pragma unroll
         for (int r = 0; r < kRows; r++)
@@ -128,7 +131,6 @@ __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* _
                                                               const int* __restrict__ offsets, uint32_t* __restrict__ items)
 {
     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     __shared__ uint32_t seq[kSeqWords + 64];   // pops first .. first + kSeqWords - 1; then where words of other passes go
     __shared__ u32x2 levels[kMaxLevel + 1];    // level l: banks at least l tall, pops made before the level starts
     __shared__ int grp_count[kRowGroups][kBanks];
@@ -149,7 +151,7 @@ __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* _
 #pragma unroll
     for (int i = 0; i < kRowsPerThread; i++) {
         const int x = b ^ ((i & 7) << 2);
-        pairs[i] = *reinterpret_cast<const uint32_t*>(own_rows + (size_t)i * K + 2 * x);
+        pairs[i] = *reinterpret_cast<const pair_any*>(own_rows + (size_t)i * K + 2 * x);
     }
     uint32_t kept = 0;  // bit i + 16 h: element h of row i
 #pragma unroll
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* _
     //    pop' % 32, arrival kk = pop' / 32 written at reverse position 4 R - 1 - kk).
     const uint32_t below = (1u << b) - 1u;
     const int vecs = words / 4, R = vecs / 32, rem = vecs % 32;
-    u32x4* const out = reinterpret_cast<u32x4*>(items) + offsets[t];
+    u32x4_word* const out = reinterpret_cast<u32x4_word*>(items) + offsets[t];
     const int dump = kSeqWords + lane;
     // The words of pops first .. last - 1 into the sequence.  Level entries are read sixteen at a time,
     // ahead of the writes that depend on them: one by one, every element pays a trip to LDS.
@@ -245,7 +247,7 @@ __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* _
     auto write_groups = [&](int from, int done, int groups) __attribute__((always_inline)) {
         for (int i = threadIdx.x; i < groups * 32; i += kThreads) {
             const int g = i >> 5, at = from + g * 128 + (i & 31);  // pops 128 g + 32 (3 - s) + lane
-            u32x4 v;
+            u32x4_word v;
 #pragma unroll
             for (int s = 0; s < 4; s++)
                 v[s] = seq[at + (3 - s) * 32];
@@ -254,7 +256,7 @@ __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* _
     };
     auto write_tail = [&]() __attribute__((always_inline)) {
         if ((int)threadIdx.x < rem) {
-            u32x4 v;
+            u32x4_word v;
 #pragma unroll
             for (int s = 0; s < 4; s++)
                 v[s] = seq[(3 - s) * rem + threadIdx.x];

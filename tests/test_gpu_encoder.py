@@ -168,3 +168,20 @@ def test_device_encoder_rejects_bad_shapes(spmm):
     assert lib.SpMM_DeviceEncodeOffsets(None, z.data_ptr(), 128, 60, z.data_ptr()) != 0
     assert lib.SpMM_DeviceEncodeOffsets(None, None, 128, 64, z.data_ptr()) != 0
     assert lib.SpMM_DeviceEncodeItems(None, z.data_ptr(), 128, 64, None, z.data_ptr()) != 0
+
+
+@pytest.mark.parametrize("at", [1, 2, 5])
+def test_device_encoder_of_a_matrix_at_any_element(spmm, oracle, at):
+    """A contiguous view that begins at any element of a larger buffer: the wide loads ask for no alignment."""
+    torch = _torch()
+    M, K = 256, 64 * 9
+    A = spmm.synth_weights(M, K, 0.7, False, seed=at)
+    flat = torch.zeros(M * K + 16, dtype=torch.float16, device="cuda:0")
+    view = flat[at:at + M * K].view(M, K)
+    view.copy_(torch.from_numpy(A.view(np.int16).copy()).cuda().view(torch.float16))
+    print(f"[gpu case] device encode at element {at}", flush=True)
+    d_items, d_offsets = spmm.encode_on_device(view)
+    torch.cuda.synchronize()
+    items, offsets = oracle.encode(A)
+    assert np.array_equal(d_offsets.cpu().numpy(), offsets)
+    assert np.array_equal(d_items.cpu().numpy().view(np.uint32), items)
