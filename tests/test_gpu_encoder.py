@@ -102,11 +102,18 @@ def test_device_encoder_matches_oracle(spmm, oracle, M, K, sparsity, skew):
     _compare(spmm, oracle, spmm.synth_weights(M, K, sparsity, skew, seed=M + K))
 
 
-@pytest.mark.parametrize("M,K,sparsity", [(128, 64, 0.516), (256, 64 * 9, 0.515), (128, 64 * 8, 0.03), (256, 64 * 17, 0.27)])
-def test_device_encoder_edges(spmm, oracle, M, K, sparsity):
+@pytest.mark.parametrize("M,K,sparsity,passes", [(128, 64, 0.516, {1, 2}), (256, 64 * 9, 0.515, {1, 2}), (128, 64 * 8, 0.03, {2}),
+                                                 (256, 64 * 17, 0.27, {2}), (256, 64 * 9, 0.01, {3})])
+def test_device_encoder_edges(spmm, oracle, M, K, sparsity, passes):
     """Tiles around the 3968 words that the GPU encoder emits in one pass (48.4 % dense) and beyond, in two
-    and in three; spans of eight tiles, whole and with a rest of one; pads of every number."""
-    _compare(spmm, oracle, spmm.synth_weights(M, K, sparsity, False, seed=M + K))
+    (31 groups of 128 words each, and a tail) and in three; spans of eight tiles, whole and with a rest of one; pads
+    of every number."""
+    A = spmm.synth_weights(M, K, sparsity, False, seed=M + K)
+    words = -(-(A != 0).reshape(M // 128, 128, K // 64, 64).sum((1, 3)).ravel() // 4) * 4
+    assert {1 if w <= 3968 else -(-(int(w) // 128) // 31) for w in words} <= passes
+    if passes == {3}:
+        assert (words % 128 > 0).all()
+    _compare(spmm, oracle, A)
 
 
 def test_device_encoder_special_tiles(spmm, oracle):
@@ -185,3 +192,29 @@ def test_device_encoder_of_a_matrix_at_any_element(spmm, oracle, at):
     items, offsets = oracle.encode(A)
     assert np.array_equal(d_offsets.cpu().numpy(), offsets)
     assert np.array_equal(d_items.cpu().numpy().view(np.uint32), items)
+
+
+def test_device_encoder_with_offsets_of_another_matrix(spmm):
+    """The second step of the encoding, given offsets of a matrix that has fewer words in some tiles and more in others:
+    tiles whose counts agree get their words, the room of all others and what lies behind stay as they were."""
+    import ctypes
+
+    torch = _torch()
+    M, K = 512, 64 * 11
+    dev = torch.device("cuda:0")
+    A = torch.from_numpy(spmm.synth_weights(M, K, 0.8, False, seed=8).view(np.int16).copy()).to(dev).view(torch.float16)
+    items, offsets = spmm.encode_on_device(A)
+    kind = (torch.arange(M // 128 * (K // 64), device=dev) % 4).view(M // 128, K // 64)  # 0: emptied, 1: dense, else its own
+    spread = kind.repeat_interleave(128, 0).repeat_interleave(64, 1)
+    other = torch.where(spread == 0, torch.zeros_like(A), torch.where(spread == 1, torch.ones_like(A), A)).contiguous()
+    mark, total = 0x5A5A5A5A, items.numel()
+    out = torch.full((total + 16384,), mark, dtype=torch.int32, device=dev)
+    print("[gpu case] device encode with foreign offsets", flush=True)
+    rc = spmm.load_library().SpMM_DeviceEncodeItems(
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream or None), ctypes.c_void_p(other.data_ptr()), M, K,
+        ctypes.c_void_p(offsets.data_ptr()), ctypes.c_void_p(out.data_ptr()))
+    assert rc == 0
+    torch.cuda.synchronize()
+    keep = np.repeat((kind.view(-1) > 1).cpu().numpy(), 4 * np.diff(offsets.cpu().numpy()[:-1]))
+    want, got = items.cpu().numpy(), out.cpu().numpy()
+    assert np.array_equal(got[:total], np.where(keep, want, mark)) and (got[total:] == mark).all()

@@ -859,14 +859,29 @@ def test_fused_row_skewed_weight_full_size(spmm, oracle):
     assert np.isfinite(C).all() and (diff <= 2e-2 + 2e-2 * np.abs(two.astype(np.float32))).all()
 
 
-@pytest.mark.parametrize("M,K,sparsity", [(8320, 4096, 0.6), (128, 384, 0.55), (1024, 896, 0.25), (256, 512, 0.85)])
+@pytest.mark.parametrize("M,K,sparsity", [(8320, 4096, 0.6), (128, 384, 0.55), (1024, 896, 0.25), (256, 512, 0.85),
+                                          (5760, 6016, 0.6), (5760, 6016, 0.25), (5760, 6016, "mixed")])
 def test_device_residual_lists_edges(spmm, oracle, M, K, sparsity):
     """Residual lists where the GPU's packer changes its way: more lists than one step of the scan takes
-    (16640), units that leave a rest of four and workgroups with a rest of 32 lists, lists beyond four
-    rounds of 64 words and more words than are dealt in one pass, lists of one round beside empty ones."""
+    (16640), units that leave a rest of four, lists beyond four rounds of 64 words and more words than are dealt
+    in one pass, lists of one round beside empty ones; and with 32 lists to a workgroup (from 16384 lists on)
+    a last workgroup with a rest of 24 of them, lists of one pass, of several, and of all lengths side by side."""
     torch = _torch()
-    A = spmm.synth_weights(M, K, sparsity, False, seed=M + K)
+    if sparsity == "mixed":  # 16-row blocks of every density, in no order: empty lists to ones of 1024 words
+        A = spmm.synth_weights(M, K, 0.0, False, seed=M + K)
+        rng = np.random.default_rng(3)
+        density = rng.permutation(np.linspace(0.0, 1.0, M // 16 * (K // 128))).reshape(M // 16, K // 128)
+        A[rng.random((M, K), dtype=np.float32) >= density.repeat(16, 0).repeat(128, 1).astype(np.float32)] = 0
+    else:
+        A = spmm.synth_weights(M, K, sparsity, False, seed=M + K)
     _, A2 = oracle.decompose(A)
+    lists = np.count_nonzero(A2.reshape(M // 16, 16, K // 128, 128), axis=(1, 3))
+    if M == 5760:  # what this case is there for
+        assert lists.size >= 16384 and lists.size % 32 == 24
+        by_group = lists.reshape(M // 128, 8, K // 128).transpose(0, 2, 1).ravel()[:lists.size // 32 * 32].reshape(-1, 32)
+        room = np.where(by_group > 256, 2 * by_group, np.where(by_group > 64, by_group, 0)).sum(1)  # bytes; 8192 a pass
+        assert {0.6: room.max() <= 8192, 0.25: room.min() > 2 * 8192,
+                "mixed": lists.min() == 0 and lists.max() > 1000 and room.max() > 8192}[sparsity]
     want_words, want_offs, want_longest = spmm.HeteroSparse_PackA2(A2)
     d_A2 = torch.from_numpy(A2.view(np.int16).copy()).to("cuda:0").view(torch.float16)
     print(f"[gpu case] device residual lists M={M} K={K} sparsity={sparsity}", flush=True)

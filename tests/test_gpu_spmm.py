@@ -1013,7 +1013,7 @@ def test_shared_activation_tiles_rejects_other_shapes(spmm):
     (256, 64 * 2, 2, 0.8, 1),      # two batches of one tile, clamped by the reduction
     (384, 64 * 6, 1, 0.5, 1),      # denser than one segment of a wave's half, clamped by the kernel
     (512, 64 * 11, 4, 0.8, 0),     # batches of 3, 3, 3, 2
-    (512, 64 * 12, 2, 0.0, 0),     # dense: five segments of ten vectors a lane and more
+    (512, 64 * 12, 2, 0.0, 0),     # dense: four segments of four vectors a lane in each half
     (640, 64 * 5, 1, 0.97, 0),     # tiles of a few vectors: the second wave's half is empty
     (1024, 64 * 6, 1, 0.999, 0),   # empty tiles
     (128 * 65, 64 * 27, 5, 0.9, 1),   # two units on some compute units, batches of 6, 6, 6, 6, 3
