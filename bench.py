@@ -335,6 +335,25 @@ def sweep(G, lib, torch, dev, sptr, with_stack):
     return out
 
 
+SWEEP_COLUMNS = ("case", "M", "K", "N", "sparsity", "row_skewed", "split_k", "split_k_from", "plan", "reduction", "ms", "frac",
+                 "kernel_ms", "kernel_frac", "tflops")
+
+
+def short_sweep(entries):
+    """The sweep as the result line holds it: the products as one table of SWEEP_COLUMNS, five digits a figure, the other cases
+    under their names.  (One object a product, every figure in full, made a line of 36 KB, too long for readers that
+    keep 32 KB of it; stderr has that form.)"""
+    def short(x):
+        if isinstance(x, float):
+            return float(f"{x:.5g}")
+        if isinstance(x, dict):
+            return {k: short(v) for k, v in x.items()}
+        return x
+
+    table = [[short(e[c]) for c in SWEEP_COLUMNS] for e in entries if "split_k_from" in e]
+    return {"columns": list(SWEEP_COLUMNS), "rows": table, "others": [short(e) for e in entries if "split_k_from" not in e]}
+
+
 def split_case(G, lib, torch, dev, sptr, workload, N, sparsity, skew=False):
     """The fork's split of a weight into a 2:4 part and a residual, at a sparsity where it can pay:
     plain Tiled-CSL, the two-kernel call and the one-launch call on the same weight, whole calls
@@ -791,7 +810,9 @@ def main():
     if not args.no_sweep:
         del d_items, d_offs, p_items, p_offs
         torch.cuda.empty_cache()
-        out["sweep"] = sweep(G, lib, torch, dev, sptr, with_stack=not args.no_stack)
+        entries = sweep(G, lib, torch, dev, sptr, with_stack=not args.no_stack)
+        print("# sweep in full: " + json.dumps(entries), file=sys.stderr)
+        out["sweep"] = short_sweep(entries)
     print(json.dumps(out))
 
 

@@ -64,3 +64,23 @@ def test_traffic_figures_name_existing_profiles():
     for (workload, n, split_k, sparsity), (nbytes, profile) in B.MEASURED_TRAFFIC_BYTES.items():
         assert workload in B.WORKLOADS and nbytes > 0
         assert os.path.exists(os.path.join(ROOT, profile)), profile
+
+
+def test_result_line_stays_short():
+    """The whole sweep fits a result line of 16 KB: readers of the line keep a bounded piece of it."""
+    import json
+
+    B = _bench()
+    entries = []
+    for label, workload, N, sparsity, skew, forced in B.sweep_cases():
+        M, K = B.WORKLOADS[workload][:2]
+        entries.append({"case": label, "M": M, "K": K, "N": N, "sparsity": sparsity, "row_skewed": skew, "split_k": 16,
+                        "split_k_from": "sweep" if forced else "planner", "layout": "B[N][K], C[N][M]", "plan": "mode 0, 2 waves, in pairs",
+                        "compressed_bytes": 10 ** 9 - 1, "reduction": "in launch", "ms": 1 / 3, "frac": 2 / 3, "kernel_ms": 1 / 7,
+                        "kernel_frac": None, "traffic": None, "traffic_profile": None, "tflops": 1000 / 3})
+    entries += [{"case": f"decoder_stack_{i}", "ms": 1 / 3, "split_k": {"records": 3}, "form": "x" * 400} for i in range(6)]
+    short = B.short_sweep(entries)
+    assert len(json.dumps(short)) < 16 * 1024
+    assert len(short["rows"]) == len(B.sweep_cases()) and len(short["others"]) == 6
+    row = dict(zip(short["columns"], short["rows"][0]))
+    assert row["case"] == entries[0]["case"] and row["ms"] == 0.33333 and row["kernel_frac"] is None
