@@ -262,7 +262,7 @@ LaunchPlan plan_launch(int M, int N, int K, int split_k, bool row_major, double*
     if (cost_us)
         *cost_us = best_cost;
     // 64 tokens: two waves to a work unit where a compute unit has one unit of up to six tiles, or two
-    // of three to 27.  Measured on 612 calls there, 128 x 64 to 47104 x 1728 and Split_K 1 to 32 at 60 to 95 % sparsity,
+    // of three to 27.  Measured on 612 calls there (up to 64256 rows and 55296 columns, Split_K 1 to 32, 60 to 95 % sparsity)
     // against the shape that the model picks: 1.006 to 1.54 times as fast (mean 1.24) with one unit, 1.004 to 1.41
     // (1.12) with two.  Slower from seven to eleven tiles on with one unit (0.97, then 0.92 to 0.55), with two
     // units of one or two tiles (0.92 to 1.1: 47104 x 64 6.5 us, 7.1 in pairs), and with more than two units

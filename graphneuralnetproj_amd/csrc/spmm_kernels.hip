@@ -881,8 +881,8 @@ __global__ __launch_bounds__(MAXW* kWave) void tcsl_spmm_kernel(const int* __res
 // for one wave per SIMD.  Half the tokens halve a wave's accumulators, MFMAs, activation fragments and
 // scatter; a pair takes 1780 cycles for a tile where it has a compute unit to itself, and three pairs fit
 // one.  The image is read twice for it (256 of about 500 LDS cycles per tile), so this wins where there is
-// little work per compute unit and the chain is what counts (512 x 704 12.2 -> 9.6 us, 1024 x 2240 12.2 -> 10.2,
-// 3072 x 2368 14.5 -> 12.1, 47232 x 1024 33.6 -> 27.9) and loses where the chip is full (28672 x 7168 49, in pairs 55
+// little work per compute unit and the chain is what counts (whole calls at 80 % with the suggested Split_K, sum included:
+// 512 x 704 12.2 -> 9.2 us, 1024 x 2240 12.6 -> 9.9, 3072 x 2368 14.2 -> 11.2, 47232 x 1024 23.6 -> 20.6) and loses where the chip is full (28672 x 7168 49, in pairs 55
 // at best).  The planner's rule: launch_plan.cpp.  (49152 x 12288 in two batches gained as well,
 // 125 -> 119, and lies outside that rule.)
 // (32 tokens, 16 for each wave, lost 2 % in the mean over the same sizes and up to 23 %.)
