@@ -12,7 +12,7 @@ spill of a register with a load in flight would save garbage).
 
 State: the queue of vector-memory operations that may still be outstanding,
 youngest last; each entry is the set of VGPRs the operation writes (empty for
-stores).  ``s_waitcnt vmcnt(N)`` keeps the N youngest entries (loads complete in
+stores, and for loads that go to LDS).  ``s_waitcnt vmcnt(N)`` keeps the N youngest entries (loads complete in
 order).  Where paths merge, queues are aligned at the youngest end and entries
 are united position by position, which over-approximates every path.  Any
 instruction that reads or writes a VGPR held in some queue entry is reported,
@@ -126,14 +126,14 @@ def transfer(queue, ins, report):
             continue
         regs = vregs(args)
         pending = set().union(*q) if q else set()
-        if VM_LOAD.match(op):
+        if VM_LOAD.match(op) and "_lds_" not in op:  # (a load to LDS writes no register, it counts like a store)
             dest = vregs(args.split(",")[0])
             srcs = regs - dest if not (dest & vregs(",".join(args.split(",")[1:]))) else vregs(",".join(args.split(",")[1:]))
             bad = srcs & pending
             if bad and report is not None:
                 report.append((lineno, op, args, sorted(bad)))
             q.append(frozenset(dest))
-        elif VM_STORE.match(op):
+        elif VM_LOAD.match(op) or VM_STORE.match(op):
             bad = regs & pending
             if bad and report is not None:
                 report.append((lineno, op, args, sorted(bad)))

@@ -530,6 +530,19 @@ int a24_waves_for(int M, int split_k)
     return (M % 256 == 0 && static_cast<long>(M / 256) * split_k > 160) ? 8 : 4;
 }
 
+// ... and for a call: B, the residual's rounds.  Where the activations go straight into LDS (aligned: a24_kernels.hip),
+// eight waves are better by 1 to 3 % as long as their workgroups run all at once, and four, two workgroups to a
+// compute unit, beyond (27648 x 9216 at 60 %, 64 tokens: two batches 74.2 us with eight, 75.6 with four; three batches
+// 97.9 and 82.6; seven 95.7 and 93.3) and for the longest lists at 64 tokens (50 %, two batches: 93.3 and 90.6).
+// Where they come through registers, four waves for the longest lists at 64 tokens: what fits.
+int a24_waves(const void* B, int M, int N, int split_k, int rounds, bool row_major)
+{
+    const int waves = a24_waves_for(M, split_k);
+    if ((reinterpret_cast<uintptr_t>(B) & 15) != 0)
+        return N == 64 && rounds >= (row_major ? 4 : 5) ? 4 : waves;
+    return static_cast<long>(M / 256) * split_k > 256 || (N == 64 && rounds >= 5) ? 4 : waves;
+}
+
 A24Plan a24_default_plan(int M, int N, int K)
 {
     // From sweeps over the OPT-30B and OPT-66B shapes (N = 16 and 64, with and without the residual):
@@ -612,7 +625,7 @@ extern "C" int HeteroSparse_A1_Partials(void* stream, const void* Packed_A1, con
     if (RowBlocks == 0 || Waves == 0) {
         const A24Plan d = a24_default_plan(M > 0 ? M : 128, N, K > 0 ? K : 128);
         p.row_blocks = d.row_blocks;
-        p.waves = a24_waves_for(M > 0 ? M : 128, Split_K);
+        p.waves = a24_waves(B, M > 0 ? M : 128, N, Split_K, 0, false);
         p.share_b = d.share_b;
     }
     if (!Packed_A1 || !B || !Partials || !a24_shape_ok(M, N, K, p.split_k, p.row_blocks, p.waves, p.share_b)) {
@@ -660,7 +673,7 @@ int hybrid_call(const char* who, void* stream, const void* Packed_A1, const void
     }
     A24Plan d = a24_shape_ok(M, N, K, Split_K_A1, 1, 1) ? a24_default_plan(M, N, K) : A24Plan{1, 1, 1};
     if (d.share_b)
-        d.waves = a24_waves_for(M, Split_K_A1);
+        d.waves = a24_waves(B, M, N, Split_K_A1, 0, row_major);
     if (!Packed_A1 || !B || !C || (residual && !TileOffsets_A2) || !a24_shape_ok(M, N, K, Split_K_A1, d.row_blocks, d.waves, d.share_b)
         || (residual && (Split_K_A2 < 1 || Split_K_A2 > 65535)) || ((residual || Split_K_A1 > 1) && !Reduction_Workspace)
         || (Flags & ~HETERO_FLAG_TWO_STREAMS)) {
@@ -795,8 +808,7 @@ int fused_call(const char* who, void* stream, const void* Packed_A1, const void*
     // is fetched where it is needed (a24_kernels.hip)
     const int rounds = (LongestList + 63) / 64;
     const int loads = rounds < HETERO_FUSED_PIPELINED_ROUNDS ? rounds : HETERO_FUSED_PIPELINED_ROUNDS;
-    // (four waves for the longest lists at 64 tokens: what fits the registers)
-    const int waves = (N == 64 && loads >= (row_major ? 4 : 5)) ? 4 : a24_waves_for(M > 0 ? M : 128, Split_K);
+    const int waves = a24_waves(B, M > 0 ? M : 128, N, Split_K, loads, row_major);
     if (!Packed_A1 || !A2_Words || !A2_Offsets || !B || !C || LongestList < 0 || LongestList > HETERO_FUSED_MAX_LIST
         || !a24_shape_ok(M, N, K, Split_K, 2, waves, 1) || (Split_K > 1 && !Reduction_Workspace) || ldb < K || ldc < M
         || ldb % 8 != 0 || ldc % 8 != 0 || (Flags & ~(SPMM_FLAG_RELU | SPMM_FLAG_SEPARATE_REDUCTION))) {

@@ -135,6 +135,24 @@ def test_stores_occupy_queue_slots():
     assert rep == []
 
 
+def test_loads_to_lds_count_and_write_no_register():
+    """A load straight into LDS takes a place in the queue; its address register is free once it is issued."""
+    ahead = """
+	buffer_load_dwordx4 v[4:7], v1, s[0:3], 0 offen
+	global_load_lds_dwordx4 v[2:3], off
+	v_add_u32 v2, v2, v2
+	s_waitcnt vmcnt({})
+	v_mov_b32 v9, v4
+"""
+    assert violations(ahead.format(1)) == []
+    assert len(violations(ahead.format(2))) == 1
+    rep = violations("""
+	global_load_dwordx2 v[2:3], v1, s[0:1]
+	global_load_lds_dwordx4 v[2:3], off
+""")
+    assert len(rep) == 1 and rep[0][3] == [2, 3]
+
+
 def test_command_line_flags_scratch_and_violations(tmp_path):
     good = tmp_path / "good.s"
     good.write_text(kernel("\tbuffer_load_dwordx4 v[4:7], v1, s[0:3], 0 offen\n\ts_waitcnt vmcnt(0)\n\tv_mov_b32 v9, v4\n"))
@@ -172,3 +190,13 @@ def test_built_sparse_mfma_kernels_pass():
     # column-major: 2 + 5 + 5 launch shapes for 64, 32 and up to 16 tokens, and 9 + 10 + 10 that take the residual along;
     # row-major (two row blocks per wave only): 2 + 2 + 2 and 8 + 10 + 10
     assert r.stdout.count("ok ") == 41 + 34
+
+
+def test_built_sparse_mfma_kernels_without_registers_for_the_tile_pass():
+    """Four waves at any number of tokens, eight above 16; lists of none to five rounds; both layouts."""
+    asm = os.path.join(HERE, "..", "graphneuralnetproj_amd", "csrc", "obj", "a24_kernels.gfx950.s")
+    if not os.path.exists(asm):
+        pytest.skip("library not built in this tree")
+    r = subprocess.run([sys.executable, CHECKER, asm, "a24_spmm_straight_b_kernel"], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
+    assert r.stdout.count("ok ") == (3 + 2) * 6 * 2

@@ -950,3 +950,57 @@ def test_device_residual_lists_with_offsets_of_another_matrix(spmm, M, K):
     keep = np.repeat(same, np.diff(o))
     assert np.array_equal(got[:total], np.where(keep, want[:total], mark))
     assert (got[total:total + 64] == 0).all() and (got[total + 64:] == mark).all()
+
+
+@pytest.mark.parametrize("N", [8, 16, 32, 64])
+@pytest.mark.parametrize("M,K,split_k,sparsity", [
+    (128, 128, 1, 0.5), (128, 256, 1, 0.95), (256, 384, 1, 0.3), (384, 512, 1, 0.6),  # one to four units: the pipeline's ends
+    (256, 640, 2, 0.7), (128, 1792, 3, 0.55),                                         # batches of unequal length
+    (5632, 1024, 8, 0.5), (10752, 512, 4, 0.45), (10752, 896, 7, 0.8),                # eight waves; four where eight do not run at once
+])
+def test_activations_straight_into_lds(spmm, oracle, N, M, K, split_k, sparsity):
+    """The tile that goes straight into LDS (aligned activations) and the one that comes through registers (a view
+    that begins at an odd element) give the same bits, in both layouts, with strides, with and without the residual;
+    the product is right to the rounding of its slabs and of itself: fp16 has 11 bits, and the inputs are exact."""
+    torch = _torch()
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(M + K + N)
+    W = torch.randn((M, K), generator=gen, device="cuda:0") * 0.02
+    W = (W * (torch.rand((M, K), generator=gen, device="cuda:0") >= sparsity)).half()
+    packed, residual = spmm.split_pack_on_device(W)
+    words, offsets, longest = spmm.pack_residual_on_device(residual)
+    ldb = K + 72
+    B = torch.randn((N, ldb), generator=gen, device="cuda:0").half()
+    odd = torch.empty(N * ldb + 8, dtype=torch.float16, device="cuda:0")[1:1 + N * ldb].view(N, ldb)
+    odd.copy_(B)
+    Bt = B[:, :K].t().contiguous()
+    odd_t = torch.empty(N * K + 8, dtype=torch.float16, device="cuda:0")[1:1 + N * K].view(K, N)
+    odd_t.copy_(Bt)
+    stream = torch.cuda.current_stream()
+    ws = torch.empty((split_k, N, M), dtype=torch.float16, device="cuda:0")
+    print(f"[gpu case] straight into LDS M={M} K={K} N={N} split_k={split_k} longest={longest}", flush=True)
+
+    def strided(b):
+        C = torch.full((N, M + 8), float("nan"), dtype=torch.float16, device="cuda:0")
+        spmm.HeteroSparse_Fused_SpMM_API_Strided(stream, packed, words, offsets, longest, b, ldb, C, M + 8, M, N, K, ws, split_k, 0)
+        return C[:, :M].contiguous()
+
+    def row_major(b):
+        C = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda:0")
+        spmm.HeteroSparse_Fused_SpMM_API_RowMajor(stream, packed, words, offsets, longest, b, C, M, N, K, ws, split_k, 0)
+        return C.t().contiguous()
+
+    def alone(b):  # the 2:4 part, row-major
+        C = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda:0")
+        spmm.HeteroSparse_SpMM_API_RowMajor(stream, packed, None, None, b, C, M, N, K, ws, split_k, 0, 0)
+        return C.t().contiguous()
+
+    got = strided(B)
+    for other in (strided(odd), row_major(Bt), row_major(odd_t)):
+        assert torch.equal(got.view(torch.int16), other.view(torch.int16))
+    assert torch.equal(alone(Bt).view(torch.int16), alone(odd_t).view(torch.int16))
+    ref = B[:, :K].double().cpu() @ W.double().cpu().t()
+    size = B[:, :K].double().cpu().abs() @ W.double().cpu().abs().t()  # bounds every partial sum
+    # one rounding of each slab and of the sum, 2^-11 of what a slab or the sum can be, and fp32 sums (K additions of 2^-24)
+    bound = size * (2 * 2.0 ** -11 + K * 2.0 ** -24) + 2.0 ** -24
+    assert ((got.double().cpu() - ref).abs() <= bound).all()
