@@ -11,75 +11,139 @@ constexpr int kGroupBlocks = 8;  // records of eight row blocks are stored toget
 }  // namespace
 
 // Split and pack on the GPU: the same bits as the host's decompose + pack (a24_pack.cpp), for
-// weights that are already in device memory.  One thread per lane of a record: it reads its row's
-// 4 x 8 columns of the unit, keeps the first two kept values of every group of four
-// (kernel_benchmark/spmm_decompose.h:12-51) in the record and writes the others to the dense
-// residual (when asked for one), zero elsewhere.
-__global__ __launch_bounds__(256) void a24_split_pack_kernel(const uint16_t* __restrict__ A, uint8_t* __restrict__ packed,
-                                                             uint16_t* __restrict__ residual, int K, int units,
-                                                             long records)
+// weights that are already in device memory: the first two kept values of every group of four
+// (kernel_benchmark/spmm_decompose.h:12-51) go to the record, the others to the dense residual (when
+// asked for one), zero elsewhere.
+//
+// Bound by HBM.  A workgroup takes 16 rows of four consecutive units, a wave four of the rows: every
+// load, and every store to the residual, is one contiguous KiB, and the four records leave through LDS in
+// whole lines.  What becomes of a group of four is a function of which of its elements are kept,
+// looked up in a table of sixteen entries.  (A thread per lane of a record, which reads its own four
+// granules, half a line to sixteen rows per load, and works the positions out by comparing: 217 us on a
+// 21504 x 7168 weight, half of them vector instructions; now 114.  1024 x 1024: 5.5 us, now 3.3.)
+namespace {
+
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+typedef u32x4 u32x4_any __attribute__((aligned(2)));   // the matrices' granules may lie at any element,
+typedef u32x4 u32x4_byte __attribute__((aligned(1)));  // the records at any byte
+typedef unsigned u32_byte __attribute__((aligned(1)));
+
+constexpr int kSplitUnits = 4;  // units per workgroup
+// A record in LDS: its eight 256-byte blocks of values (block = step / 2 * 4 + column group) 272 bytes apart, then the
+// positions; records 2432 apart.  The 64 eight-byte writes of a row (a unit's 16 granules, four units) fall
+// two to a bank, which is as few as there can be.
+constexpr int kBlockStride = 272, kRecordStride = 8 * kBlockStride + 256;
+
+struct SplitEntry {
+    unsigned values;     // v_perm selector: the record's two values of the group (0xc: a zero byte)
+    unsigned rest;       // ... and the residual's elements 2 and 3 (elements 0 and 1 are among the first two)
+    unsigned positions;  // 2 bits each
+    unsigned unused;
+};
+// Entry for the kept elements `mask` of a group; a group with fewer than two is filled at free positions.
+constexpr SplitEntry split_entry(unsigned mask)
 {
-    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long record = id >> 6;
-    if (record >= records)
-        return;
-    const int L = static_cast<int>(id & 63);
-    // records are numbered ((rb / 8) * units + u) * 8 + rb % 8
-    const long group = record / (static_cast<long>(units) * kGroupBlocks);
-    const int within = static_cast<int>(record - group * units * kGroupBlocks);
-    const int u = within / kGroupBlocks;
-    const long rb = group * kGroupBlocks + within % kGroupBlocks;
-    const size_t row = (size_t)(rb * 16 + (L & 15)) * K + (size_t)u * 128 + (L >> 4) * 8;
-    uint8_t* rec = packed + (size_t)record * kRecordBytes;
-    typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
-    unsigned word = 0;
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-        const u16x8 in = *reinterpret_cast<const u16x8*>(A + row + s * 32);
-        u16x8 rest = {0, 0, 0, 0, 0, 0, 0, 0};
-        unsigned short val[4];
-#pragma unroll
-        for (int half = 0; half < 2; half++) {
-            int pos[2] = {0, 1}, n = 0;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const unsigned short v = in[half * 4 + e];
-                if ((v & 0x7fffu) != 0) {  // compares unequal to zero as a float: NaN counts, -0 does not
-                    if (n < 2)
-                        pos[n] = e;
-                    else
-                        rest[half * 4 + e] = v;
-                    n++;
-                }
-            }
-            unsigned short v0 = 0, v1 = 0;
-            if (n >= 2) {
-                v0 = in[half * 4 + pos[0]];
-                v1 = in[half * 4 + pos[1]];
-            } else if (n == 1) {
-                if (pos[0] == 3) {  // the free slot goes before it
-                    v1 = in[half * 4 + 3];
-                    pos[0] = 2;
-                    pos[1] = 3;
-                } else {
-                    v0 = in[half * 4 + pos[0]];
-                    pos[1] = 3;
-                }
-            } else {
-                pos[0] = 0;
-                pos[1] = 1;
-            }
-            val[half * 2] = v0;
-            val[half * 2 + 1] = v1;
-            word |= static_cast<unsigned>(pos[0]) << (8 * s + 4 * half) | static_cast<unsigned>(pos[1]) << (8 * s + 4 * half + 2);
+    unsigned pos[2] = {0, 1}, rest = 0x0c0c0c0cu;
+    int n = 0;
+    for (unsigned e = 0; e < 4; e++)
+        if (mask >> e & 1) {
+            if (n < 2)
+                pos[n] = e;
+            else
+                rest = e == 2 ? (rest & 0xffff0000u) | 0x0504u : (rest & 0xffffu) | 0x07060000u;
+            n++;
         }
-        typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
-        const u16x4 out = {val[0], val[1], val[2], val[3]};
-        *reinterpret_cast<u16x4*>(rec + (s >> 1) * 1024 + L * 16 + (s & 1) * 8) = out;
-        if (residual)
-            *reinterpret_cast<u16x8*>(residual + row + s * 32) = rest;
+    bool have0 = n >= 1, have1 = n >= 2;
+    if (n == 1 && pos[0] == 3) {  // the free slot goes before it
+        have0 = false;
+        have1 = true;
+        pos[0] = 2;
+        pos[1] = 3;
+    } else if (n == 1) {
+        pos[1] = 3;
     }
-    *reinterpret_cast<unsigned*>(rec + 2048 + L * 4) = word;
+    const unsigned v0 = have0 ? 0x0100u + 0x0202u * pos[0] : 0x0c0cu, v1 = have1 ? 0x0100u + 0x0202u * pos[1] : 0x0c0cu;
+    return SplitEntry{v0 | v1 << 16, rest, pos[0] | pos[1] << 2, 0u};
+}
+struct SplitTable {
+    SplitEntry e[16];
+};
+constexpr SplitTable make_split_table()
+{
+    SplitTable t{};
+    for (unsigned m = 0; m < 16; m++)
+        t.e[m] = split_entry(m);
+    return t;
+}
+__constant__ const SplitTable split_table = make_split_table();
+
+}  // namespace
+
+template<bool RESIDUAL>
+__global__ __launch_bounds__(256) void a24_split_pack_kernel(const uint16_t* __restrict__ A, uint8_t* __restrict__ packed,
+                                                             uint16_t* __restrict__ residual, int K, int units)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t records[kSplitUnits * kRecordStride];
+    __shared__ u32x4 table[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int spans = (units + kSplitUnits - 1) / kSplitUnits;
+    const unsigned rb = blockIdx.x / spans;
+    const int u0 = static_cast<int>(blockIdx.x % spans) * kSplitUnits;
+    const int u = u0 + (lane >> 4), g = lane & 15;
+    const bool live = u < units;
+    const size_t at = ((size_t)rb * 16 + wave * 4) * K + (size_t)u * 128 + g * 8;
+    u32x4 in[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        in[j] = u32x4{0u, 0u, 0u, 0u};
+        if (live)
+            in[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(A + at + (size_t)j * K));
+    }
+    if (threadIdx.x < 16)
+        table[threadIdx.x] = reinterpret_cast<const u32x4*>(split_table.e)[threadIdx.x];
+    __syncthreads();
+    // lane (column group g % 4, row) of a record keeps step g / 4's values of this granule
+    uint8_t* const rec = records + (lane >> 4) * kRecordStride;
+    uint8_t* const value = rec + ((g >> 3) * 4 + (g & 3)) * kBlockStride + wave * 64 + ((g >> 2) & 1) * 8;
+    uint8_t* const place = rec + 8 * kBlockStride + (g & 3) * 64 + wave * 16;
+    const uint8_t* const entries = reinterpret_cast<const uint8_t*>(table);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        unsigned flags = 0;  // element 2 i + h kept: bit 2 i + 16 h
+#pragma unroll
+        for (int i = 0; i < 4; i++)  // (unequal to zero as a float: NaN counts, -0 does not)
+            flags |= __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_bit_cast(u16x2, in[j][i] & 0x7fff7fffu), u16x2{1, 1}))
+                     << (2 * i);
+        const unsigned mask = flags | flags >> 15;
+        const u32x4 lo = *reinterpret_cast<const u32x4*>(entries + ((mask << 4) & 0xf0u));
+        const u32x4 hi = *reinterpret_cast<const u32x4*>(entries + (mask & 0xf0u));
+        *reinterpret_cast<u32x2*>(value + j * 16) = u32x2{__builtin_amdgcn_perm(in[j][1], in[j][0], lo[0]),
+                                                          __builtin_amdgcn_perm(in[j][3], in[j][2], hi[0])};
+        if (RESIDUAL && live)
+            *reinterpret_cast<u32x4_any*>(residual + at + (size_t)j * K) =
+                u32x4{0u, __builtin_amdgcn_perm(in[j][1], in[j][0], lo[1]), 0u, __builtin_amdgcn_perm(in[j][3], in[j][2], hi[1])};
+        // the four steps' positions of (column group, row) are four lanes apart
+        int word = static_cast<int>((lo[2] | hi[2] << 4) << (8 * (g >> 2)));
+        word |= __builtin_amdgcn_update_dpp(0, word, 0x124, 0xf, 0xf, false);  // row_ror 4, 8
+        word |= __builtin_amdgcn_update_dpp(0, word, 0x128, 0xf, 0xf, false);
+        if (g < 4)
+            *reinterpret_cast<int*>(place + j * 4) = word;
+    }
+    __syncthreads();
+    // records are numbered ((rb / 8) * units + u) * 8 + rb % 8
+    uint8_t* const out = packed + ((size_t)(rb / kGroupBlocks * units + u0) * kGroupBlocks + rb % kGroupBlocks) * kRecordBytes;
+#pragma unroll
+    for (int j = 0; j < kSplitUnits * 128 / 256; j++) {
+        const int id = threadIdx.x + j * 256, r = id >> 7, granule = id & 127;
+        if (u0 + r < units)
+            *reinterpret_cast<u32x4_byte*>(out + (size_t)r * kGroupBlocks * kRecordBytes + granule * 16) =
+                *reinterpret_cast<const u32x4*>(records + r * kRecordStride + (granule >> 4) * kBlockStride + (granule & 15) * 16);
+    }
+    if (u0 + wave < units)
+        *reinterpret_cast<u32_byte*>(out + (size_t)wave * kGroupBlocks * kRecordBytes + 2048 + lane * 4) =
+            *reinterpret_cast<const unsigned*>(records + wave * kRecordStride + 8 * kBlockStride + lane * 4);
 }
 
 // A: row-major M x K fp16 in device memory (M % 16 == 0, K % 128 == 0, checked by the caller);
@@ -87,13 +151,12 @@ __global__ __launch_bounds__(256) void a24_split_pack_kernel(const uint16_t* __r
 extern "C" int a24_launch_split_pack(void* stream, const void* A, void* packed, void* residual, int M, int K)
 {
     const int units = K / 128;
-    const long records = static_cast<long>(M / 16) * units;
-    const long blocks = (records * 64 + 255) / 256;
+    const long blocks = static_cast<long>(M / 16) * ((units + kSplitUnits - 1) / kSplitUnits);
     if (blocks < 1 || blocks > 0x7fffffffL)
         return static_cast<int>(hipErrorInvalidValue);
-    hipLaunchKernelGGL(a24_split_pack_kernel, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream),
-                       static_cast<const uint16_t*>(A), static_cast<uint8_t*>(packed), static_cast<uint16_t*>(residual), K,
-                       units, records);
+    auto* const kernel = residual ? a24_split_pack_kernel<true> : a24_split_pack_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const uint16_t*>(A), static_cast<uint8_t*>(packed), static_cast<uint16_t*>(residual), K, units);
     return static_cast<int>(hipGetLastError());
 }
 
@@ -118,8 +181,6 @@ __device__ __forceinline__ bool residual_kept(unsigned v)
 __global__ __launch_bounds__(256) void a24_residual_count_kernel(const uint16_t* __restrict__ A2, int K, int units,
                                                                  unsigned tasks, int* __restrict__ offsets)
 {
-    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
     const unsigned task = (gridDim.x - 1 - blockIdx.x) * 4 + (threadIdx.x >> 6);
     if (task >= tasks)
         return;

@@ -1004,3 +1004,28 @@ def test_activations_straight_into_lds(spmm, oracle, N, M, K, split_k, sparsity)
     # one rounding of each slab and of the sum, 2^-11 of what a slab or the sum can be, and fp32 sums (K additions of 2^-24)
     bound = size * (2 * 2.0 ** -11 + K * 2.0 ** -24) + 2.0 ** -24
     assert ((got.double().cpu() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M,K", [(128, 128), (128, 256), (256, 384), (384, 512), (128, 640), (256, 1152)])  # spans of one to four units
+@pytest.mark.parametrize("begin", [0, 1])  # ... of a view that begins anywhere
+def test_device_split_pack_groups_of_every_kind(spmm, M, K, begin):
+    """Every choice of kept elements in a group of four beside every other, with signed zeros (not kept), NaN,
+    infinities, subnormals and extremes among them: the host functions' bits, with and without the residual."""
+    torch = _torch()
+    rng = np.random.default_rng(M + K)
+    kept = np.array([0x7E00, 0xFE01, 0x7C00, 0xFC00, 0x0001, 0x8001, 0x7BFF, 0xFBFF, 0x3C00], dtype=np.uint16)
+    A = np.where(np.arange(M * K) // 7 % 2, 0x8000, 0).astype(np.uint16)
+    masks = np.repeat(np.arange(M * K // 4) % 16, 4) >> (np.arange(M * K) % 4) & 1
+    A[masks == 1] = rng.choice(kept, size=int(masks.sum()))
+    A = A.reshape(M // 16, 16, K // 4, 4).transpose(0, 2, 1, 3).reshape(M, K)  # the sixteen kinds over a record's rows as well
+    A1, A2 = spmm.HeteroSparse_Decompose(A.view(np.float16))
+    want = spmm.HeteroSparse_PackA1(A1)
+    buf = torch.zeros(M * K + 8, dtype=torch.float16, device="cuda:0")
+    d_A = buf[begin:begin + M * K].view(M, K)
+    d_A.copy_(torch.from_numpy(A.view(np.int16).copy()).to("cuda:0").view(torch.float16))
+    print(f"[gpu case] split pack kinds M={M} K={K} begin={begin}", flush=True)
+    packed, residual = spmm.split_pack_on_device(d_A)
+    alone, none = spmm.split_pack_on_device(d_A, want_residual=False)
+    assert none is None
+    assert np.array_equal(packed.cpu().numpy(), want) and torch.equal(packed, alone)
+    assert np.array_equal(residual.cpu().numpy().view(np.uint16), A2.view(np.uint16))
