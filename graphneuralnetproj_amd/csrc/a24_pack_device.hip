@@ -167,6 +167,12 @@ namespace {
 
 constexpr int kMaxListWords = 16 * 128 / 2;  // a residual holds at most two of every four
 
+// x + the lanes of the mask below this one
+__device__ __forceinline__ int lower_lanes(uint64_t mask, int x)
+{
+    return static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(mask >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), static_cast<unsigned>(x))));
+}
 __device__ __forceinline__ bool residual_kept(unsigned v)
 {
     return (v & 0x7fffu) != 0;
@@ -232,54 +238,114 @@ __global__ __launch_bounds__(offscan::kThreads) void a24_residual_scan_kernel(in
     }
 }
 
-// The words.  Bound by instruction issue and by the dealing below; the residual is read once.
+// The words.  Bound by instruction issue beside the read of the residual (21504 x 7168: 51 us at 95 % sparsity, where
+// nothing is dealt, 99 at 60 %).
 //
 // In a list's order (a24_pack.cpp: order_by_bank) the words of one LDS bank are neighbours: banks by
 // (count descending, number ascending), a bank's words as collected.  A bank's words come from 16
 // known column pairs, one per row (row r: pair bank ^ (r << 2)), so lane b of a list's wave reads
 // bank b's 32 candidates itself, a whole 256-byte row per load, and knows its count, its place
-// among the banks (six ballots) and its words without any exchange.  Where a word goes is then
-// the result of dealing the banks' words to the rounds one by one, each word depending on the one
-// before; it depends on the counts alone, so one LANE deals for one list: 32 lists of a workgroup
+// among the banks (a ballot per count there is) and its words without any exchange.  Where a word goes is then
+// the result of dealing the banks' words to the rounds, bank after bank, each depending on the one
+// before; it depends on the counts alone, so one LANE deals for one list: the lists of a workgroup
 // side by side (one lane of one wave dealing for the wave's only list took 1150 us on the
-// 21504 x 7168 residual of a 60 % sparse weight; now 138).  A list of at most 64 words stays in
-// row-major order, as the host leaves it.
+// 21504 x 7168 residual of a 60 % sparse weight; 32 lists side by side, word by word, 137; a lap of a bank at a time, every
+// lane at its own bank, 110; with 16 lists 99).  A list of at most 64 words stays in row-major order, as the host leaves it.
 //
-// So many workgroups per compute unit as the dealing waves need to hide each other: 256 threads, 18.5
-// KiB of LDS, 64 registers (lists beyond four rounds spill a few), the residual read a second time for
-// the writing (from the last-level cache) instead of kept in registers.  (Eight waves with 51 KiB, registers kept, words placed as 16-bit numbers: 211 us.
-// Dealing by laps, every round with room one word in the order of its room, four keys sorted per lap:
-// 302 us instead of 211, the lanes diverge.)
+// The residual is read a second time for the writing (from the last-level cache) instead of kept in
+// registers: more workgroups per compute unit, whose dealing waves hide each other.
 constexpr int kEmitWaves = 4;
-// Lists per workgroup: 32 where that makes a chip full of workgroups (eight per compute unit), else
-// eight: the lists of a wave follow one another, so few lists are better spread over more waves
-// (whole calls at 50 / 70 / 95 % sparsity, 2048 x 4096 = 4096 lists: 72 / 56 / 47 us, with 32 a group
-// 91 / 75 / 59; 16384 lists are the 2048 groups of eight that run at once).
-constexpr int kManyLists = 32, kFewLists = 8;
+// Lists per workgroup: the lists of a wave follow one another and the others wait while one wave deals, so few lists
+// are better spread over more waves, and many are better dealt 16 at a time (whole calls at 50 / 60 / 95 %:
+// 2048 x 4096 = 4096 lists: eight to a workgroup 22 / 17 / 7 us, 16 25 / 19 / 10; 5120 x 5248 = 13120: 35 / 26 / 15 and
+// 36 / 29 / 16; 4096 x 8192 = 16384: 40 / 30 / 16 and 37 / 30 / 16; 7168 x 7168 = 25088: 56 / 42 / 22 and 52 / 41 / 23).
+constexpr int kManyLists = 16, kFewLists = 8;
 constexpr long kManyFrom = 16384;
 
 // A word of the bank-sorted sequence goes to the round that has the fewest words of its bank, then
-// the most room, then the lowest number: the largest of keys (63 - words of the bank, room - 1, last -
-// round), zero for a full round.  For a list of at most four rounds the lower two fields are one
-// byte, the word's place in code; for longer lists the place is written as two bytes.
+// the most room, then the lowest number.  So a bank's words go round by round in laps: once around the
+// rounds that have room, those with the most room first, then around again.
+//
+// For a list of at most four rounds a word's place in code is one byte, (room - 1) * 4 + (3 - round); for longer
+// lists the place is written as two bytes.  (Three more bytes: what a lap writes beyond its own words.)
 __device__ __forceinline__ int place_bytes(int n)
 {
-    return n <= 256 ? n : 2 * n;
+    return n <= 256 ? n + 3 : 2 * n;
 }
-__device__ __forceinline__ int place_of(const uint8_t* places, int p, int n)
+// The last places of a list's four rounds, a byte each, the last round's first (n <= 256).
+__device__ __forceinline__ unsigned round_ends(int n)
+{
+    unsigned ends = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        ends |= static_cast<unsigned>((256 - 64 * k < n ? 256 - 64 * k : n) - 1) << (8 * k);
+    return ends;
+}
+// n > 256: `ends` is not looked at
+__device__ __forceinline__ int place_of(const uint8_t* places, int p, int n, unsigned ends)
 {
     if (n > 256)
         return places[p] | places[p + n] << 8;
-    const int code = places[p];
-    const int end = 256 - 64 * (code & 3);  // 64 * (round + 1)
-    return (end < n ? end : n) - 1 - (code >> 2);
+    const unsigned code = places[p];
+    return static_cast<int>(__builtin_amdgcn_perm(0, ends, (code & 3u) | 0x0c0c0c00u) - (code >> 2));
 }
 
-// Deals one list of n words, 64 < n <= 64 * R, whose banks hold counts[0] >= counts[1] >= ... words.
+// Deals one list of n words, 64 < n <= 64 * R and n <= 256, whose banks hold counts[0] >= counts[1] >= ... words
+// (a byte after the last one may be read).  A step of the loop is one lap of this lane's current bank, whatever bank the
+// other lanes are at.  The rounds' codes are kept in order, largest first; a round without room has a negative one.
 template<int R>
-__device__ __forceinline__ void deal(const unsigned* counts, int n, uint8_t* places)
+__device__ __forceinline__ void deal_laps(const uint8_t* counts, int n, uint8_t* places)
 {
-    constexpr int kRoundBits = R <= 4 ? 2 : 4, kLast = (1 << kRoundBits) - 1;
+    static_assert(R >= 2 && R <= 4, "two bits for the round");
+    int key[R];
+    const int rounds = (n + 63) >> 6;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int room = r < rounds - 1 ? 64 : (r == rounds - 1 ? n - 64 * (rounds - 1) : 0);
+        key[r] = (room - 1) * 4 + (3 - r);
+    }
+    auto order = [&](int a, int b) __attribute__((always_inline)) {
+        const int x = key[a], y = key[b];
+        key[a] = x > y ? x : y;
+        key[b] = x > y ? y : x;
+    };
+    const uint8_t* const end = places + n;
+    int c = counts[0], following = counts[1];
+    while (places < end) {
+#pragma unroll
+        for (int j = 0; j < R; j++)  // what is not taken is written over by the next lap
+            places[j] = static_cast<uint8_t>(key[j]);
+        int taken = 1;
+        key[0] -= 4;
+#pragma unroll
+        for (int j = 1; j < R; j++) {
+            const bool takes = c > j && key[j] >= 0;
+            key[j] -= takes ? 4 : 0;
+            taken += takes ? 1 : 0;
+        }
+        places += taken;
+        c -= taken;
+        order(0, 1);
+        if constexpr (R == 3) {
+            order(1, 2);
+            order(0, 1);
+        } else if constexpr (R == 4) {
+            order(2, 3);
+            order(0, 2);
+            order(1, 3);
+            order(1, 2);
+        }
+        counts += c == 0 ? 1 : 0;
+        c = c == 0 ? following : c;
+        following = counts[1];
+    }
+}
+
+// ... of 256 < n <= 1024 words, word by word: the largest of keys (63 - words of the bank, room - 1, last - round), zero
+// for a full round.
+__device__ __forceinline__ void deal_long(const unsigned* counts, int n, uint8_t* places)
+{
+    constexpr int R = 16, kRoundBits = 4, kLast = (1 << kRoundBits) - 1;
     constexpr unsigned kRoom = 1u << kRoundBits, kOne = 64u << kRoundBits;  // units of the two upper fields
     unsigned key[R];
     const int rounds = (n + 63) >> 6;
@@ -301,14 +367,10 @@ __device__ __forceinline__ void deal(const unsigned* counts, int n, uint8_t* pla
                 for (int r = 1; r < R; r++)
                     best = key[r] > best ? key[r] : best;
                 const unsigned room = best & (kOne - kRoom);  // minus one
-                if constexpr (R <= 4) {
-                    *places = static_cast<uint8_t>(best);
-                } else {
-                    const int end = 1024 - 64 * static_cast<int>(best & kLast);
-                    const int place = (end < n ? end : n) - 1 - static_cast<int>(room / kRoom);
-                    places[0] = static_cast<uint8_t>(place);
-                    places[n] = static_cast<uint8_t>(place >> 8);
-                }
+                const int end = 1024 - 64 * static_cast<int>(best & kLast);
+                const int place = (end < n ? end : n) - 1 - static_cast<int>(room / kRoom);
+                places[0] = static_cast<uint8_t>(place);
+                places[n] = static_cast<uint8_t>(place >> 8);
                 const unsigned then = room == 0 ? 0u : best - kOne - kRoom;
 #pragma unroll
                 for (int r = 0; r < R; r++)
@@ -325,9 +387,9 @@ __global__ __launch_bounds__(kEmitWaves * 64, 8) void a24_residual_emit_kernel(c
                                                                                uint32_t* __restrict__ words)
 {
     constexpr int kListsPerWave = kEmitLists / kEmitWaves;
-    constexpr int kPlaces = kEmitLists * 256;  // bytes: lists of 256 words (an ordinary residual has up to 200) are dealt in one pass
+    constexpr int kPlaces = kEmitLists * 256 > 2 * kMaxListWords ? kEmitLists * 256 : 2 * kMaxListWords;  // bytes: lists of 256 words (an ordinary residual has up to 200) are dealt in one pass
     static_assert(kPlaces >= 2 * kMaxListWords, "the longest list has to fit");
-    __shared__ unsigned images[kEmitWaves][8 * 64];  // per wave: half of a list's block, [row][bank] column pairs
+    __shared__ unsigned images[kEmitWaves][16 * 64];  // per wave: a list's block, [row][bank] column pairs
     __shared__ unsigned sorted[kEmitLists][17];      // counts of a list's banks, one byte each, largest first
     __shared__ int length[kEmitLists];
     __shared__ uint8_t places[kPlaces];
@@ -370,30 +432,29 @@ __global__ __launch_bounds__(kEmitWaves * 64, 8) void a24_residual_emit_kernel(c
         }
         unsigned pairs[16];
         load_list(list, pairs);
-        unsigned mask = 0;
+        unsigned halves[2] = {0, 0};  // rows 0 .. 7, 8 .. 15: bit 2 (r % 8) + 16 h
 #pragma unroll
         for (int r = 0; r < 16; r++)
-            mask |= (residual_kept(pairs[r]) ? 1u << (2 * r) : 0u) | (residual_kept(pairs[r] >> 16) ? 2u << (2 * r) : 0u);
+            halves[r >> 3] |= __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_bit_cast(u16x2, pairs[r] & 0x7fff7fffu), u16x2{1, 1}))
+                              << (2 * (r & 7));
+        const unsigned mask = ((halves[0] | halves[0] >> 15) & 0xffffu) | (halves[1] | halves[1] >> 15) << 16;
         kept[i] = mask;
         const int count = __popc(mask);
-        // the banks with more words, and those with as many and a lower number, bit by bit
-        uint64_t more = 0, equal = ~0ull, planes[6];
-        int n = 0;
-#pragma unroll
-        for (int bit = 5; bit >= 0; bit--) {
-            const bool set = (count >> bit) & 1;
-            planes[bit] = __ballot(set);
-            n += __popcll(planes[bit]) << bit;
-            more |= set ? 0ull : equal & planes[bit];
-            equal &= set ? planes[bit] : ~planes[bit];
+        // the banks' places from the last one on: by count upwards (a few counts only), equal ones by number
+        int n = 0, banks = 64, before = 0, place = 0;  // words and banks of the counts so far; this bank's
+        uint64_t left = ~0ull;
+        for (int c = 0; left != 0; c++) {
+            const uint64_t same = __ballot(count == c);
+            const int number = __popcll(same);
+            const int lower = lower_lanes(same, 0);
+            n += c * number;
+            banks -= number;
+            before = count == c ? c * lower - n : before;
+            place = count == c ? banks + lower : place;
+            left &= ~same;
         }
-        const uint64_t before = more | (equal & ((1ull << L) - 1));
-        int s = 0;
-#pragma unroll
-        for (int bit = 0; bit < 6; bit++)
-            s += __popcll(before & planes[bit]) << bit;
-        start[i] = s;
-        reinterpret_cast<uint8_t*>(sorted[li])[__popcll(before)] = static_cast<uint8_t>(count);
+        start[i] = n + before;
+        reinterpret_cast<uint8_t*>(sorted[li])[place] = static_cast<uint8_t>(count);
         // (a block with more kept values than a residual can hold is not this format's input: nothing is written,
         // nor where the offsets are not those of this matrix: the words would land in other lists' room or behind all)
         int at = offsets[list];
@@ -416,14 +477,14 @@ __global__ __launch_bounds__(kEmitWaves * 64, 8) void a24_residual_emit_kernel(c
                     const int r = half * 8 + r8;
                     const unsigned pair = natural[r8];
                     const bool lo = residual_kept(pair), hi = residual_kept(pair >> 16);
-                    const uint64_t los = __ballot(lo), his = __ballot(hi), below = (1ull << L) - 1;
-                    const int place = at + __popcll(los & below) + __popcll(his & below);
+                    const uint64_t los = __ballot(lo), his = __ballot(hi);
+                    const int place = lower_lanes(his, lower_lanes(los, at));
                     const unsigned address = r * 256 + (((L >> 2) ^ r) << 4) + (L & 3) * 4;
                     if (lo)
                         words[(size_t)place] = (pair & 0xffffu) | address << 16;
                     if (hi)
                         words[(size_t)place + (lo ? 1 : 0)] = pair >> 16 | (address + 2) << 16;
-                    at += __popcll(los) + __popcll(his);
+                    at += static_cast<int>(__popcll(los) + __popcll(his));
                 }
                 asm volatile("" ::: "memory");
             }
@@ -439,12 +500,15 @@ __global__ __launch_bounds__(kEmitWaves * 64, 8) void a24_residual_emit_kernel(c
         const int last = __popcll(fit);
         const int at = through - place_bytes(mine) - dealt;
         if (w == 0 && L >= first && L < last && mine > 0) {
+            const uint8_t* const counts = reinterpret_cast<const uint8_t*>(sorted[L]);
             if (mine > 256)  // (lane by lane: the form of a list's places goes by its own length)
-                deal<16>(sorted[L], mine, places + at);
+                deal_long(sorted[L], mine, places + at);
             else if (__any(mine > 192))
-                deal<4>(sorted[L], mine, places + at);
+                deal_laps<4>(counts, mine, places + at);
+            else if (__any(mine > 128))
+                deal_laps<3>(counts, mine, places + at);
             else
-                deal<3>(sorted[L], mine, places + at);
+                deal_laps<2>(counts, mine, places + at);
         }
         __syncthreads();
 #pragma unroll
@@ -457,21 +521,19 @@ __global__ __launch_bounds__(kEmitWaves * 64, 8) void a24_residual_emit_kernel(c
             load_list(list_of(i), pairs);
             const uint8_t* const list_places = places + __builtin_amdgcn_readlane(at, li);
             uint32_t* const out = words + (size_t)offsets[list_of(i)];
+            const unsigned ends = round_ends(n);
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                image[r * 64 + L] = pairs[r];
+            asm volatile("" ::: "memory");
             int p = start[i];
-#pragma unroll
-            for (int half = 0; half < 2; half++) {
-#pragma unroll
-                for (int r = 0; r < 8; r++)
-                    image[r * 64 + L] = pairs[half * 8 + r];
-                asm volatile("" ::: "memory");
-                for (unsigned mask = kept[i] >> (16 * half) & 0xffffu; mask; mask &= mask - 1, p++) {
-                    const int e = __ffs(static_cast<int>(mask)) - 1;
-                    const unsigned address = (e >> 1) * 256 + L * 4 + (e & 1) * 2;  // in the half image as in the kernel's own
-                    const unsigned value = *reinterpret_cast<const unsigned short*>(reinterpret_cast<const uint8_t*>(image) + address);
-                    out[place_of(list_places, p, n)] = value | (address + half * 2048) << 16;
-                }
-                asm volatile("" ::: "memory");
+            for (unsigned mask = kept[i]; mask; mask &= mask - 1, p++) {
+                const unsigned e = __builtin_ctz(mask);
+                const unsigned address = (e * 130u & 0xf02u) | L * 4;  // (e / 2) * 256 + (e % 2) * 2: here as in the product's own image
+                const unsigned value = *reinterpret_cast<const unsigned short*>(reinterpret_cast<const uint8_t*>(image) + address);
+                out[static_cast<unsigned>(place_of(list_places, p, n, ends))] = value | address << 16;
             }
+            asm volatile("" ::: "memory");
         }
         first = last;
         if (first < kEmitLists) {

@@ -1029,3 +1029,40 @@ def test_device_split_pack_groups_of_every_kind(spmm, M, K, begin):
     assert none is None
     assert np.array_equal(packed.cpu().numpy(), want) and torch.equal(packed, alone)
     assert np.array_equal(residual.cpu().numpy().view(np.uint16), A2.view(np.uint16))
+
+
+@pytest.mark.parametrize("M,K", [(256, 1280), (4224, 8192)])  # eight lists to a workgroup, and 16
+def test_device_residual_lists_of_uneven_banks(spmm, oracle, M, K):
+    """The dealing of a bank's words to the rounds: lengths at the edges of one to five rounds, with the words
+    spread over all banks, over a few of them (up to 32 words each: many laps, rounds that fill up on the way), and over
+    the leading or trailing ones, side by side in a workgroup; the host's words, bit for bit."""
+    torch = _torch()
+    rng = np.random.default_rng(K)
+    rows, units = M // 16, K // 128
+    A2 = np.zeros((rows, units, 16, 128), dtype=np.uint16)
+    lengths = (1, 63, 64, 65, 66, 96, 127, 128, 129, 160, 191, 192, 193, 194, 224, 255, 256, 257, 300, 511, 512, 513)
+    kinds = []
+    for words in lengths:
+        for share in (1.0, 0.5, 0.25, 0.15):  # of the 2048 places
+            for first in (True, False):
+                n = max(int(2048 * share), words)
+                kinds.append((words, n, first))
+    # place (bank, row, half) in bank order: bank b's pair in row r is b ^ (r << 2)
+    bank, row, half = np.meshgrid(np.arange(64), np.arange(16), np.arange(2), indexing="ij")
+    flat = (row * 128 + (bank ^ (row << 2)) * 2 + half).ravel()
+    order = rng.permutation(rows * units)
+    for i, at in enumerate(order):
+        words, n, first = kinds[i % len(kinds)]
+        places = flat[:n] if first else flat[2048 - n:]
+        block = np.zeros(2048, dtype=np.uint16)
+        block[rng.choice(places, size=words, replace=False)] = rng.integers(1, 0x7C00, size=words)
+        A2[at // units, at % units] = block.reshape(16, 128)
+    A2 = np.ascontiguousarray(A2.transpose(0, 2, 1, 3).reshape(M, K)).view(np.float16)
+    want_words, want_offs, want_longest = spmm.HeteroSparse_PackA2(A2)
+    d_A2 = torch.from_numpy(A2.view(np.int16).copy()).to("cuda:0").view(torch.float16)
+    print(f"[gpu case] residual lists of uneven banks M={M} K={K}", flush=True)
+    words, offs, longest = spmm.pack_residual_on_device(d_A2)
+    torch.cuda.synchronize()
+    assert longest == want_longest
+    assert np.array_equal(offs.cpu().numpy(), want_offs)
+    assert np.array_equal(words.cpu().numpy().view(np.uint32), want_words)
