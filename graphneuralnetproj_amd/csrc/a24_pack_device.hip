@@ -25,10 +25,16 @@ namespace {
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+using offscan::u16x2;
 typedef u32x4 u32x4_any __attribute__((aligned(2)));   // the matrices' granules may lie at any element,
 typedef u32x4 u32x4_byte __attribute__((aligned(1)));  // the records at any byte
 typedef unsigned u32_byte __attribute__((aligned(1)));
+
+// 1 in each half that is kept: unequal to zero as a float (NaN counts, -0 does not)
+__device__ __forceinline__ unsigned kept_halves(unsigned pair)
+{
+    return __builtin_bit_cast(unsigned, offscan::at_most_one(__builtin_bit_cast(u16x2, pair & 0x7fff7fffu)));
+}
 
 constexpr int kSplitUnits = 4;  // units per workgroup
 // A record in LDS: its eight 256-byte blocks of values (block = step / 2 * 4 + column group) 272 bytes apart, then the
@@ -113,9 +119,8 @@ __global__ __launch_bounds__(256) void a24_split_pack_kernel(const uint16_t* __r
     for (int j = 0; j < 4; j++) {
         unsigned flags = 0;  // element 2 i + h kept: bit 2 i + 16 h
 #pragma unroll
-        for (int i = 0; i < 4; i++)  // (unequal to zero as a float: NaN counts, -0 does not)
-            flags |= __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_bit_cast(u16x2, in[j][i] & 0x7fff7fffu), u16x2{1, 1}))
-                     << (2 * i);
+        for (int i = 0; i < 4; i++)
+            flags |= kept_halves(in[j][i]) << (2 * i);
         const unsigned mask = flags | flags >> 15;
         const u32x4 lo = *reinterpret_cast<const u32x4*>(entries + ((mask << 4) & 0xf0u));
         const u32x4 hi = *reinterpret_cast<const u32x4*>(entries + (mask & 0xf0u));
@@ -138,8 +143,8 @@ __global__ __launch_bounds__(256) void a24_split_pack_kernel(const uint16_t* __r
     for (int j = 0; j < kSplitUnits * 128 / 256; j++) {
         const int id = threadIdx.x + j * 256, r = id >> 7, granule = id & 127;
         if (u0 + r < units)
-            *reinterpret_cast<u32x4_byte*>(out + (size_t)r * kGroupBlocks * kRecordBytes + granule * 16) =
-                *reinterpret_cast<const u32x4*>(records + r * kRecordStride + (granule >> 4) * kBlockStride + (granule & 15) * 16);
+            __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(records + r * kRecordStride + (granule >> 4) * kBlockStride + (granule & 15) * 16),
+                                        reinterpret_cast<u32x4_byte*>(out + (size_t)r * kGroupBlocks * kRecordBytes + granule * 16));
     }
     if (u0 + wave < units)
         *reinterpret_cast<u32_byte*>(out + (size_t)wave * kGroupBlocks * kRecordBytes + 2048 + lane * 4) =
@@ -206,8 +211,7 @@ __global__ __launch_bounds__(256) void a24_residual_count_kernel(const uint16_t*
         for (int r = 0; r < 16; r++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const u16x2 mag = __builtin_bit_cast(u16x2, v[r][i] & 0x7fff7fffu);
-                c += __builtin_elementwise_min(mag, u16x2{1, 1});
+                c += __builtin_bit_cast(u16x2, kept_halves(v[r][i]));
             }
         n = c[0] + c[1];
     }
@@ -435,8 +439,7 @@ __global__ __launch_bounds__(kEmitWaves * 64, 8) void a24_residual_emit_kernel(c
         unsigned halves[2] = {0, 0};  // rows 0 .. 7, 8 .. 15: bit 2 (r % 8) + 16 h
 #pragma unroll
         for (int r = 0; r < 16; r++)
-            halves[r >> 3] |= __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_bit_cast(u16x2, pairs[r] & 0x7fff7fffu), u16x2{1, 1}))
-                              << (2 * (r & 7));
+            halves[r >> 3] |= kept_halves(pairs[r]) << (2 * (r & 7));
         const unsigned mask = ((halves[0] | halves[0] >> 15) & 0xffffu) | (halves[1] | halves[1] >> 15) << 16;
         kept[i] = mask;
         const int count = __popc(mask);

@@ -1,5 +1,5 @@
-// Running totals of per-tile or per-list counts in device memory, in place, by one workgroup.
-// Shared by the Tiled-CSL encoder and the residual packer.
+// Running totals of per-tile or per-list counts in device memory, in place, by one workgroup, and two small functions on
+// lanes and halves.  Shared by the Tiled-CSL encoder and the residual packer.
 //
 // Bound by the latency of its few trips to memory, not by bandwidth: 75264 counts are 0.3 MB.  A
 // workgroup takes 16384 counts per step, 16 bytes per lane and load with whole lines per wave, the
@@ -14,6 +14,17 @@ namespace offscan {
 
 constexpr int kThreads = 1024, kWaves = kThreads / 64, kRows = 4;
 constexpr int kStep = kThreads * 4 * kRows;
+
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+// min(x, 1) in both halves, in one instruction: the compiler takes a minimum with one apart into a comparison and a
+// select per half.
+__device__ __forceinline__ u16x2 at_most_one(u16x2 x)
+{
+    u16x2 r;
+    asm("v_pk_min_u16 %0, %1, %2" : "=v"(r) : "v"(x), "s"(0x00010001));
+    return r;
+}
 
 typedef int i32x4_u __attribute__((ext_vector_type(4), aligned(4)));  // any int boundary will do
 

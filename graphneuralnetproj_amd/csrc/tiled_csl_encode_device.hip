@@ -24,9 +24,9 @@ namespace {
 
 constexpr int kTileRows = 128, kTileCols = 64, kBanks = 32, kThreads = 256, kWaves = kThreads / 64;
 constexpr int kRowGroups = kThreads / kBanks, kRowsPerThread = kTileRows / kRowGroups;  // 8, 16
-constexpr int kMaxLevel = 2 * kTileRows + 4;  // 256 per bank + up to 3 pads, rounded up
+constexpr int kMaxLevel = 2 * kTileRows + 4;  // 256 per bank + up to 3 pads stay below
 
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+using offscan::u16x2;
 // The matrix and the words may lie at any element: callers' views begin anywhere (the loads and stores are as wide all the same).
 typedef uint32_t pair_any __attribute__((aligned(2)));
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
@@ -37,13 +37,14 @@ typedef uint32_t u32x4_word __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ u16x2 kept_halves(uint32_t pair)
 {
     const u16x2 mag = __builtin_bit_cast(u16x2, pair & 0x7fff7fffu);
-    const u16x2 nan = (mag + u16x2{0x3ff, 0x3ff}) >> u16x2{15, 15};  // past 0x7c00
-    return __builtin_elementwise_min(mag, u16x2{1, 1}) - nan;
+    const u16x2 number = __builtin_elementwise_sub_sat(u16x2{0x7c01, 0x7c01}, mag);  // zero for NaN
+    return offscan::at_most_one(__builtin_elementwise_min(mag, number));
 }
 
 // Vectors per tile into offsets[tile + 1].  Bound by HBM (the matrix is read once): a wave reads 32
 // rows of up to eight consecutive tiles, a contiguous KiB per load, all in flight.  (Four bytes per
-// lane, one tile per workgroup: 86 us for 411 MB, now 74.)  Workgroups go from the matrix's
+// lane, one tile per workgroup: 86 us for 411 MB, now 74, and 63 where the emit kernel before it stored past
+// the cache.)  Workgroups go from the matrix's
 // start to its end, the emit kernel's from end to start: it begins with what is left in the
 // last-level cache.
 constexpr int kCountTiles = 8;
@@ -117,14 +118,18 @@ __device__ __forceinline__ int half_wave_reduce(int x, int neutral, Op op)
 // the write of the words.
 //   * An element's place in its bank's list is a prefix count; its place in the pop order is the
 //     number of pops before its level plus the number of lower banks as tall, both from one LDS
-//     read of the level's entry (mask of banks, pops before).  The four waves fill that table level by
-//     level from ballots on the banks' sizes, each its quarter of the levels.
+//     read of the level's entry (mask of banks, pops before).  The four waves fill that table two levels at a
+//     time from ballots on the banks' sizes (the upper lanes hold the banks as well), each its quarter of the levels.
+//     A candidate that is not kept reads an entry whose pops lie behind the sequence: eight instructions a candidate, kept or not.
 //   * Words go into LDS in pop order and leave it in the order of emission (:379-424), which is plain
 //     arithmetic on the output position: four conflict-free reads and one 16-byte store per vector.
 //   * 4096 words of LDS for the sequence, so that seven workgroups share a compute unit; a tile beyond
 //     that (50 % dense) takes another pass over the registers for every 3968 words.
+//   * The words are stored past the caches (nt): whole lines that nothing here reads again (21504 x 7168 at 60 %: 111 us,
+//     now 97; the count kernel of the next weight 72 us, now 63).
 // (Bank lists staged in LDS, level sums by one thread over 260 levels, words stored one by one:
-// 303 us for a 28672 x 7168 weight at 80 %, now 130, 4.4 TB/s.)
+// 303 us for a 28672 x 7168 weight at 80 %; 766 instructions per wave and tile: 124; now 109, 5.3 TB/s.  Alone, 21504 x 7168
+// at 50 / 80 / 95 %: 157 / 97 / 88 us, now 132 / 77 / 70; 1024 x 1024 at 80 %: 5.3, now 4.9.)
 constexpr int kSeqWords = 4096, kPassWords = kSeqWords - 128;  // the first pass takes the tail's up to 124 pops as well
 
 __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* __restrict__ A, int K, int tiles_k,
@@ -132,7 +137,8 @@ __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* _
 {
     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
     __shared__ uint32_t seq[kSeqWords + 64];   // pops first .. first + kSeqWords - 1; then where words of other passes go
-    __shared__ u32x2 levels[kMaxLevel + 1];    // level l: banks at least l tall, pops made before the level starts
+    // entry kMaxLevel - l: banks at least l tall, pops made before the level starts; entry 0: where words that are not go
+    __shared__ u32x2 levels[kMaxLevel + 1];
     __shared__ int grp_count[kRowGroups][kBanks];
     __shared__ int grp_zero[kRowGroups][kBanks];
 
@@ -146,21 +152,20 @@ __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* _
 
     // 1. this thread's 16 rows of bank b: mark the kept elements, note the first other position.
     //    Row m gives bank b the pair of adjacent columns whose swizzled positions are 2 b, 2 b + 1.
-    const uint16_t* const own_rows = tile + (size_t)(rg * kRowsPerThread) * K;
+    // (a row's address is uniform but for this lane's part, of which there are eight)
+    const uint8_t* const rows = reinterpret_cast<const uint8_t*>(tile) + (size_t)(wave * 2 * kRowsPerThread) * K * 2;
+    const uint32_t own_row = (rg & 1) * (uint32_t)kRowsPerThread * K * 2;
     uint32_t pairs[kRowsPerThread];
 #pragma unroll
-    for (int i = 0; i < kRowsPerThread; i++) {
-        const int x = b ^ ((i & 7) << 2);
-        pairs[i] = *reinterpret_cast<const pair_any*>(own_rows + (size_t)i * K + 2 * x);
-    }
-    uint32_t kept = 0;  // bit i + 16 h: element h of row i
+    for (int i = 0; i < kRowsPerThread; i++)
+        pairs[i] = *reinterpret_cast<const pair_any*>(rows + (size_t)i * K * 2 + (own_row + ((b << 2) ^ ((i & 7) << 4))));
+    uint32_t halves[2] = {0, 0};  // rows 0 .. 7, 8 .. 15: bit 2 (i % 8) + 16 h for element h of row i
 #pragma unroll
     for (int i = 0; i < kRowsPerThread; i++)
-        kept |= __builtin_bit_cast(uint32_t, kept_halves(pairs[i])) << i;
+        halves[i >> 3] |= __builtin_bit_cast(uint32_t, kept_halves(pairs[i])) << (2 * (i & 7));
+    const uint32_t kept = ((halves[0] | halves[0] >> 15) & 0xffffu) | (halves[1] | halves[1] >> 15) << 16;  // bit 2 i + h
     const int own = __popc(kept);
-    const uint32_t gone = ~kept;  // the first position in row order: the lower row, then the lower element
-    const int z0 = __ffs(static_cast<int>(gone & 0xffffu)) - 1, z1 = __ffs(static_cast<int>(gone >> 16)) - 1;
-    const int z = z0 >= 0 && (z1 < 0 || z0 <= z1) ? 2 * z0 : (z1 < 0 ? -1 : 2 * z1 + 1);
+    const int z = __ffs(static_cast<int>(~kept)) - 1;  // the first position in row order
     const int corner = rg * kRowsPerThread * kTileCols + 2 * b;  // position = row * 64 + swizzled column (:330-339)
     grp_count[rg][b] = own;
     grp_zero[rg][b] = z < 0 ? -1 : corner + (z >> 1) * kTileCols + (z & 1);
@@ -191,13 +196,18 @@ __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* _
     if (lo <= hi) {
         const int above = size - hi;
         int pops = __builtin_amdgcn_readlane(offscan::wave_inclusive_sum(lane < kBanks && above > 0 ? above : 0), 63);
-        for (int l = hi; l >= lo; l--) {
-            const uint32_t mask = static_cast<uint32_t>(__ballot(size >= l));
-            if (lane == 0)
-                levels[l] = u32x2{mask, static_cast<uint32_t>(pops)};
-            pops += __popc(mask);
+        const int upper = lane >> 5;  // the upper lanes' copies of the banks look at the level below
+        for (int l = hi; l >= lo; l -= 2) {  // (level lo - 1 may be written as well: the next wave's, with the same entry)
+            const uint64_t both = __ballot(size >= l - upper);
+            const uint32_t mask = static_cast<uint32_t>(both), mask_below = static_cast<uint32_t>(both >> 32);
+            const int pops_below = pops + __popc(mask);
+            if (b == 0)
+                levels[kMaxLevel - l + upper] = u32x2{upper ? mask_below : mask, static_cast<uint32_t>(upper ? pops_below : pops)};
+            pops = pops_below + __popc(mask_below);
         }
     }
+    if (threadIdx.x == 0)
+        levels[0] = u32x2{~0u, words <= kPassWords ? static_cast<uint32_t>(kSeqWords) : 1u << 30};
     __syncthreads();
 
     // 5. emission (:379-424): V vectors = R groups of 32 lanes + rem lanes.  The first 4 * rem pops
@@ -210,29 +220,32 @@ __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* _
     // The words of pops first .. last - 1 into the sequence.  Level entries are read sixteen at a time,
     // ahead of the writes that depend on them: one by one, every element pays a trip to LDS.
     auto place_words = [&](int first, int last, auto all) __attribute__((always_inline)) {
-        auto slot = [&](u32x2 e, bool used) {
-            const int pop = static_cast<int>(e[1]) + __popc(e[0] & below);
-            if constexpr (decltype(all)::value)  // the tile's words fit one pass
-                return used ? pop : dump;
-            return used && pop >= first && pop < last ? pop - first : dump;
+        auto place = [&](u32x2 e, uint32_t word) __attribute__((always_inline)) {
+            int pop = static_cast<int>(e[1]) + __popc(e[0] & below);
+            if constexpr (!decltype(all)::value)  // else the tile's words fit one pass
+                pop = pop >= first && pop < last ? pop - first : dump;
+            seq[pop] = word;
         };
-        int level = rank, at = corner;
-        uint32_t live = kept;
+        const uint8_t* const entries = reinterpret_cast<const uint8_t*>(levels);
+        int entry = (kMaxLevel - rank) * 8;  // the byte of the level below the next kept element's
+        uint32_t at = static_cast<uint32_t>(corner) << 16, live = kept;
         // (opaque: or the compiler prepares all 32 words and places ahead of both ways, and spills)
-        asm volatile("" : "+v"(level), "+v"(at), "+v"(live));
+        asm volatile("" : "+v"(entry), "+v"(at), "+v"(live));
 #pragma unroll
         for (int i0 = 0; i0 < kRowsPerThread; i0 += 8) {
             u32x2 e[16];
 #pragma unroll
             for (int j = 0; j < 16; j++) {
-                level += (live >> (i0 + j / 2 + 16 * (j & 1))) & 1;
-                e[j] = levels[level];
+                const int used = static_cast<int>(live << (31 - 2 * i0 - j)) >> 31;  // 0 or -1
+                entry += used << 3;
+                asm("" : "+v"(entry));  // (or the compiler sums `used` up on the side)
+                e[j] = *reinterpret_cast<const u32x2*>(entries + (entry & used));
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int j = 0; j < 16; j++) {
-                const uint32_t pair = pairs[i0 + j / 2], position = at + (i0 + j / 2) * kTileCols + (j & 1);
-                seq[slot(e[j], (live >> (i0 + j / 2 + 16 * (j & 1))) & 1)] = (j & 1 ? pair >> 16 : pair & 0xffffu) | position << 16;
+                const uint32_t pair = pairs[i0 + j / 2], position = at + (((i0 + j / 2) * kTileCols + (j & 1)) << 16);
+                place(e[j], (j & 1 ? pair >> 16 : pair & 0xffffu) | position);
             }
         }
         if (rg == 0 && size > real) {  // the pads, behind the bank's last element
@@ -240,7 +253,7 @@ __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* _
             for (int g = 0; g < kRowGroups && p < 0; g++)
                 p = grp_zero[g][b];
             for (int l = real + 1; l <= size; l++)
-                seq[slot(levels[l], true)] = static_cast<uint32_t>(p) << 16;
+                place(levels[kMaxLevel - l], static_cast<uint32_t>(p) << 16);
         }
     };
     // groups of 32 vectors out of the sequence, whose word `from` is the first of their 128 pops
@@ -251,7 +264,7 @@ __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* _
 #pragma unroll
             for (int s = 0; s < 4; s++)
                 v[s] = seq[at + (3 - s) * 32];
-            out[(R - 1 - done - g) * 32 + (i & 31)] = v;
+            __builtin_nontemporal_store(v, out + ((R - 1 - done - g) * 32 + (i & 31)));
         }
     };
     auto write_tail = [&]() __attribute__((always_inline)) {

@@ -218,3 +218,27 @@ def test_device_encoder_with_offsets_of_another_matrix(spmm):
     keep = np.repeat((kind.view(-1) > 1).cpu().numpy(), 4 * np.diff(offsets.cpu().numpy()[:-1]))
     want, got = items.cpu().numpy(), out.cpu().numpy()
     assert np.array_equal(got[:total], np.where(keep, want, mark)) and (got[total:] == mark).all()
+
+
+@pytest.mark.parametrize("heights", ["one", "few", "full", "staggered"])
+@pytest.mark.parametrize("extra", [0, 1, 2, 3])
+def test_device_encoder_uneven_banks(spmm, oracle, heights, extra):
+    """Levels: tiles whose words lie in one bank (256 of them: the tallest there is, with pads on the empty banks),
+    in a few, all full, and 32 different heights of odd and even distances, with 0 to 3 words more for the pads; NaN and
+    signed zeros (not kept) everywhere else."""
+    rng = np.random.default_rng(extra)
+    M, K = 256, 64 * 5
+    want = {"one": [256] + [0] * 31, "few": [0, 0, 255, 0, 1, 128] + [0] * 25 + [2], "full": [256] * 32,
+            "staggered": [(7 * b * b) % 257 for b in range(32)]}[heights]
+    column = ((np.arange(64) ^ ((np.arange(128)[:, None] & 7) << 3)) >> 1)  # the bank of (row, column)
+    A = np.where(rng.random((M, K)) < 0.5, 0x8000, 0x7E01).astype(np.uint16)
+    for r in range(0, M, 128):
+        for c in range(0, K, 64):
+            tile = np.ascontiguousarray(A[r:r + 128, c:c + 64])
+            order = rng.permutation(32)
+            for b in range(32):
+                at = np.flatnonzero(column.ravel() == order[b])
+                n = min(want[b] + (extra if b == 4 else 0), 256)
+                tile.ravel()[rng.choice(at, size=n, replace=False)] = rng.choice([0x0001, 0x8001, 0x7C00, 0xFC00, 0x3C00], size=n)
+            A[r:r + 128, c:c + 64] = tile
+    _compare(spmm, oracle, A.view(np.float16))
