@@ -147,6 +147,12 @@ __device__ __forceinline__ half8 load_activations(const _Float16* p)
     return r;
 }
 
+// 16 bytes per lane from base + voff straight into LDS, lane l's at lds + 16 l; counts like any load.
+__device__ __forceinline__ void load_to_lds(const uint8_t* base, uint32_t voff, uint32_t lds)
+{
+    asm volatile("s_mov_b32 m0, %0\n s_nop 0\n global_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "m0", "memory");
+}
+
 // One tile offset per lane, asynchronous like the loads above (to be waited for by hand).
 __device__ __forceinline__ int load_offset(const int* p)
 {
@@ -1128,6 +1134,348 @@ __global__ __launch_bounds__(2 * kWave, 2) void tcsl_spmm_pair_kernel(const int*
     }
 }
 
+// 64 tokens, ROWS tile rows to a workgroup and two waves to each: a wave takes all 128 rows and all tokens of one half of the
+// batch's tiles, and the two sums meet in LDS at the end.
+//
+// What bounds 64 tokens in the first kernel is the instruction issue of one wave to a SIMD (1744 of 2953 cycles a tile: 74 LDS
+// instructions, 64 MFMAs, the rest) with nothing beside it, and the activation fragments, a quarter of a line per lane and
+// load (512 of 614 accesses to the vector L1 a tile).  Multiplying a tile between the scatter instructions of the next one, in
+// one wave, gained nothing for the first reason (49152 x 12288 131 -> 142 us).  Two waves fit a SIMD at 256 registers: one set
+// of words, fetched while the tile before it is multiplied, instead of a ring of two; no fragments in flight, because the ROWS
+// waves of a half share each activation tile through LDS, where it goes straight from memory in whole lines; and no addresses
+// kept to undo the scatter, except for small tiles: larger ones are cleared in whole lines.
+//
+// A barrier per kTiles tiles: in front of it each wave has waited for its share of the activations that its half reads next,
+// behind it nobody reads the ones before, and the next are fetched into their place.  Two tiles between barriers, where LDS has
+// the room, let the waves' memory latencies even out (126 -> 120 us).  Every wave of the workgroup takes the same number of steps;
+// an empty tile (or one past a half's end) is not multiplied.
+// Measured, and where it is used: tcsl_launch_spmm.  The images are ROWS * 32 KiB of LDS, the activations kTiles * 32 KiB.
+constexpr int halves_tiles(int rows)  // tiles between two barriers
+{
+    return rows < 4 ? 2 : 1;
+}
+template<int ROWS, bool ROWMAJ>
+__global__ __launch_bounds__(2 * ROWS * kWave) void tcsl_spmm_halves_kernel(const int* __restrict__ offsets,
+                                                                           const u32x4* __restrict__ items,
+                                                                           const _Float16* __restrict__ B,
+                                                                           _Float16* __restrict__ out, int K, int avg, int ldb,
+                                                                           int M, int ldo, int relu)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    constexpr int NB = 4, NTOK = 16 * NB, rows = ROWS;
+    constexpr int kTiles = halves_tiles(ROWS), kBufs = 2 * kTiles, kTokenBytes = NTOK * 128;
+    constexpr int BL = (kTokenBytes / 1024 + ROWS - 1) / ROWS;  // activation loads of a wave per tile, a KiB each
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int half = wave >= rows ? 1 : 0;
+    const int rt = blockIdx.x * rows + wave - (half ? rows : 0), batch = blockIdx.y;
+    const bool active = rt < M / kTileRows;
+    const int nkb = K / kTileCols;
+    int kb0 = batch * avg;
+    kb0 = kb0 < nkb ? kb0 : nkb;
+    int kb1 = kb0 + avg;
+    kb1 = kb1 < nkb ? kb1 : nkb;
+    const int steps = (kb1 - kb0 + 1) / 2;  // of every wave: the second half may have a tile less
+    const int middle = kb0 + steps;
+    if (half)
+        kb0 = middle;
+    else
+        kb1 = middle;
+    const int ntile = kb1 - kb0;
+    uint8_t* const tile = lds + wave * kTileBytes;
+    const int* const toff = offsets + (size_t)(active ? rt : 0) * nkb + kb0;
+    int wbase = 0;
+    int wreg = !active ? 0 : toff[lane <= ntile ? lane : ntile];  // lane l: first vector of tile wbase + l
+    for (int i = 0; i < kTileBytes / (kWave * 16); i++)
+        *reinterpret_cast<u32x4*>(tile + (i * kWave + lane) * 16) = u32x4{0u, 0u, 0u, 0u};
+
+    auto tile_range = [&](int i, int& begin, int& end) __attribute__((always_inline)) {  // 0 <= i < ntile
+        if (i + 1 - wbase >= kWave) {  // (more than 63 tiles per wave only)
+            wbase = i;
+            const int idx = i + lane;
+            wreg = active ? toff[idx <= ntile ? idx : ntile] : 0;
+            settle(wreg);
+        }
+        begin = __builtin_amdgcn_readlane(wreg, i - wbase);
+        end = __builtin_amdgcn_readlane(wreg, i + 1 - wbase);
+    };
+
+    f32x4 acc[NB][8];
+#pragma unroll
+    for (int c = 0; c < NB; c++)
+#pragma unroll
+        for (int r = 0; r < 8; r++)
+            acc[c][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int l15 = lane & 15, q = lane >> 4;
+    int a_off[2];
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+        a_off[s] = l15 * 128 + (((s * 4 + q) ^ (lane & 7)) << 4);
+    // This wave's loads of its half's activation tiles: eight tokens' 128-byte lines each (row-major: a KiB of the tile's
+    // contiguous block), in the order that the granules have in LDS; the same order of granules as the weight tile's
+    // (row-major: the 32-byte column chunks of row k permuted by (k >> 1) & 3, for the transposing reads).
+    const uint32_t from_lane = ROWMAJ ? (lane ^ ((lane >> 4) << 1)) * 16
+                                      : (lane >> 3) * (uint32_t)ldb * 2 + (((lane & 7) ^ (lane >> 3)) << 4);
+    uint8_t* const tokens = lds + 2 * ROWS * kTileBytes + half * kBufs * kTokenBytes;
+    const uint32_t tokens_at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(tokens)));
+    const int first_piece = (wave - half * ROWS) * BL;
+    auto issue_activations = [&](int t, int buf) __attribute__((always_inline)) {
+        const int bt = kb0 + (t < ntile ? t : (ntile > 0 ? ntile - 1 : 0));  // (a half without tiles: its neighbour's)
+        const uint8_t* const from = reinterpret_cast<const uint8_t*>(B) + (size_t)(bt < nkb ? bt : nkb - 1) * (ROWMAJ ? kTokenBytes : kTileCols * 2);
+#pragma unroll
+        for (int i = 0; i < BL; i++) {
+            const int piece = first_piece + i < kTokenBytes / 1024 ? first_piece + i : kTokenBytes / 1024 - 1;
+            load_to_lds(from + piece * (ROWMAJ ? (size_t)1024 : (size_t)ldb * 16), from_lane, tokens_at + buf * kTokenBytes + piece * 1024);
+        }
+    };
+    int b_off[2][2];  // where the fragments of token block 0 lie, by k step (row-major: [.][0], [.][1]: see below)
+    if constexpr (ROWMAJ) {
+        // (lane of a group of sixteen: row 4 h + l15 / 4 of the eight, columns 4 (l15 % 4) .. + 3; the chunk of block c is
+        // c ^ (2 h + l15 / 8), whose upper bit is a constant and whose lower one is l15 / 8 for even c, its complement for odd)
+        const int base = (8 * q + (l15 >> 2)) * 128 + (l15 & 3) * 8;
+        b_off[0][0] = base + 32 * (l15 >> 3);
+        b_off[0][1] = base + 32 - 32 * (l15 >> 3);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+            b_off[k][0] = l15 * 128 + (((k * 4 + q) ^ (l15 & 7)) << 4);
+    }
+    auto read_b = [&](const uint8_t* from, int k, int c) __attribute__((always_inline)) {
+        if constexpr (ROWMAJ) {
+            typedef short short4v __attribute__((ext_vector_type(4)));
+            typedef short short8v __attribute__((ext_vector_type(8)));
+            typedef __attribute__((address_space(3))) short4v lds_short4v;
+            const uint8_t* const at = from + b_off[0][c & 1] + k * 4096;
+            const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4v*)(at + 64 * (c >> 1)));
+            const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4v*)(at + 512 + 64 * ((c >> 1) ^ 1)));
+            const short8v both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            return __builtin_bit_cast(half8, both);
+        } else {
+            return *reinterpret_cast<const half8*>(from + b_off[k][0] + c * 2048);
+        }
+    };
+    const int voff_lo = lane * 16, voff_hi = lane * 16 + 4096, voff_top = lane * 16 + 8192;
+    uint32_t vzero = 0, vtwo = 2, vbase = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(tile));
+    asm volatile("" : "+v"(vzero), "+v"(vtwo), "+v"(vbase));
+
+    auto stream_run = [&](auto vpl_c) __attribute__((always_inline)) {
+        constexpr int VPL = decltype(vpl_c)::value;
+        constexpr int kSeg = VPL * kWave;
+        struct Seg {
+            int tile;     // index within the run; ntile = past the end
+            int begin;    // first vector, absolute
+            int n;        // vectors in this segment
+            bool last;    // last segment of its tile
+        };
+        struct Cur {
+            int tile, off;
+        };
+        auto make_seg = [&](Cur c, Seg& s, Cur& nxt) __attribute__((always_inline)) {
+            if (c.tile >= ntile) {
+                s = Seg{ntile, 0, 0, true};
+                nxt = c;
+                return;
+            }
+            int b, e;
+            tile_range(c.tile, b, e);
+            const int rest = e - b - c.off;
+            s.tile = c.tile;
+            s.begin = b + c.off;
+            s.n = rest < kSeg ? rest : kSeg;
+            s.last = rest <= kSeg;
+            nxt = s.last ? Cur{c.tile + 1, 0} : Cur{c.tile, c.off + kSeg};
+        };
+        u32x4 regs[VPL];
+        auto issue_words = [&](const Seg& s) __attribute__((always_inline)) {
+            const uint64_t base = reinterpret_cast<uint64_t>(items + s.begin);
+            i32x4 rs = {(int)(uint32_t)base, (int)((uint32_t)(base >> 32) & 0xffff), s.n * 16, 0x00020000};
+            static_for<VPL>([&](auto uc) {
+                constexpr int u = decltype(uc)::value;
+                if constexpr (u < 4)
+                    regs[u] = load_words<u * 1024>(rs, voff_lo);
+                else if constexpr (u < 8)
+                    regs[u] = load_words<(u - 4) * 1024>(rs, voff_hi);
+                else
+                    regs[u] = load_words<(u - 8) * 1024>(rs, voff_top);
+            });
+        };
+        // Small tiles are undone word by word, larger ones cleared in whole lines (16 writes, and no registers for the addresses).
+        constexpr bool kUndo = VPL <= kVecPerLaneShort;
+        uint32_t kept[kUndo ? VPL : 1][4];
+        // op(u) for every vector u of this lane's that a segment of n vectors holds (see the kernel above)
+        auto by_chunks = [&](int n, auto&& op) __attribute__((always_inline)) {
+            const int full = n >> 6;
+            const bool in_part = (full << 6) + lane < n;
+            bool done = false;
+            static_for<VPL + 1>([&](auto pc) {
+                constexpr int P = decltype(pc)::value;
+                if (!done && full == P) {
+                    static_for<P>([&](auto uc) { op(uc); });
+                    if constexpr (P < VPL) {
+                        if (in_part)
+                            op(pc);
+                    }
+                    done = true;
+                }
+            });
+        };
+        Seg s;
+        Cur next{0, 0};
+        make_seg(next, s, next);
+        if constexpr (kTiles == 1)
+            issue_words(s);
+        static_for<kTiles>([&](auto j) { issue_activations(decltype(j)::value, decltype(j)::value); });
+        if constexpr (kTiles > 1)
+            issue_words(s);
+        int buf = 0;
+        for (int t = 0; t < steps; t += kTiles) {
+            static_for<kTiles>([&](auto j_c) __attribute__((always_inline)) {
+                constexpr int j = decltype(j_c)::value;
+                // this step's words into the image; the first segment of the next tile on its way
+                wait_loads<kTiles == 1 ? BL : j * kTiles * BL>();
+                static_for<VPL>([&](auto uc) { pin(regs[decltype(uc)::value]); });
+                const bool whole = s.last;  // the tile is one segment
+                const int held = s.n;       // ... of so many vectors
+                for (;;) {
+                    by_chunks(s.n, [&](auto uc) {
+                        constexpr int u = decltype(uc)::value;
+                        scatter_words_keep(regs[u], vbase, vtwo, kept[kUndo ? u : 0]);
+                    });
+                    if (s.last)
+                        break;
+                    make_seg(next, s, next);  // further segments of the tile, one after the other
+                    issue_words(s);
+                    wait_loads<0>();
+                    static_for<VPL>([&](auto uc) { pin(regs[decltype(uc)::value]); });
+                }
+                make_seg(next, s, next);
+                issue_words(s);
+                if constexpr (j == 0) {
+                    // Behind the barrier every wave's share of the activations is there that the next kTiles steps read, and nobody
+                    // reads the other buffers any more.
+                    if constexpr (kTiles == 1)
+                        wait_loads<VPL>();
+                    __syncthreads();
+                    static_for<kTiles>([&](auto i) { issue_activations(t + kTiles + decltype(i)::value, (buf ^ kTiles) + decltype(i)::value); });
+                }
+                if (held == 0)
+                    return;  // an empty tile
+                const uint8_t* const from = tokens + (buf + j) * kTokenBytes;
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    half8 afrag[8], bf[NB];
+#pragma unroll
+                    for (int c = 0; c < NB; c++)
+                        bf[c] = read_b(from, k, c);
+#pragma unroll
+                    for (int r = 0; r < 8; r++)
+                        afrag[r] = *reinterpret_cast<const half8*>(tile + a_off[k] + r * 2048);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (k == 1) {
+                        bool cleared = false;
+                        if constexpr (kUndo) {
+                            if (whole) {
+                                by_chunks(held, [&](auto uc) { clear_words(kept[decltype(uc)::value], vzero); });
+                                cleared = true;
+                            }
+                        }
+                        if (!cleared) {
+#pragma unroll
+                            for (int i = 0; i < kTileBytes / (kWave * 16); i++)
+                                *reinterpret_cast<u32x4*>(tile + (i * kWave + lane) * 16) = u32x4{0u, 0u, 0u, 0u};
+                        }
+                    }
+#pragma unroll
+                    for (int r = 0; r < 8; r++)
+#pragma unroll
+                        for (int cb = 0; cb < NB; cb++)
+                            acc[cb][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag[r], bf[cb], acc[cb][r], 0, 0, 0);
+                }
+            });
+            buf ^= kTiles;
+        }
+        wait_loads<0>();
+        static_for<VPL>([&](auto uc) { pin(regs[decltype(uc)::value]); });
+    };
+    if (steps > 0) {
+        const int nw = ntile < kWave - 1 ? ntile : kWave - 1;
+        const int segments = segment_choice(__builtin_amdgcn_readlane(wreg, nw) - __builtin_amdgcn_readlane(wreg, 0), nw);
+        if (segments == 3)
+            stream_run(std::integral_constant<int, kVecPerLaneLong>{});
+        else if (segments == 1)
+            stream_run(std::integral_constant<int, kVecPerLaneShort>{});
+        else if (segments == 0)
+            stream_run(std::integral_constant<int, kVecPerLaneTiny>{});
+        else
+            stream_run(std::integral_constant<int, kVecPerLane>{});
+    }
+
+    // The two halves' sums meet: each wave hands its partner two of the four column blocks through its own image, and
+    // finishes the other two.
+    const int partner = half ? wave - rows : wave + rows;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    f32x4* const park = reinterpret_cast<f32x4*>(tile) + lane;
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int r = 0; r < 8; r++)
+            park[(c * 8 + r) * kWave] = half ? acc[c][r] : acc[c + 2][r];
+    __syncthreads();
+    uint8_t* const stage = lds + partner * kTileBytes;  // the partner's image: read by this wave alone
+    f32x4 sum[2][8];
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            const f32x4 other = reinterpret_cast<const f32x4*>(stage)[(c * 8 + r) * kWave + lane];
+            const f32x4 mine = half ? acc[c + 2][r] : acc[c][r];
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                sum[c][r][i] = half ? other[i] + mine[i] : mine[i] + other[i];
+        }
+    if (!active)
+        return;
+    _Float16* const oslab = out + (size_t)batch * M * NTOK + (size_t)rt * kTileRows * (ROWMAJ ? NTOK : 1);
+    if constexpr (ROWMAJ) {  // 32 tokens of each row: [row][32], 64 bytes a row
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int r = 0; r < 8; r++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    *reinterpret_cast<_Float16*>(stage + (r * 16 + q * 4 + i) * 64 + (c * 16 + l15) * 2) =
+                        static_cast<_Float16>(relu ? fmaxf(sum[c][r][i], 0.f) : sum[c][r][i]);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < kTileRows * 64 / (kWave * 16); i++) {
+            const int e = i * kWave + lane;
+            *reinterpret_cast<half8*>(oslab + (size_t)(e >> 2) * NTOK + half * 32 + (e & 3) * 8) = *reinterpret_cast<const half8*>(stage + e * 16);
+        }
+        return;
+    }
+    constexpr int kTokStride = 272;
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            half4 h;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                h[i] = static_cast<_Float16>(relu ? fmaxf(sum[c][r][i], 0.f) : sum[c][r][i]);
+            *reinterpret_cast<half4*>(stage + l15 * kTokStride + (r * 16 + q * 4) * 2) = h;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int e = i * kWave + lane, tok = e >> 4, part = e & 15;
+            const half8 v = *reinterpret_cast<const half8*>(stage + tok * kTokStride + part * 16);
+            *reinterpret_cast<half8*>(oslab + (size_t)((half * 2 + c) * 16 + tok) * ldo + part * 8) = v;
+        }
+    }
+}
+
 // sum += slabs s .. s + COUNT - 1, in slab order.  TOGETHER: every load is issued before the first one is waited
 // for; else the compiler has eight or so in flight, and adds up what has come meanwhile.
 template<int COUNT, bool TOGETHER>
@@ -1270,6 +1618,32 @@ int launch_spmm(hipStream_t stream, const void* items, const int* offsets, const
     return static_cast<int>(hipGetLastError());
 }
 
+template<int ROWS, bool ROWMAJ>
+int launch_halves(hipStream_t stream, const void* items, const int* offsets, const void* B, void* out, int M, int K, int split_k, int ldb,
+                  int ldo, int relu)
+{
+    constexpr unsigned kLds = 2 * ROWS * kTileBytes + 2 * 2 * halves_tiles(ROWS) * 64 * 128;
+    static_assert(kLds <= kMaxLdsBytes, "the images and both halves' activation tiles");
+    if (split_k > 65535)
+        return static_cast<int>(hipErrorInvalidValue);
+    auto kernel = tcsl_spmm_halves_kernel<ROWS, ROWMAJ>;
+    static std::atomic<int> armed_device{-1};
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess)
+        return static_cast<int>(e);
+    if (armed_device.load(std::memory_order_acquire) != dev) {
+        e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLdsBytes);
+        if (e != hipSuccess)
+            return static_cast<int>(e);
+        armed_device.store(dev, std::memory_order_release);
+    }
+    hipLaunchKernelGGL(kernel, dim3((M / kTileRows + ROWS - 1) / ROWS, split_k), dim3(2 * ROWS * kWave), kLds, stream, offsets,
+                       static_cast<const u32x4*>(items), static_cast<const _Float16*>(B), static_cast<_Float16*>(out), K,
+                       (K / kTileCols - 1) / split_k + 1, ldb, M, ldo, relu);
+    return static_cast<int>(hipGetLastError());
+}
+
 int launch_pair(hipStream_t stream, const void* items, const int* offsets, const void* B, void* out, int M, int K, int split_k,
                 int ldb, int ldo, int relu)
 {
@@ -1354,6 +1728,21 @@ extern "C" int tcsl_launch_spmm(void* stream, const void* items, const int* offs
         case 64:
             if (stage_b == 2)
                 return TCSL_GO(4, false, false, false, false, 4, 4);
+            // Two waves to a tile row (tcsl_spmm_halves_kernel) where the row-sharing layout has three or four tile rows to a
+            // workgroup and a batch is long enough to pay for the second barrier and the sum of the halves.  Measured on 60
+            // calls, the other kernel -> this one: three rows, column-major, 1.02 to 1.16 times as fast from four tiles a batch
+            // on (49152 x 12288 at 80 % 130 -> 119 us, at 60 % 216 -> 177, at 90 % 106 -> 92; 0.97 to 0.99 with one or two
+            // tiles), row-major 1.05 to 1.4 (149 -> 119, 219 -> 175, 129 -> 93); four rows, row-major, 1.01 to 1.33 from 20 tiles
+            // on (36864 x 9216 in three batches 82 -> 74), 0.97 to 1.08 below; four rows, column-major, 0.98 to 1.04 at 60 to
+            // 80 %: left to the other kernel.  (The activations go straight into LDS: aligned, and 32-bit offsets of eight tokens.)
+            if (const int tiles = (K / kTileCols - 1) / split_k + 1;
+                mode == 0 && (waves == 3 ? tiles >= 4 : waves == 4 && row_major && tiles >= 20) &&
+                (reinterpret_cast<uintptr_t>(B) & 15) == 0 && (row_major || (ldb % 8 == 0 && ldb <= 1 << 28))) {
+                if (waves == 4)
+                    return launch_halves<4, true>(s, items, offsets, B, out, M, K, split_k, ldb, ldo, relu);
+                return row_major ? launch_halves<3, true>(s, items, offsets, B, out, M, K, split_k, ldb, ldo, relu)
+                                 : launch_halves<3, false>(s, items, offsets, B, out, M, K, split_k, ldb, ldo, relu);
+            }
             return TCSL_PICK(4, false, 4);
         default:
             return static_cast<int>(hipErrorInvalidValue);

@@ -1138,3 +1138,62 @@ def test_reduction_kernel_adds_slabs_of_large_outputs(spmm, split_k):
     got = d_C.cpu()
     assert torch.isfinite(want).all() and torch.equal(got[:, :M], want.half())
     assert torch.isnan(got[:, M:].float()).all()
+
+
+@pytest.mark.parametrize("M,K,split_k,sparsity,flags", [
+    (384, 64 * 4, 1, 0.8, 0),            # two tiles for each half
+    (128, 64 * 5, 1, 0.8, 1),            # one tile row of a workgroup's, halves of three tiles and two, clamped by the kernel
+    (640, 64 * 29, 3, 0.7, 1),           # rows 4 and 5 of three, batches of 10, 10 and 9 tiles, clamped by the reduction
+    (512, 64 * 22, 5, 0.0, 0),           # dense tiles: two segments of ten vectors a lane; batches of 5, 5, 5, 5, 2
+    (768, 64 * 21, 1, 0.5, 0),           # ... of eight and ten
+    (896, 64 * 40, 2, 0.97, 0),          # tiles of a few vectors, undone word by word
+    (384, 64 * 131, 1, 0.9, 0),          # more tiles for each half than one window of offsets has
+    (1152, 64 * 24, 1, "mixed", 0),      # tile rows of every density side by side, empty tiles among them
+    (128 * 385, 64 * 5, 1, 0.85, 0),     # more units than run at once
+])
+@pytest.mark.parametrize("row_major", [0, 1])
+@pytest.mark.parametrize("waves", [3, 4])
+def test_two_waves_per_tile_row_at_64_tokens(spmm, oracle, M, K, split_k, sparsity, flags, row_major, waves):
+    """The row-sharing layout at 64 tokens with two waves to each tile row where its rule takes it (and the one-wave kernel
+    beside it): against the oracle, and against the same launch with activations that begin at an odd element,
+    which the one-wave kernel takes; a tile without words hides what the activations hold there."""
+    torch = _torch()
+    N, dev = 64, torch.device("cuda:0")
+    if sparsity == "mixed":
+        A = spmm.synth_weights(M, K, 0.0, False, seed=M)
+        rng = np.random.default_rng(5)
+        density = rng.permutation(np.linspace(0.0, 0.6, M // 128 * (K // 64))).reshape(M // 128, K // 64)
+        density[:, 7] = 0.0
+        A[rng.random((M, K), dtype=np.float32) >= density.repeat(128, 0).repeat(64, 1).astype(np.float32)] = 0
+    else:
+        A = spmm.synth_weights(M, K, sparsity, False, seed=M + K)
+    B = spmm.synth_activations(N, K, seed=9)
+    ref = oracle.gemm_f32(A, B)
+    if sparsity == "mixed":  # in columns that no tile row has words for
+        B = B.copy()
+        B[3, 7 * 64 + 5] = np.inf
+        B[60, 7 * 64 + 63] = np.nan
+    if flags & 1:
+        ref = np.maximum(ref, 0)
+    items, offsets = spmm.InitSparseMatrixA_API(A)
+    d_items = torch.from_numpy(items.view(np.int32).copy()).to(dev)
+    d_offs = torch.from_numpy(offsets.copy()).to(dev)
+    d_W = torch.full((split_k, N * M), float("nan"), dtype=torch.float16, device=dev)
+    d_B = torch.from_numpy(np.ascontiguousarray(B).view(np.int16).copy()).to(dev).view(torch.float16)
+    if row_major:
+        d_B = d_B.t().contiguous()
+    odd = torch.empty(N * K + 8, dtype=torch.float16, device=dev)[1:1 + N * K].view(d_B.shape)
+    odd.copy_(d_B)
+    print(f"[gpu case] halves M={M} K={K} split_k={split_k} sparsity={sparsity} flags={flags} row_major={row_major} waves={waves}", flush=True)
+    got = []
+    for b in (d_B, odd):
+        C = torch.full((M, N) if row_major else (N, M), float("nan"), dtype=torch.float16, device=dev)
+        spmm.SpMM_SplitK_API_Planned(torch.cuda.current_stream(), d_items, d_offs, b, C, M, N, K, d_W, split_k, 0, waves, 0, row_major, flags)
+        torch.cuda.synchronize()
+        got.append((C.t() if row_major else C).cpu().numpy())
+        assert_close(got[-1], ref)
+    # the two differ in the order of fp32 sums, in one rounding of a slab and one of the result: two units in the last place of
+    # what a slab can be
+    size = np.abs(A.astype(np.float32))
+    bound = 2.0 ** -10 * (np.abs(np.nan_to_num(B.astype(np.float32), posinf=0.0)) @ size.T) + 2.0 ** -24
+    assert (np.abs(got[0].astype(np.float32) - got[1].astype(np.float32)) <= bound).all()
