@@ -104,11 +104,12 @@ void* allocate_words(void* user, size_t bytes)
     return *room;
 }
 
+constexpr int kLevels = kTileRows * kTileCols / kBanks + kVec;  // 256 positions per bank + pads
 struct TileScratch {
-    uint32_t bank[kBanks][kTileRows * kTileCols / kBanks + kVec];  // 256 positions per bank + pads
+    uint32_t words[kLevels * kBanks];  // a bank's element number l in row kLevels - 1 - l: levels upwards run backwards
+    uint32_t next[kBanks];             // where each bank's next element goes
     int16_t size[kBanks];
-    uint64_t row[kTileRows];              // kept_mask of every row
-    uint32_t seq[kTileRows * kTileCols + kVec];  // pop sequence
+    uint64_t row[kTileRows];           // kept_mask of every row
 };
 
 // First position of bank b that is not kept, in row order; -1: none.
@@ -125,15 +126,17 @@ int first_zero_of(const TileScratch& ws, int b)
 
 // Encodes one tile into dst; returns the number of words written (a multiple of 4).
 //
-// Bound by the instructions per kept element (two: into its bank's list, and out of it), so rows are
-// tested 16 elements at a time and only set bits are visited, and the emission order's groups of
-// 32 x 4 words are transposed 4 x 4 words at a time.  (7168 x 7168 at 80 % on 16 threads, the whole call
-// from Python with no copy of the words: 3.1 ms; element by element, in two sets of threads, with
-// the copy: 15.1.)
+// Bound by the instructions per kept element, so rows are tested 16 elements at a time and only set bits are
+// visited; the banks' elements lie level by level, the first level last, so that the levels that all banks
+// reach are the pop sequence as they lie (37 of some 66 levels at 80 %, most of the words) and only those above
+// them are moved together; and the emission order's groups of 32 x 4 words are transposed 4 x 4 words at a time.
+// (7168 x 7168 on 16 threads, the whole call from Python with no copy of the words: 2.4 ms at 80 %, 3.1 at 60 %; with a
+// list per bank, every word moved into the pop sequence: 2.9 and 4.2; element by element, in two sets of
+// threads, with the copy: 15.1 at 80 %.)
 int emit_tile(const uint16_t* tile, int ld, uint32_t* dst, TileScratch& ws)
 {
     for (int b = 0; b < kBanks; b++)
-        ws.size[b] = 0;
+        ws.next[b] = (kLevels - 1) * kBanks + b;
     int count = 0;
     for (int m = 0; m < kTileRows; m++) {
         const uint16_t* row = tile + static_cast<size_t>(m) * ld;
@@ -147,11 +150,15 @@ int emit_tile(const uint16_t* tile, int ld, uint32_t* dst, TileScratch& ws)
             const int n = __builtin_ctzll(rest);
             const int swz = n ^ flip;  // swizzled column (csrc/SpMM_API.cu:332-333)
             const int b = swz >> 1;    // 4-byte LDS bank of that position (:334)
-            ws.bank[b][ws.size[b]++] = pack_item(row[n], m * kTileCols + swz);
+            const uint32_t at = ws.next[b];
+            ws.next[b] = at - kBanks;
+            ws.words[at] = pack_item(row[n], m * kTileCols + swz);
         }
     }
     if (count == 0)
         return 0;
+    for (int b = 0; b < kBanks; b++)
+        ws.size[b] = static_cast<int16_t>(kLevels - 1 - static_cast<int>(ws.next[b] / kBanks));
     // zero padding to a multiple of 4, each pad on the currently smallest bank (:352-365)
     const int pad = (kVec - count % kVec) % kVec;
     for (int p = 0; p < pad; p++) {
@@ -160,22 +167,31 @@ int emit_tile(const uint16_t* tile, int ld, uint32_t* dst, TileScratch& ws)
             if (ws.size[i] < ws.size[b])
                 b = i;
         // the smallest bank of a tile that needs padding always has a zero position
-        ws.bank[b][ws.size[b]++] = pack_item(0, first_zero_of(ws, b));
+        ws.words[ws.next[b]] = pack_item(0, first_zero_of(ws, b));
+        ws.next[b] -= kBanks;
+        ws.size[b]++;
         count++;
     }
-    // pop sequence, closed form
-    int top = 0;
-    for (int b = 0; b < kBanks; b++)
+    // pop sequence, closed form: levels from the tallest down, banks in order.  The levels above the smallest bank's
+    // are moved up against those below, from the lowest one on: a word never moves over one that is still to move.
+    int top = 0, full = kLevels;
+    for (int b = 0; b < kBanks; b++) {
         top = std::max<int>(top, ws.size[b]);
-    uint32_t* next = ws.seq;
+        full = std::min<int>(full, ws.size[b]);
+    }
+    uint32_t* seq = ws.words + (kLevels - full) * kBanks;
     const __m128i* const sizes = reinterpret_cast<const __m128i*>(ws.size);
-    for (int level = top; level >= 1; level--) {
+    for (int level = full + 1; level <= top; level++) {
         const __m128i under = _mm_set1_epi16(static_cast<short>(level - 1));
         auto taller = [&](int i) { return _mm_cmpgt_epi16(_mm_loadu_si128(sizes + i), under); };
         uint32_t banks = static_cast<uint32_t>(_mm_movemask_epi8(_mm_packs_epi16(taller(0), taller(1))))
                          | static_cast<uint32_t>(_mm_movemask_epi8(_mm_packs_epi16(taller(2), taller(3)))) << 16;
-        for (; banks; banks &= banks - 1)
-            *next++ = ws.bank[__builtin_ctz(banks)][level - 1];
+        const uint32_t* const from = ws.words + (kLevels - level) * kBanks;
+        while (banks) {  // from the last bank on
+            const int b = 31 - __builtin_clz(banks);
+            *--seq = from[b];
+            banks ^= 1u << b;
+        }
     }
     // emission (:379-424).  V vectors = R full groups of 32 lanes + `rem` lanes.
     // The first 4*rem pops fill the tail, lane b receiving pops v*rem + b; the
@@ -183,7 +199,7 @@ int emit_tile(const uint16_t* tile, int ld, uint32_t* dst, TileScratch& ws)
     // Both are written out in reverse arrival order, main part first.
     const int vecs = count / kVec;
     const int R = vecs / kGroup, rem = vecs % kGroup;
-    const uint32_t* mainq = ws.seq + kVec * rem;
+    const uint32_t* mainq = seq + kVec * rem;
     for (int r = 0; r < R; r++) {
         const uint32_t* const group = mainq + (kVec * (R - r) - kVec) * kGroup;  // arrivals k = 4(R-r)-4 .. +3
         for (int b = 0; b < kGroup; b += 4) {
@@ -201,7 +217,7 @@ int emit_tile(const uint16_t* tile, int ld, uint32_t* dst, TileScratch& ws)
     uint32_t* tail = dst + R * kGroup * kVec;
     for (int b = 0; b < rem; b++)
         for (int v = 0; v < kVec; v++)
-            tail[b * kVec + v] = ws.seq[(kVec - 1 - v) * rem + b];
+            tail[b * kVec + v] = seq[(kVec - 1 - v) * rem + b];
     return count;
 }
 
@@ -337,7 +353,13 @@ int encode_into(const uint16_t* A, int M, int K, bool reorder, void* (*allocate)
             ok = false;
             return;
         }
-        for (long c; (c = next_chunk.fetch_add(1)) < chunks;) {
+        // The chunks that are encoded at the same time are a share apart: threads next to each other would all fault on
+        // the same huge page of new memory, and each clear one for it (words of 7168 x 7168 at 80 %: 2.2 ms, now 1.8).
+        const long share = (chunks + threads - 1) / threads;
+        for (long taken; (taken = next_chunk.fetch_add(1)) < share * threads;) {
+            const long c = taken % threads * share + taken / threads;
+            if (c >= chunks)
+                continue;
             const long i = c / chunks_per_row;
             const int j0 = static_cast<int>(c % chunks_per_row) * kChunkTiles, j1 = std::min(j0 + kChunkTiles, tc);
             for (int j = j0; j < j1; j++) {

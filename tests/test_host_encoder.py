@@ -339,3 +339,26 @@ def test_encoded_arrays_own_their_memory(spmm, entry):
     assert np.array_equal(np.ctypeslib.as_array(w, shape=items.shape), items)
     lib.SpMM_FreeHost(w)
     lib.SpMM_FreeHost(o)
+
+
+@pytest.mark.parametrize("heights", ["one", "few", "full", "staggered"])
+@pytest.mark.parametrize("extra", [0, 1, 2, 3])
+def test_uneven_banks(spmm, oracle, heights, extra):
+    """Levels that no bank but one reaches, that all reach (none, or all 256), and everything between, with 0 to 3 words
+    more for the pads: what is moved together of the pop sequence and what already lies in it."""
+    rng = np.random.default_rng(extra)
+    M, K = 128, 64 * 20
+    want = {"one": [256] + [0] * 31, "few": [0, 0, 255, 0, 1, 128] + [0] * 25 + [2], "full": [256] * 32,
+            "staggered": [(7 * b * b) % 257 for b in range(32)]}[heights]
+    bank = ((np.arange(64) ^ ((np.arange(128)[:, None] & 7) << 3)) >> 1).ravel()  # of (row, column)
+    A = np.zeros((M, K), dtype=np.uint16)
+    for c in range(0, K, 64):
+        tile = np.zeros(128 * 64, dtype=np.uint16)
+        order = rng.permutation(32)
+        for b in range(32):
+            n = min(want[b] + (extra if b == 4 else 0), 256)
+            tile[rng.choice(np.flatnonzero(bank == order[b]), size=n, replace=False)] = rng.integers(1, 0x7C01, size=n)
+        A[:, c:c + 64] = tile.reshape(128, 64)
+    items, offsets = spmm.InitSparseMatrixA_API(A.view(np.float16))
+    o_items, o_offsets = oracle.encode(A.view(np.float16))
+    assert np.array_equal(offsets, o_offsets) and np.array_equal(items, o_items)
