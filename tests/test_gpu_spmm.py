@@ -1197,3 +1197,29 @@ def test_two_waves_per_tile_row_at_64_tokens(spmm, oracle, M, K, split_k, sparsi
     size = np.abs(A.astype(np.float32))
     bound = 2.0 ** -10 * (np.abs(np.nan_to_num(B.astype(np.float32), posinf=0.0)) @ size.T) + 2.0 ** -24
     assert (np.abs(got[0].astype(np.float32) - got[1].astype(np.float32)) <= bound).all()
+
+
+@pytest.mark.parametrize("row_major", [0, 1])
+@pytest.mark.parametrize("waves,tiles,split_k", [(1, 2, 1), (2, 1, 1), (2, 3, 2), (3, 2, 1), (3, 7, 1), (4, 1, 1), (4, 2, 1),
+                                                 (4, 3, 1), (4, 16, 3)])
+def test_final_sum_at_64_tokens_of_every_wave_count(spmm, waves, tiles, split_k, row_major):
+    """The K-splitting layout's final sum in groups of cells: wave counts that divide the cells and that do not, fewer tiles
+    than waves. Whole numbers, so that every sum is exact: |a| <= 2, |b| <= 3 at 0.9 sparsity stay below 2048."""
+    torch = _torch()
+    M, K, N, dev = 256, 64 * tiles, 64, torch.device("cuda:0")
+    rng = np.random.default_rng(waves * 100 + tiles)
+    A = rng.integers(-2, 3, (M, K)).astype(np.float16)
+    A[rng.random((M, K)) < 0.9] = 0
+    B = rng.integers(-3, 4, (N, K)).astype(np.float16)
+    ref = B.astype(np.float32) @ A.astype(np.float32).T
+    assert (np.abs(B.astype(np.float32)) @ np.abs(A.astype(np.float32)).T).max() <= 2048
+    items, offsets = spmm.InitSparseMatrixA_API(A)
+    d_items = torch.from_numpy(items.view(np.int32).copy()).to(dev)
+    d_offs = torch.from_numpy(offsets.copy()).to(dev)
+    d_B = torch.from_numpy(np.ascontiguousarray(B.T if row_major else B)).to(dev)
+    d_W = torch.full((split_k, N * M), float("nan"), dtype=torch.float16, device=dev)
+    C = torch.full((M, N) if row_major else (N, M), float("nan"), dtype=torch.float16, device=dev)
+    print(f"[gpu case] final sum waves={waves} tiles={tiles} split_k={split_k} row_major={row_major}", flush=True)
+    spmm.SpMM_SplitK_API_Planned(torch.cuda.current_stream(), d_items, d_offs, d_B, C, M, N, K, d_W, split_k, 1, waves, 0, row_major)
+    torch.cuda.synchronize()
+    assert np.array_equal((C.t() if row_major else C).cpu().numpy().astype(np.float32), ref)
