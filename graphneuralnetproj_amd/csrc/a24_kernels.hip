@@ -767,9 +767,9 @@ __device__ __forceinline__ void shared_b_product(const uint8_t* __restrict__ pac
     // stride ldc, clamped if relu), like the main kernel's K-splitting layout and with the same bits
     // as the reduction kernel.
     if (arrivals)
-        inlaunch::fused_reduction_tail(out, fused_out, M, n_tokens, static_cast<int>(ldc), gridDim.y, relu,
-                                       blockIdx.x * (16 * RB * W), 16 * RB * W, arrivals + blockIdx.x,
-                                       reinterpret_cast<unsigned int*>(tile), W * kWave, RM);
+        inlaunch::fused_reduction_tail<16 * RB * W, RM>(out, fused_out, M, n_tokens, static_cast<int>(ldc), gridDim.y, relu,
+                                                        blockIdx.x * (16 * RB * W), arrivals + blockIdx.x,
+                                                        reinterpret_cast<unsigned int*>(tile), W * kWave);
 }
 
 #define A24_PARAMS                                                                                                             \

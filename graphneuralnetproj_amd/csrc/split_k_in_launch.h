@@ -40,20 +40,25 @@ __device__ __forceinline__ half8 load_through(const _Float16* p)
 }
 
 // Fused split-K reduction, called by every thread of a workgroup that has just written its slab
-// of partial sums (through to memory) for rows [row0, row0 + nrows): the last of the Split_K
+// of partial sums (through to memory) for rows [row0, row0 + NROWS): the last of the Split_K
 // workgroups that share those rows adds the slabs up, in slab order like the separate kernel
 // (csrc/Reduction_Kernel.cuh:36-46), so both paths give the same bits.  `counter` is the rows'
 // arrival count in device memory (zero between calls), `flag` one free LDS word, nthreads the
 // number of threads of the workgroup that are still there (the first nthreads).
 // Bits 8 and up of `relu` count further slabs that an earlier launch on the same stream left right
 // behind this launch's own Split_K (the 2:4 part's partial sums); they are added after them.
-// row_major: slabs and C are [M][N] (the rows' block is one contiguous run of nrows * N values;
+// ROWMAJ: slabs and C are [M][N] (the rows' block is one contiguous run of NROWS * N values;
 // ldc is not used) instead of one M vector per token.
-// The sum moves eight rows at a time: nrows, M and row0 must be multiples of 8 (the launchers check M).
+// The sum moves eight rows at a time: NROWS, M and row0 must be multiples of 8, and M one of NROWS (the launchers check M).
+// What bounds it is trips to memory (0.7 us each), then its own instructions, which nothing in the launch has run before:
+// the number of rows and the layout are constants (no division for a run's place), and what is left behind the groups
+// of four slabs takes one trip (one by one before), its code out of the way of those.  1024 x 1024 at 8 tokens in four
+// batches 6.38 -> 6.26 us, 1024 x 2048 at 16 tokens in three 8.3 -> 7.9, in seven 7.93 -> 7.30.  (A last group of four
+// that repeats its last slab and masks it: 2 to 4 % slower at five and eight slabs, each load goes to memory.)
+template <int NROWS, bool ROWMAJ>
 __device__ __forceinline__ void fused_reduction_tail(const _Float16* __restrict__ slabs, _Float16* __restrict__ C, int M,
-                                                     int N, int ldc, int split_k, int relu, int row0, int nrows,
-                                                     unsigned int* counter, unsigned int* flag, int nthreads,
-                                                     bool row_major)
+                                                     int N, int ldc, int split_k, int relu, int row0,
+                                                     unsigned int* counter, unsigned int* flag, int nthreads)
 {
     // This workgroup's partial sums have reached memory before it is counted.  The hardware side
     // of that is the wait (the write-through stores are acknowledged at the coherence point); the
@@ -72,9 +77,8 @@ __device__ __forceinline__ void fused_reduction_tail(const _Float16* __restrict_
         return;
     split_k += relu >> 8;
     relu &= 0xff;
-    nrows = nrows < M - row0 ? nrows : M - row0;
-    const int per_tok = nrows / 8;
-    const int total = per_tok * N;  // runs of eight rows to sum
+    constexpr int kPerTok = NROWS / 8;
+    const int total = kPerTok * N;  // runs of eight rows to sum
     const size_t slab = (size_t)M * N;
     // Every load is served from memory, and a thread can only add what has arrived.  A thread with
     // several runs of eight rows (64 tokens: four per thread) keeps four slabs of four runs in flight,
@@ -82,65 +86,72 @@ __device__ __forceinline__ void fused_reduction_tail(const _Float16* __restrict_
     // run (9216 x 9216, 64 tokens, three batches: 28.9 -> 26.2 us).  Each element's slabs are still
     // added in slab order.  (Sixteen slabs of one run at a time, for the threads that have a single
     // run, measured 2 to 3 % slower than four even where there are only four.)
-    auto sum_runs = [&](auto it_c, auto g_c) __attribute__((always_inline)) {
-        constexpr int IT = decltype(it_c)::value, G = decltype(g_c)::value;
-        for (int c0 = threadIdx.x; c0 < total; c0 += nthreads * IT) {
-            size_t at[IT];
-            float sum[IT][8];
+    auto sum_runs = [&](int c0, auto it_c) __attribute__((always_inline)) {
+        constexpr int IT = decltype(it_c)::value, G = 4;
+        int tok[IT], row[IT];
+        uint32_t at[IT];  // (a slab is 4096 groups of rows and 64 tokens at most: 32 bits)
+        float sum[IT][8];
 #pragma unroll
-            for (int i = 0; i < IT; i++) {
-                const int c = c0 + i * nthreads < total ? c0 + i * nthreads : c0;  // a run past the end repeats the first
-                const int tok = c / per_tok, m8 = c - tok * per_tok;
-                at[i] = row_major ? (size_t)row0 * N + (size_t)c * 8 : (size_t)tok * M + row0 + m8 * 8;
+        for (int i = 0; i < IT; i++) {
+            const int c = IT == 1 || c0 + i * nthreads < total ? c0 + i * nthreads : c0;  // a run past the end repeats the first
+            tok[i] = c / kPerTok, row[i] = c % kPerTok * 8;
+            at[i] = ROWMAJ ? static_cast<uint32_t>(row0) * N + c * 8 : static_cast<uint32_t>(tok[i]) * M + row0 + row[i];
 #pragma unroll
-                for (int j = 0; j < 8; j++)
-                    sum[i][j] = 0.f;
-            }
-            int sidx = 0;
-            for (; sidx + G <= split_k; sidx += G) {
-                half8 w[IT][G];
+            for (int j = 0; j < 8; j++)
+                sum[i][j] = 0.f;
+        }
+        const _Float16* from = slabs;
+        int left = split_k;
+        for (; left >= G; left -= G, from += G * slab) {
+            half8 w[G][IT];
 #pragma unroll
-                for (int u = 0; u < G; u++)
-#pragma unroll
-                    for (int i = 0; i < IT; i++)
-                        w[i][u] = load_through(slabs + at[i] + (size_t)(sidx + u) * slab);
-#pragma unroll
-                for (int u = 0; u < G; u++)
-#pragma unroll
-                    for (int i = 0; i < IT; i++)
-#pragma unroll
-                        for (int j = 0; j < 8; j++)
-                            sum[i][j] += static_cast<float>(w[i][u][j]);
-            }
-            for (; sidx < split_k; sidx++) {
-                half8 w[IT];
+            for (int u = 0; u < G; u++)
 #pragma unroll
                 for (int i = 0; i < IT; i++)
-                    w[i] = load_through(slabs + at[i] + (size_t)sidx * slab);
+                    w[u][i] = load_through(from + u * slab + at[i]);
+#pragma unroll
+            for (int u = 0; u < G; u++)
 #pragma unroll
                 for (int i = 0; i < IT; i++)
 #pragma unroll
                     for (int j = 0; j < 8; j++)
-                        sum[i][j] += static_cast<float>(w[i][j]);
-            }
+                        sum[i][j] += static_cast<float>(w[u][i][j]);
+        }
+        if (__builtin_expect(left > 0, 0)) {  // the rest
+            half8 w[G - 1][IT];
 #pragma unroll
-            for (int i = 0; i < IT; i++) {
-                const int c = c0 + i * nthreads;
-                if (c >= total)
-                    break;
-                half8 o;
+            for (int u = 0; u < G - 1; u++)
+                if (u == 0 || u < left)
 #pragma unroll
-                for (int j = 0; j < 8; j++)
-                    o[j] = static_cast<_Float16>(relu ? fmaxf(sum[i][j], 0.f) : sum[i][j]);
-                const int tok = c / per_tok, m8 = c - tok * per_tok;
-                *reinterpret_cast<half8*>(C + (row_major ? at[i] : (size_t)tok * ldc + row0 + m8 * 8)) = o;
-            }
+                    for (int i = 0; i < IT; i++)
+                        w[u][i] = load_through(from + u * slab + at[i]);
+#pragma unroll
+            for (int u = 0; u < G - 1; u++)
+                if (u == 0 || u < left)
+#pragma unroll
+                    for (int i = 0; i < IT; i++)
+#pragma unroll
+                        for (int j = 0; j < 8; j++)
+                            sum[i][j] += static_cast<float>(w[u][i][j]);
+        }
+#pragma unroll
+        for (int i = 0; i < IT; i++) {
+            if (IT > 1 && c0 + i * nthreads >= total)
+                break;
+            half8 o;
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                o[j] = static_cast<_Float16>(relu ? fmaxf(sum[i][j], 0.f) : sum[i][j]);
+            *reinterpret_cast<half8*>(C + (ROWMAJ ? (size_t)at[i] : (size_t)tok[i] * ldc + row0 + row[i])) = o;
         }
     };
-    if (total <= nthreads)
-        sum_runs(std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{});
-    else
-        sum_runs(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
+    if (total <= nthreads) {
+        if (static_cast<int>(threadIdx.x) < total)
+            sum_runs(threadIdx.x, std::integral_constant<int, 1>{});
+    } else {
+        for (int c0 = threadIdx.x; c0 < total; c0 += nthreads * 4)
+            sum_runs(c0, std::integral_constant<int, 4>{});
+    }
     if (threadIdx.x == 0)
         *counter = 0;  // ready for the next call
 }

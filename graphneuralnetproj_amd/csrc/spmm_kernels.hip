@@ -910,8 +910,8 @@ __global__ __launch_bounds__(MAXW* kWave) void tcsl_spmm_kernel(const int* __res
         write_out();
     if (!KSPLIT || !arrivals)
         return;
-    fused_reduction_tail(out, fused_out, M, NTOK, ldc, split_k, relu, blockIdx.x * kTileRows, kTileRows,
-                         arrivals + blockIdx.x, reinterpret_cast<unsigned int*>(lds), W * kWave, ROWMAJ);
+    fused_reduction_tail<kTileRows, ROWMAJ>(out, fused_out, M, NTOK, ldc, split_k, relu, blockIdx.x * kTileRows,
+                                            arrivals + blockIdx.x, reinterpret_cast<unsigned int*>(lds), W * kWave);
 }
 
 // 64 tokens, two waves to a work unit: both work on every tile of the unit's run, each scatters half of

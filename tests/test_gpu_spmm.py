@@ -1223,3 +1223,30 @@ def test_final_sum_at_64_tokens_of_every_wave_count(spmm, waves, tiles, split_k,
     spmm.SpMM_SplitK_API_Planned(torch.cuda.current_stream(), d_items, d_offs, d_B, C, M, N, K, d_W, split_k, 1, waves, 0, row_major)
     torch.cuda.synchronize()
     assert np.array_equal((C.t() if row_major else C).cpu().numpy().astype(np.float32), ref)
+
+
+@pytest.mark.parametrize("row_major", [0, 1])
+@pytest.mark.parametrize("N", [8, 16, 32, 64])
+@pytest.mark.parametrize("split_k", [2, 3, 4, 5, 6, 7, 8, 11])
+def test_in_launch_sum_of_every_rest(spmm, split_k, N, row_major):
+    """The sum in the launch takes slabs four at a time and what is left in one more trip: every rest, one and four runs of
+    eight rows a thread, against the reduction kernel bit for bit."""
+    torch = _torch()
+    M, K, dev = 256, 64 * 24, torch.device("cuda:0")
+    A = spmm.synth_weights(M, K, 0.8, False, seed=split_k)
+    B = spmm.synth_activations(N, K, seed=N)
+    items, offsets = spmm.InitSparseMatrixA_API(A)
+    d_items = torch.from_numpy(items.view(np.int32).copy()).to(dev)
+    d_offs = torch.from_numpy(offsets.copy()).to(dev)
+    d_B = torch.from_numpy(np.ascontiguousarray(B).view(np.int16).copy()).to(dev).view(torch.float16)
+    if row_major:
+        d_B = d_B.t().contiguous()
+    print(f"[gpu case] in-launch sum split_k={split_k} N={N} row_major={row_major}", flush=True)
+    got = []
+    for flags in (0, spmm.SPMM_FLAG_SEPARATE_REDUCTION):
+        d_W = torch.full((split_k, N * M), float("nan"), dtype=torch.float16, device=dev)
+        C = torch.full((M, N) if row_major else (N, M), float("nan"), dtype=torch.float16, device=dev)
+        spmm.SpMM_SplitK_API_Planned(torch.cuda.current_stream(), d_items, d_offs, d_B, C, M, N, K, d_W, split_k, 1, 4, 0, row_major, flags)
+        torch.cuda.synchronize()
+        got.append(C.cpu())
+    assert torch.isfinite(got[0]).all() and torch.equal(got[0], got[1])
