@@ -132,6 +132,9 @@ __device__ __forceinline__ int half_wave_reduce(int x, int neutral, Op op)
 // at 50 / 80 / 95 %: 157 / 97 / 88 us, now 132 / 77 / 70; 1024 x 1024 at 80 %: 5.3, now 4.9.)
 constexpr int kSeqWords = 4096, kPassWords = kSeqWords - 128;  // the first pass takes the tail's up to 124 pops as well
 
+// Offset: of a lane's rows in bytes, the upper row group's being 32 K.  64 bits from K = 2^27 on; below, 32, which the loads
+// take beside a uniform address (two instructions fewer for each of a lane's sixteen).
+template<typename Offset>
 __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* __restrict__ A, int K, int tiles_k,
                                                               const int* __restrict__ offsets, uint32_t* __restrict__ items)
 {
@@ -154,7 +157,7 @@ __global__ __launch_bounds__(kThreads, 7) void tcsl_emit_tiles(const uint16_t* _
     //    Row m gives bank b the pair of adjacent columns whose swizzled positions are 2 b, 2 b + 1.
     // (a row's address is uniform but for this lane's part, of which there are eight)
     const uint8_t* const rows = reinterpret_cast<const uint8_t*>(tile) + (size_t)(wave * 2 * kRowsPerThread) * K * 2;
-    const uint32_t own_row = (rg & 1) * (uint32_t)kRowsPerThread * K * 2;
+    const Offset own_row = (rg & 1) * static_cast<Offset>(kRowsPerThread * 2) * K;
     uint32_t pairs[kRowsPerThread];
 #pragma unroll
     for (int i = 0; i < kRowsPerThread; i++)
@@ -317,7 +320,8 @@ extern "C" int tcsl_launch_encode_items(void* stream, const void* A, int M, int 
     const long tiles_k = K / kTileCols, tiles = (long)(M / kTileRows) * tiles_k;
     if (tiles < 1 || tiles > 0x7fffffffL)
         return static_cast<int>(hipErrorInvalidValue);
-    hipLaunchKernelGGL(tcsl_emit_tiles, dim3((unsigned)tiles), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
+    auto* const emit = K < 1 << 27 ? tcsl_emit_tiles<uint32_t> : tcsl_emit_tiles<uint64_t>;
+    hipLaunchKernelGGL(emit, dim3((unsigned)tiles), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
                        static_cast<const uint16_t*>(A), K, (int)tiles_k, offsets, static_cast<uint32_t*>(items));
     return static_cast<int>(hipGetLastError());
 }

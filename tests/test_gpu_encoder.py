@@ -242,3 +242,35 @@ def test_device_encoder_uneven_banks(spmm, oracle, heights, extra):
                 tile.ravel()[rng.choice(at, size=n, replace=False)] = rng.choice([0x0001, 0x8001, 0x7C00, 0xFC00, 0x3C00], size=n)
             A[r:r + 128, c:c + 64] = tile
     _compare(spmm, oracle, A.view(np.float16))
+
+
+@pytest.mark.parametrize("K", [(1 << 27) - 64, 1 << 27, (1 << 27) + 64])
+def test_device_encoder_rows_of_a_quarter_gigabyte(spmm, oracle, K):
+    """Sixteen rows of 2^27 columns are 2^32 bytes: tiles of odd and even row groups at the matrix's start, end and
+    in between, all other tiles empty, each against the oracle on the tile alone."""
+    torch = _torch()
+    M, tiles = 128, K // 64
+    if torch.cuda.mem_get_info()[0] < 2 * M * K + (4 << 30):
+        pytest.skip("needs 36 GiB of device memory")
+    rng = np.random.default_rng(K % 1000)
+    at = sorted({0, 1, tiles // 2, tiles - 2, tiles - 1, *rng.integers(0, tiles, 20).tolist()})
+    A = rng.standard_normal((M, 64 * len(at))).astype(np.float16)
+    A[rng.random(A.shape) < 0.8] = 0
+    A[64:] = np.where(rng.random((64, A.shape[1])) < 0.5, A[64:], np.float16(0))  # row groups of different densities
+    d_A = torch.zeros((M, K), dtype=torch.float16, device="cuda:0")
+    for i, t in enumerate(at):
+        d_A[:, 64 * t:64 * t + 64] = torch.from_numpy(A[:, 64 * i:64 * i + 64].copy()).cuda()
+    print(f"[gpu case] device encode {M} x {K}", flush=True)
+    d_items, d_offsets = spmm.encode_on_device(d_A)
+    torch.cuda.synchronize()
+    del d_A
+    torch.cuda.empty_cache()
+    counts = np.zeros(tiles, dtype=np.int64)
+    words = []
+    for i, t in enumerate(at):
+        items, offsets = oracle.encode(A[:, 64 * i:64 * i + 64])
+        counts[t] = offsets[-1]
+        words.append(items[:4 * offsets[-1]])
+    offsets = d_offsets.cpu().numpy()
+    assert offsets[0] == 0 and np.array_equal(np.diff(offsets), np.append(counts, 0))
+    assert np.array_equal(d_items.cpu().numpy().view(np.uint32), np.concatenate(words))
