@@ -313,7 +313,7 @@ def sweep(G, lib, torch, dev, sptr, with_stack):
         out.append({"case": label, "M": M, "K": K, "N": N, "sparsity": sparsity, "row_skewed": skew, "split_k": split_k,
                     "split_k_from": "sweep" if forced_split else "planner",
                     "layout": "B[K][N], C[M][N]" if row_major else "B[N][K], C[N][M]",
-                    "plan": f"mode {plan['mode']}, {plan['waves']} waves" + (", in pairs" if plan["paired"] else ""), "compressed_bytes": a_bytes,
+                    "plan": f"mode {plan['mode']}, {plan['waves']} waves" + (", in pairs" if plan["paired"] else ", two to a tile row" if plan["two_per_row"] and not row_major else ""), "compressed_bytes": a_bytes,
                     "reduction": ("none" if split_k == 1 else
                                   "in launch" if G.SpMM_PlanReductionInLaunch(M, N, K, split_k) else "kernel"),
                     "ms": ms, "frac": a_bytes / (ms * 1e-3) / 1e9 / HBM_PEAK_GBPS,

@@ -122,7 +122,7 @@ bool complete_plan(int N, int K, int split_k, bool row_major, LaunchPlan& p)
     const long tiles = (nkb - 1) / split_k + 1;  // tiles of the longest batch
     long lds = p.waves * kTileLds;
     if (row_major) {
-        if (p.stage_b)
+        if (p.stage_b && p.stage_b != 4)
             return false;
         lds += static_cast<long>(p.waves) * N * 128;  // one tile's activations per wave, being transposed
     }
@@ -139,6 +139,10 @@ bool complete_plan(int N, int K, int split_k, bool row_major, LaunchPlan& p)
             if (row_major || N != 64 || p.waves != 2 || tiles > 63)
                 return false;
             lds = 3 * kTileLds;
+        } else if (p.stage_b == 4) {  // two images a tile row, and each half's activation tiles of the step and of the next
+            if (N != 64 || !(p.waves == 3 || (p.waves == 4 && row_major)))
+                return false;
+            lds = p.waves * 2 * kTileLds + 2L * (p.waves == 3 ? 4 : 2) * N * 128;
         } else if (p.stage_b != 0) {
             return false;
         }
@@ -155,6 +159,21 @@ bool complete_plan(int N, int K, int split_k, bool row_major, LaunchPlan& p)
         return false;
     p.lds_bytes = static_cast<unsigned>(lds);
     return true;
+}
+
+// Two waves to a tile row where the row-sharing layout has three or four tile rows to a workgroup and a batch is long enough
+// to pay for the second barrier and the sum of the halves.  Measured on 60 calls, one wave to a row -> two: three rows,
+// column-major, 1.02 to 1.16 times as fast from four tiles a batch on (49152 x 12288 at 80 % 130 -> 119 us, at 60 % 216 ->
+// 177, at 90 % 106 -> 92; 0.97 to 0.99 with one or two tiles), row-major 1.05 to 1.4 (149 -> 119, 219 -> 175, 129 -> 93);
+// four rows, row-major, 1.01 to 1.33 from 20 tiles on (36864 x 9216 in three batches 82 -> 74), 0.97 to 1.08 below; four
+// rows, column-major, 0.98 to 1.04 at 60 to 80 %: left to one wave.
+LaunchPlan with_two_waves(int N, int K, int split_k, bool row_major, const LaunchPlan& p)
+{
+    const long tiles = (K / kTileCols - 1) / split_k + 1;
+    LaunchPlan two{0, p.waves, 4, 0};
+    if (N == 64 && p.mode == 0 && p.stage_b == 0 && tiles >= (p.waves == 3 ? 4 : 20) && complete_plan(N, K, split_k, row_major, two))
+        return two;
+    return p;
 }
 
 double plan_cost_us(int M, int N, int K, int split_k, const LaunchPlan& p, double tile_bytes)
@@ -224,8 +243,8 @@ LaunchPlan plan_launch(int M, int N, int K, int split_k, bool row_major, double*
         p.separate_reduction = t->separate_reduction != 0;
         if (complete_plan(N, K, split_k, row_major, p)) {
             if (cost_us)
-                *cost_us = plan_cost_us(M, N, K, split_k, p, tile_bytes);
-            return p;
+                *cost_us = plan_cost_us(M, N, K, split_k, p, tile_bytes);  // (of one wave to a tile row)
+            return with_two_waves(N, K, split_k, row_major, p);
         }
     }
     LaunchPlan best{0, 1, 0, static_cast<unsigned>(kTileLds)};
@@ -275,7 +294,7 @@ LaunchPlan plan_launch(int M, int N, int K, int split_k, bool row_major, double*
             complete_plan(N, K, split_k, row_major, pair))
             return pair;
     }
-    return best;
+    return with_two_waves(N, K, split_k, row_major, best);
 }
 
 int suggest_split_k(int M, int N, int K, LaunchPlan* plan, double tile_bytes)
@@ -285,7 +304,7 @@ int suggest_split_k(int M, int N, int K, LaunchPlan* plan, double tile_bytes)
         p.separate_reduction = t->separate_reduction != 0;
         if (complete_plan(N, K, t->split_k, false, p)) {
             if (plan)
-                *plan = p;
+                *plan = with_two_waves(N, K, t->split_k, false, p);
             return t->split_k;
         }
     }

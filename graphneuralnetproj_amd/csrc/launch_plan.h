@@ -1,5 +1,6 @@
 // Launch shape of the main kernel and the cost model that picks it.  Host only.
 #pragma once
+#include <cstdint>
 
 namespace tcsl {
 
@@ -11,6 +12,8 @@ namespace tcsl {
 //         kernel instead of by the last workgroup of each tile row inside the launch (mode 0 always
 //         uses the reduction kernel).
 // stage_b = 3 (mode 0, 2 waves, 64 tokens): both waves work on every tile of one tile row, with 32 tokens each.
+// stage_b = 4 (mode 0, 64 tokens, waves = 3 or, row-major, 4): `waves` tile rows to a workgroup with two waves each, which
+//         take the two halves of the batch; only for activations that two_waves_fit() takes.
 struct LaunchPlan {
     int mode;
     int waves;
@@ -21,6 +24,15 @@ struct LaunchPlan {
 
 // True (and lds_bytes filled in) when the kernels can run this shape.
 bool complete_plan(int N, int K, int split_k, bool row_major, LaunchPlan& p);
+
+// p, or the same tile rows with two waves each (stage_b = 4) where those are faster.
+LaunchPlan with_two_waves(int N, int K, int split_k, bool row_major, const LaunchPlan& p);
+// What stage_b = 4 asks of the activations: they go straight into LDS, 16 bytes a lane, at 32-bit offsets from a group of
+// eight tokens.
+inline bool two_waves_fit(const void* B, long ldb, bool row_major)
+{
+    return (reinterpret_cast<uintptr_t>(B) & 15) == 0 && (row_major || (ldb % 8 == 0 && ldb <= 1L << 28));
+}
 
 // Estimated time in microseconds of SpMM_SplitK_API (main kernel + reduction) with this plan.
 // tile_bytes: average compressed bytes per 128 x 64 tile of the weight (16 * vectors / tiles);

@@ -183,10 +183,19 @@ int launch_main(void* stream, const void* Compressed_A, const int* TileOffsets, 
     }
     if (fused)
         *fused = page >= 0;
+    tcsl::LaunchPlan run = p;
+    if (o.forced && o.adaptive_waves)
+        run = tcsl::with_two_waves(N, K, Split_K, o.row_major, p);
+    if (run.stage_b == 4 && !tcsl::two_waves_fit(B, ldb, o.row_major)) {
+        if (p.stage_b == 4 && o.forced)
+            return tcsl_error_invalid_value();
+        run = tcsl::LaunchPlan{0, run.waves, 0, 0};  // one wave to a tile row reads them anywhere
+        if (!tcsl::complete_plan(N, K, Split_K, o.row_major, run))
+            return tcsl_error_invalid_value();
+    }
     // The plan's wave count is tuned on 80 % sparse weights.  Sparser ones want every wave the
     // registers allow (a wave's turnaround per tile becomes the limit), which the host cannot see:
     // in the K-splitting layout it launches them all and lets each workgroup look at its own tiles.
-    tcsl::LaunchPlan run = p;
     int dense_waves = 0;
     if ((!o.forced || o.adaptive_waves) && p.mode == 1 && N <= 32 && p.waves < 8) {
         tcsl::LaunchPlan all{1, 8, 0, 0};
@@ -311,7 +320,7 @@ extern "C" int SpMM_PlanLaunch(int M, int N, int K, int Split_K, int* Mode, int*
     if (Waves)
         *Waves = p.waves;
     if (StageB)
-        *StageB = p.stage_b == 3 ? 0 : p.stage_b;  // (told apart by LdsBytes)
+        *StageB = p.stage_b >= 3 ? 0 : p.stage_b;  // (told apart by LdsBytes)
     if (LdsBytes)
         *LdsBytes = static_cast<int>(p.lds_bytes);
     if (EstimatedUs)

@@ -62,6 +62,7 @@
 #include <mutex>
 #include <utility>
 
+#include "launch_plan.h"
 #include "split_k_in_launch.h"
 
 namespace {
@@ -1184,7 +1185,7 @@ __global__ __launch_bounds__(2 * kWave, 2) void tcsl_spmm_pair_kernel(const int*
 // behind it nobody reads the ones before, and the next are fetched into their place.  Two tiles between barriers, where LDS has
 // the room, let the waves' memory latencies even out (126 -> 120 us).  Every wave of the workgroup takes the same number of steps;
 // an empty tile (or one past a half's end) is not multiplied.
-// Measured, and where it is used: tcsl_launch_spmm.  The images are ROWS * 32 KiB of LDS, the activations kTiles * 32 KiB.
+// Measured, and where it is used: launch_plan.cpp, with_two_waves.  The images are ROWS * 32 KiB of LDS, the activations kTiles * 32 KiB.
 constexpr int halves_tiles(int rows)  // tiles between two barriers
 {
     return rows < 4 ? 2 : 1;
@@ -1701,10 +1702,11 @@ int launch_pair(hipStream_t stream, const void* items, const int* offsets, const
 //         (N <= 16) they share the batch's activation slice, staged once in LDS; with stage_b = 2
 //         (N = 32: 4 or 8 waves, N = 64: 4 waves) they walk the batch in step and share each
 //         activation tile through LDS; with stage_b = 3 (N = 64, two waves) both work on one tile row,
-//         with half of the tokens each;
+//         with half of the tokens each; with stage_b = 4 (N = 64, W = 3, or 4 row-major; B as two_waves_fit() asks) the
+//         workgroup has two waves to each of W tile rows, which take the halves of the batch;
 // mode 1: the W waves of a workgroup split the batch of one tile row among themselves and
 //         add their results up in LDS (stage_b must be 0).
-// row_major: B is [K][N] and the output [M][N] instead of [N][K] and [N][M] (stage_b must be 0).
+// row_major: B is [K][N] and the output [M][N] instead of [N][K] and [N][M] (stage_b must be 0 or 4).
 // waves = 1..8 for N <= 32, 1..4 for N = 64; lds_bytes = what the shape needs (the host plans it).
 // ldb, ldo: token strides of B and of the output in elements (column-major; multiples of 8).
 // fuse_page >= 0: out = Split_K dense slabs, and the kernel itself reduces them into fused_out
@@ -1730,6 +1732,15 @@ extern "C" int tcsl_launch_spmm(void* stream, const void* items, const int* offs
         if (mode != 0 || row_major || N != 64 || waves != 2 || fuse_page >= 0)
             return static_cast<int>(hipErrorInvalidValue);
         return launch_pair(s, items, offsets, B, out, M, K, split_k, ldb, ldo, relu);
+    }
+    if (stage_b == 4) {
+        if (mode != 0 || N != 64 || fuse_page >= 0 || !tcsl::two_waves_fit(B, ldb, row_major))
+            return static_cast<int>(hipErrorInvalidValue);
+        if (waves == 3)
+            return row_major ? launch_halves<3, true>(s, items, offsets, B, out, M, K, split_k, ldb, ldo, relu)
+                             : launch_halves<3, false>(s, items, offsets, B, out, M, K, split_k, ldb, ldo, relu);
+        return waves == 4 && row_major ? launch_halves<4, true>(s, items, offsets, B, out, M, K, split_k, ldb, ldo, relu)
+                                       : static_cast<int>(hipErrorInvalidValue);
     }
     if (stage_b < 0 || stage_b > 2)
         return static_cast<int>(hipErrorInvalidValue);
@@ -1763,21 +1774,6 @@ extern "C" int tcsl_launch_spmm(void* stream, const void* items, const int* offs
         case 64:
             if (stage_b == 2)
                 return TCSL_GO(4, false, false, false, false, 4, 4);
-            // Two waves to a tile row (tcsl_spmm_halves_kernel) where the row-sharing layout has three or four tile rows to a
-            // workgroup and a batch is long enough to pay for the second barrier and the sum of the halves.  Measured on 60
-            // calls, the other kernel -> this one: three rows, column-major, 1.02 to 1.16 times as fast from four tiles a batch
-            // on (49152 x 12288 at 80 % 130 -> 119 us, at 60 % 216 -> 177, at 90 % 106 -> 92; 0.97 to 0.99 with one or two
-            // tiles), row-major 1.05 to 1.4 (149 -> 119, 219 -> 175, 129 -> 93); four rows, row-major, 1.01 to 1.33 from 20 tiles
-            // on (36864 x 9216 in three batches 82 -> 74), 0.97 to 1.08 below; four rows, column-major, 0.98 to 1.04 at 60 to
-            // 80 %: left to the other kernel.  (The activations go straight into LDS: aligned, and 32-bit offsets of eight tokens.)
-            if (const int tiles = (K / kTileCols - 1) / split_k + 1;
-                mode == 0 && (waves == 3 ? tiles >= 4 : waves == 4 && row_major && tiles >= 20) &&
-                (reinterpret_cast<uintptr_t>(B) & 15) == 0 && (row_major || (ldb % 8 == 0 && ldb <= 1 << 28))) {
-                if (waves == 4)
-                    return launch_halves<4, true>(s, items, offsets, B, out, M, K, split_k, ldb, ldo, relu);
-                return row_major ? launch_halves<3, true>(s, items, offsets, B, out, M, K, split_k, ldb, ldo, relu)
-                                 : launch_halves<3, false>(s, items, offsets, B, out, M, K, split_k, ldb, ldo, relu);
-            }
             return TCSL_PICK(4, false, 4);
         default:
             return static_cast<int>(hipErrorInvalidValue);

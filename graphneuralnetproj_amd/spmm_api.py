@@ -390,8 +390,9 @@ def SpMM_SuggestSplitK_Bytes(M_Global, N_Global, K_Global, Vectors):
 
 
 def SpMM_PlanLaunch(M_Global, N_Global, K_Global, Split_K):
-    """The planner's launch shape for a call: dict(mode, waves, stage_b, lds_bytes, estimated_us, paired).  paired: both
-    waves work on every tile (64 tokens); SpMM_SplitK_API_Planned launches that shape with StageB = 3."""
+    """The planner's launch shape for a call: dict(mode, waves, stage_b, lds_bytes, estimated_us, paired, two_per_row).
+    paired: both waves work on every tile (64 tokens); SpMM_SplitK_API_Planned launches that shape with StageB = 3.  two_per_row:
+    `waves` counts tile rows, of two waves each (64 tokens); StageB = 4 there."""
     vals = [ctypes.c_int() for _ in range(4)]
     est = ctypes.c_double()
     rc = load_library().SpMM_PlanLaunch(M_Global, N_Global, K_Global, Split_K, *[ctypes.byref(v) for v in vals],
@@ -399,7 +400,8 @@ def SpMM_PlanLaunch(M_Global, N_Global, K_Global, Split_K):
     if rc != 0:
         raise SpMMError("SpMM_PlanLaunch", rc)
     return {"mode": vals[0].value, "waves": vals[1].value, "stage_b": vals[2].value, "lds_bytes": vals[3].value,
-            "estimated_us": est.value, "paired": (vals[0].value, vals[1].value, vals[3].value) == (0, 2, 3 * 16384)}
+            "estimated_us": est.value, "paired": (vals[0].value, vals[1].value, vals[3].value) == (0, 2, 3 * 16384),
+            "two_per_row": N_Global == 64 and (vals[0].value, vals[1].value, vals[2].value, vals[3].value) == (0, 3, 0, 160 * 1024)}
 
 
 def SpMM_PlanReductionInLaunch(M_Global, N_Global, K_Global, Split_K):

@@ -25,6 +25,9 @@ OPT_SHAPES = ("28672x7168,7168x28672,21504x7168,7168x7168,27648x9216,9216x9216,3
 
 SEPARATE = 3  # in a plan tuple's last place with mode 1: the slabs are added up by the reduction kernel
 PAIRED = 3  # ... with mode 0: two waves on every tile, 64 tokens.  Timed, but no row: the planner has a rule of its own for it
+# ... with mode 0, three waves, 64 tokens: two waves to a tile row or one, where a planned call of that shape does the other.
+# Timed, but no row: a row's call goes by the planner's rule.
+TWO_PER_ROW, ONE_PER_ROW = 4, 5
 
 
 def planned_args(plan):
@@ -34,6 +37,8 @@ def planned_args(plan):
     S, mode, w, st = plan
     if mode == 1 and st == SEPARATE:
         return S, mode, w, 0, SPMM_FLAG_ADAPTIVE_WAVES | SPMM_FLAG_SEPARATE_REDUCTION
+    if st == ONE_PER_ROW:
+        return S, mode, w, 0, 0
     return S, mode, w, st, SPMM_FLAG_ADAPTIVE_WAVES
 
 
@@ -47,10 +52,13 @@ def table_row(M, K, N, plan):
 def best_row(M, K, N, results):
     """The table's line for the fastest of results, (us, plan) in ascending order of time.  Where that is the paired launch a
     row would keep the planner from it: with the planner pairing there the line is a remark, else it is the
-    row of the fastest other plan."""
+    row of the fastest other plan.  So it is where the planner's rule does not take the form that won (TWO_PER_ROW, ONE_PER_ROW)."""
     from graphneuralnetproj_amd import SpMM_PlanLaunch
 
     us, plan = results[0]
+    if plan[3] in (TWO_PER_ROW, ONE_PER_ROW):
+        form = "two waves" if plan[3] == TWO_PER_ROW else "one wave"
+        return best_row(M, K, N, results[1:]) + f" ({plan[0]} batches, {form} to a tile row: {us:.1f})"
     if plan[1:] != (0, 2, PAIRED):
         return f"    {table_row(M, K, N, plan)},  // {us:.1f} us"
     if SpMM_PlanLaunch(M, N, K, plan[0])["paired"]:
@@ -64,6 +72,10 @@ def candidate_plans(N, tiles_k, only=None):
     Mode 1 with more than one batch is tried with the sum inside the launch and, from four batches on and
     with four waves, with the reduction kernel (last place SEPARATE)."""
     max_w = 8 if N <= 32 else 4
+
+    def other_form(S):  # of (S, 0, 3, 0) at 64 tokens: the planner gives batches of four tiles and more two waves to a tile row
+        return (S, 0, 3, ONE_PER_ROW if -(-tiles_k // S) >= 4 else TWO_PER_ROW)
+
     if only:
         plans = []
         for S in only:
@@ -78,7 +90,7 @@ def candidate_plans(N, tiles_k, only=None):
                 plans += [(S, 0, w, 0) for w in ((1, 2, 3, 4, 5, 6, 8) if N == 32 else (1, 2, 3, 4))]
                 plans += [(S, 0, w, 2) for w in ((4, 8) if N == 32 else (4,))]
             if N == 64:
-                plans.append((S, 0, 2, PAIRED))
+                plans += [(S, 0, 2, PAIRED), other_form(S)]
         return plans
     plans = []
     for S in (1, 2, 3, 4, 6, 8, 12, 16, 24, 32):
@@ -98,7 +110,7 @@ def candidate_plans(N, tiles_k, only=None):
             if S <= tiles_k:
                 plans += [(S, 0, w, 2) for w in ((4, 8) if N == 32 else (4,))]
             if S <= tiles_k and N == 64:
-                plans.append((S, 0, 2, PAIRED))
+                plans += [(S, 0, 2, PAIRED), other_form(S)]
     return plans
 
 

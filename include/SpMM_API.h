@@ -92,7 +92,9 @@ SPMM_EXPORT int SpMM_EncodeInto(const uint16_t* A_h, int M, int K, int Reorder, 
  *                 SpMM_PlanReductionInLaunch tells which).
  *                 Reduction_Workspace must hold Split_K*M*N fp16 values and may be
  *                 shared by successive calls on one stream.
- * Accumulation is fp32.  Returns the hipError_t value: 0 on success;
+ * Accumulation is fp32.  The order of the sums, and with it the last bit of a result, goes by the launch shape: by M,
+ * N, K and Split_K, and at 64 tokens also by the operands' layout and by whether B is 16-byte aligned (below,
+ * SpMM_PlanLaunch).  Returns the hipError_t value: 0 on success;
  * hipErrorUnknown, after printing the reference's message, for N outside
  * {8, 16, 32, 64} (csrc/SpMM_API.cu:192-193); hipErrorInvalidValue for M % 128,
  * K % 64, Split_K < 1, Split_K > 65535 or a null pointer (the reference checks these only in
@@ -160,8 +162,9 @@ SPMM_EXPORT int SpMM_SplitK_API_RowMajor(void* stream, const void* A, const void
  */
 #define SPMM_FLAG_RELU 1
 #define SPMM_FLAG_SEPARATE_REDUCTION 2 /* Split_K > 1: always run the reduction as its own kernel */
-#define SPMM_FLAG_ADAPTIVE_WAVES 4     /* SpMM_SplitK_API_Planned only: treat Waves (Mode 1, N <= 32) the way a planned
-                                          call does, as the count for dense tile rows, and launch eight */
+#define SPMM_FLAG_ADAPTIVE_WAVES 4     /* SpMM_SplitK_API_Planned only: treat Waves the way a planned call does: in Mode 1,
+                                          N <= 32, as the count for dense tile rows, and launch eight; in Mode 0 with
+                                          StageB = 0, 64 tokens, give each tile row two waves where that is faster */
 SPMM_EXPORT int SpMM_SplitK_API_Strided(void* stream, const void* Compressed_A, const int* TileOffsets, const void* B,
                                         long ldb, void* C, long ldc, int M_Global, int N_Global, int K_Global,
                                         void* Reduction_Workspace, int Split_K, int Flags);
@@ -268,11 +271,16 @@ SPMM_EXPORT int SpMM_SuggestSplitK_Bytes(int M_Global, int N_Global, int K_Globa
  *           staged once in LDS; StageB = 2, 32 tokens with 4 or 8 waves and 64 tokens with 4:
  *           they walk the batch in step and share each 64-column activation tile through LDS;
  *           64 tokens with two waves and LdsBytes = 49152: both work on every tile of one tile row,
- *           with half of the tokens each; StageB is 0 here, and 3 for SpMM_SplitK_API_Planned);
+ *           with half of the tokens each; StageB is 0 here, and 3 for SpMM_SplitK_API_Planned;
+ *           64 tokens with three waves and LdsBytes = 163840: three tile rows with two waves each, six in all, which
+ *           take the two halves of the batch; StageB is 0 here, and 4 for SpMM_SplitK_API_Planned.  That shape reads
+ *           its activations straight into LDS: a call whose B is not 16-byte aligned launches one wave to a tile row
+ *           instead, and so does one with ldb % 8 != 0 or above 2^28.  Row-major calls, whose shape may be another,
+ *           also use it with four tile rows and eight waves);
  *   Mode 1  the Waves waves of a workgroup split the batch of one tile row among
  *           themselves and add their accumulators up in LDS.
  * Any output pointer may be NULL.  EstimatedUs is the cost model's figure for the whole
- * call (in the last shape of Mode 0 that of the shape which the planner would take otherwise).
+ * call (in the last two shapes of Mode 0 that of the shape which the planner would take otherwise).
  * Returns 0, or -1 for a shape the kernels do not take.  The reference has one
  * fixed block shape (csrc/SpMM_API.cu:25-71) and nothing like this.
  */
@@ -294,8 +302,10 @@ SPMM_EXPORT int SpMM_PlanReductionInLaunch(int M_Global, int N_Global, int K_Glo
  * SpMM_SplitK_API with the launch shape given by the caller instead of the planner
  * (for tuning a table of plans on the target machine, and for tests).  Returns
  * hipErrorInvalidValue when the shape does not fit (Waves above 8, or 4 for N = 64;
- * StageB with Mode 1 or RowMajor, StageB = 1 with N > 16, StageB = 2 outside the shapes above, StageB = 3
- * with other than two waves, 64 tokens and batches of up to 63 tiles; more than 160 KiB of LDS).  RowMajor != 0 selects
+ * StageB with Mode 1, StageB = 1, 2 or 3 with RowMajor, StageB = 1 with N > 16, StageB = 2 outside the shapes above, StageB = 3
+ * with other than two waves, 64 tokens and batches of up to 63 tiles, StageB = 4 with other than Waves = 3 (tile rows,
+ * of two waves each; with RowMajor also 4), 64 tokens and a 16-byte aligned B; more than 160 KiB of LDS).  StageB = 0 is
+ * one wave to a tile row in Mode 0, unless SPMM_FLAG_ADAPTIVE_WAVES asks for what a planned call does.  RowMajor != 0 selects
  * the operand layout of SpMM_SplitK_API_RowMajor; Flags as for SpMM_SplitK_API_Strided.  No
  * counterpart in the reference.
  */

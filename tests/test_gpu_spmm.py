@@ -1141,22 +1141,25 @@ def test_reduction_kernel_adds_slabs_of_large_outputs(spmm, split_k):
 
 
 @pytest.mark.parametrize("M,K,split_k,sparsity,flags", [
-    (384, 64 * 4, 1, 0.8, 0),            # two tiles for each half
+    (384, 64 * 4, 1, 0.8, 0),            # two tiles for each half; 410 vectors a tile: eight a lane
+    (128, 64, 1, 0.8, 0),                # one tile: the second half has none
+    (256, 64 * 3, 3, 0.9, 1),            # ... in each batch
+    (384, 64 * 4, 3, 0.8, 0),            # batches of two tiles, two and none
     (128, 64 * 5, 1, 0.8, 1),            # one tile row of a workgroup's, halves of three tiles and two, clamped by the kernel
-    (640, 64 * 29, 3, 0.7, 1),           # rows 4 and 5 of three, batches of 10, 10 and 9 tiles, clamped by the reduction
-    (512, 64 * 22, 5, 0.0, 0),           # dense tiles: two segments of ten vectors a lane; batches of 5, 5, 5, 5, 2
-    (768, 64 * 21, 1, 0.5, 0),           # ... of eight and ten
+    (640, 64 * 29, 3, 0.7, 1),           # rows 4 and 5 of three, batches of 10, 10 and 9 tiles, clamped by the reduction; ten a lane
+    (512, 64 * 22, 5, 0.0, 0),           # dense tiles: four segments of eight vectors a lane; batches of 5, 5, 5, 5, 2
+    (768, 64 * 21, 1, 0.5, 0),           # ... two segments or three
+    (512, 64 * 43, 2, 0.72, 0),          # halves of eleven tiles and ten or eleven; ten a lane (573 vectors a tile)
     (896, 64 * 40, 2, 0.97, 0),          # tiles of a few vectors, undone word by word
-    (384, 64 * 131, 1, 0.9, 0),          # more tiles for each half than one window of offsets has
+    (384, 64 * 131, 1, 0.9, 0),          # more tiles for each half than one window of offsets has; four a lane
     (1152, 64 * 24, 1, "mixed", 0),      # tile rows of every density side by side, empty tiles among them
     (128 * 385, 64 * 5, 1, 0.85, 0),     # more units than run at once
 ])
-@pytest.mark.parametrize("row_major", [0, 1])
-@pytest.mark.parametrize("waves", [3, 4])
-def test_two_waves_per_tile_row_at_64_tokens(spmm, oracle, M, K, split_k, sparsity, flags, row_major, waves):
-    """The row-sharing layout at 64 tokens with two waves to each tile row where its rule takes it (and the one-wave kernel
-    beside it): against the oracle, and against the same launch with activations that begin at an odd element,
-    which the one-wave kernel takes; a tile without words hides what the activations hold there."""
+@pytest.mark.parametrize("rows,row_major", [(3, 0), (3, 1), (4, 1)])
+def test_two_waves_per_tile_row_at_64_tokens(spmm, oracle, M, K, split_k, sparsity, flags, rows, row_major):
+    """Two waves to each of three or four tile rows (StageB = 4): against the oracle, and against one wave to a tile row
+    (StageB = 0); a tile without words hides what the activations hold there.  With activations that begin at an odd element the
+    shape is refused, and what a planned call does instead is one wave to a tile row, bit for bit."""
     torch = _torch()
     N, dev = 64, torch.device("cuda:0")
     if sparsity == "mixed":
@@ -1184,24 +1187,107 @@ def test_two_waves_per_tile_row_at_64_tokens(spmm, oracle, M, K, split_k, sparsi
         d_B = d_B.t().contiguous()
     odd = torch.empty(N * K + 8, dtype=torch.float16, device=dev)[1:1 + N * K].view(d_B.shape)
     odd.copy_(d_B)
-    print(f"[gpu case] halves M={M} K={K} split_k={split_k} sparsity={sparsity} flags={flags} row_major={row_major} waves={waves}", flush=True)
-    got = []
-    for b in (d_B, odd):
+
+    def call(b, stage_b, more=0):
         C = torch.full((M, N) if row_major else (N, M), float("nan"), dtype=torch.float16, device=dev)
-        spmm.SpMM_SplitK_API_Planned(torch.cuda.current_stream(), d_items, d_offs, b, C, M, N, K, d_W, split_k, 0, waves, 0, row_major, flags)
+        print(f"[gpu case] halves M={M} K={K} split_k={split_k} sparsity={sparsity} flags={flags | more} row_major={row_major} rows={rows} stage_b={stage_b}", flush=True)
+        spmm.SpMM_SplitK_API_Planned(torch.cuda.current_stream(), d_items, d_offs, b, C, M, N, K, d_W, split_k, 0, rows, stage_b, row_major, flags | more)
         torch.cuda.synchronize()
-        got.append((C.t() if row_major else C).cpu().numpy())
-        assert_close(got[-1], ref)
+        return (C.t() if row_major else C).cpu().numpy()
+
+    two, one = call(d_B, 4), call(d_B, 0)
+    for got in (two, one):
+        assert_close(got, ref)
     # the two differ in the order of fp32 sums, in one rounding of a slab and one of the result: two units in the last place of
     # what a slab can be
     size = np.abs(A.astype(np.float32))
     bound = 2.0 ** -10 * (np.abs(np.nan_to_num(B.astype(np.float32), posinf=0.0)) @ size.T) + 2.0 ** -24
-    assert (np.abs(got[0].astype(np.float32) - got[1].astype(np.float32)) <= bound).all()
+    assert (np.abs(two.astype(np.float32) - one.astype(np.float32)) <= bound).all()
+    planned = call(d_B, 0, spmm.SPMM_FLAG_ADAPTIVE_WAVES)
+    tiles = -(-(K // 64) // split_k)
+    assert np.array_equal(planned.view(np.uint16), (two if tiles >= (4 if rows == 3 else 20) else one).view(np.uint16))
+    with pytest.raises(spmm.SpMMError):
+        call(odd, 4)
+    assert np.array_equal(call(odd, 0, spmm.SPMM_FLAG_ADAPTIVE_WAVES).view(np.uint16), one.view(np.uint16))
+
+
+@pytest.mark.parametrize("M,K,split_k,sparsity,flags", [
+    (128 * 513, 64 * 4, 1, 0.8, 0), (128 * 514, 64 * 5, 1, 0.6, 1),  # the kernel writes C
+    (128 * 257, 64 * 7, 2, 0.9, 1), (128 * 172, 64 * 10, 3, 0.7, 0),  # slabs, the last batch shorter
+])
+def test_planned_calls_with_two_waves_per_tile_row(spmm, oracle, M, K, split_k, sparsity, flags):
+    """Calls that the planner gives two waves to a tile row, on strided operands: the bits of that launch shape on dense
+    ones, and of one wave to a tile row where B is not aligned (the two do differ here); nothing is written between the
+    vectors of C.  Forms that the shape does not have are refused."""
+    torch = _torch()
+    N, dev = 64, torch.device("cuda:0")
+    p = spmm.SpMM_PlanLaunch(M, N, K, split_k)
+    assert (p["mode"], p["waves"], p["stage_b"], p["lds_bytes"], p["two_per_row"]) == (0, 3, 0, 163840, True)
+    A, B, items, offsets = make_case(spmm, M, K, N, sparsity, seed=K)
+    d_items = torch.from_numpy(items.view(np.int32).copy()).to(dev)
+    d_offs = torch.from_numpy(offsets.copy()).to(dev)
+    d_W = torch.full((split_k, N, M), float("nan"), dtype=torch.float16, device=dev)
+    d_B = torch.from_numpy(np.ascontiguousarray(B).view(np.int16).copy()).to(dev).view(torch.float16)
+    ldb, ldc = K + 72, M + 24
+    stream = torch.cuda.current_stream()
+
+    def strided(begin):
+        wide = torch.full((N * ldb + 16,), float("nan"), dtype=torch.float16, device=dev)[begin:begin + N * ldb].view(N, ldb)
+        wide[:, :K] = d_B
+        C = torch.full((N, ldc), float("nan"), dtype=torch.float16, device=dev)
+        print(f"[gpu case] planned halves M={M} K={K} split_k={split_k} begin={begin}", flush=True)
+        spmm.SpMM_SplitK_API_Strided(stream, d_items, d_offs, wide, ldb, C, ldc, M, N, K, d_W, split_k, flags)
+        torch.cuda.synchronize()
+        assert torch.isnan(C[:, M:]).all()
+        return C[:, :M].contiguous()
+
+    def planned(waves, stage_b, row_major=0, n=N):
+        C = torch.full((N, M), float("nan"), dtype=torch.float16, device=dev)
+        print(f"[gpu case] ... plan {waves} {stage_b} {row_major}", flush=True)
+        spmm.SpMM_SplitK_API_Planned(stream, d_items, d_offs, d_B, C, M, n, K, d_W, split_k, 0, waves, stage_b, row_major, flags)
+        torch.cuda.synchronize()
+        return C
+
+    two, one = planned(3, 4), planned(3, 0)
+    assert not torch.equal(two, one)
+    assert torch.equal(strided(0), two) and torch.equal(strided(8), two) and torch.equal(strided(1), one)
+    ref = oracle.gemm_f32(A, B)
+    assert_close(two.cpu().numpy(), np.maximum(ref, 0) if flags & 1 else ref)
+    for waves, stage_b, row_major, n in ((4, 4, 0, N), (2, 4, 0, N), (2, 4, 1, N), (1, 4, 1, N), (3, 4, 0, 32), (3, 5, 0, N), (3, 5, 1, N)):
+        with pytest.raises(spmm.SpMMError):
+            planned(waves, stage_b, row_major, n)
+
+
+def test_row_major_calls_with_two_waves_per_tile_row(spmm):
+    """The row-major call that takes four tile rows of two waves each (36864 x 9216 in three batches), and three rows
+    (49152 x 12288 in two): the bits of those launch shapes."""
+    torch = _torch()
+    N, dev = 64, torch.device("cuda:0")
+    stream = torch.cuda.current_stream()
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(3)
+    for M, K, split_k, rows in ((36864, 9216, 3, 4), (49152, 12288, 2, 3)):
+        W = torch.randn((M, K), generator=gen, device=dev, dtype=torch.float16)
+        W *= torch.rand((M, K), generator=gen, device=dev, dtype=torch.float16) < 0.1
+        items, offsets = spmm.encode_on_device(W)
+        del W
+        B = torch.randn((K, N), generator=gen, device=dev, dtype=torch.float16)
+        ws = torch.empty((split_k, M, N), dtype=torch.float16, device=dev)
+        C = torch.full((M, N), float("nan"), dtype=torch.float16, device=dev)
+        print(f"[gpu case] row-major halves M={M} K={K} split_k={split_k}", flush=True)
+        spmm.SpMM_SplitK_API_RowMajor(stream, None, items, offsets, B, C, M, N, K, ws, split_k)
+        got = []
+        for stage_b in (4, 0):
+            D = torch.full((M, N), float("nan"), dtype=torch.float16, device=dev)
+            spmm.SpMM_SplitK_API_Planned(stream, items, offsets, B, D, M, N, K, ws, split_k, 0, rows, stage_b, 1, 0)
+            torch.cuda.synchronize()
+            got.append(D)
+        assert torch.isfinite(C).all() and torch.equal(C, got[0]) and not torch.equal(C, got[1])
 
 
 @pytest.mark.parametrize("row_major", [0, 1])
 @pytest.mark.parametrize("waves,tiles,split_k", [(1, 2, 1), (2, 1, 1), (2, 3, 2), (3, 2, 1), (3, 7, 1), (4, 1, 1), (4, 2, 1),
-                                                 (4, 3, 1), (4, 16, 3)])
+                                                 (4, 3, 1), (4, 16, 3), (4, 4, 3), (3, 1, 2)])  # the last two: an empty batch
 def test_final_sum_at_64_tokens_of_every_wave_count(spmm, waves, tiles, split_k, row_major):
     """The K-splitting layout's final sum in groups of cells: wave counts that divide the cells and that do not, fewer tiles
     than waves. Whole numbers, so that every sum is exact: |a| <= 2, |b| <= 3 at 0.9 sparsity stay below 2048."""

@@ -199,6 +199,30 @@ def test_planner_pairs_waves_only_where_that_is_faster(spmm):
         assert paired(M, K, S), (M, K, S)
 
 
+def test_planner_says_where_two_waves_take_a_tile_row(spmm):
+    """64 tokens, three tile rows to a workgroup and batches of four tiles or more: two waves to each row, all of the compute
+    unit's LDS; batches of three tiles and other token counts keep one wave to a row.  The tuner times the form that a
+    row's call does not take as well, and writes no row for it."""
+    from graphneuralnetproj_amd import tune_plans
+
+    def two(M, K, S, N=64):
+        p = spmm.SpMM_PlanLaunch(M, N, K, S)
+        assert not p["two_per_row"] or (p["mode"], p["waves"], p["stage_b"], p["lds_bytes"], p["paired"]) == (0, 3, 0, 163840, False)
+        return p["two_per_row"]
+
+    assert two(49152, 12288, 2) and two(128 * 513, 256, 1) and two(128 * 257, 64 * 7, 2) and two(128 * 2246, 64 * 165, 1)
+    for M, K, S, N in ((128 * 513, 192, 1, 64), (36864, 9216, 3, 64), (28672, 7168, 1, 64), (49152, 12288, 2, 32), (49152, 12288, 2, 16)):
+        assert not two(M, K, S, N), (M, K, S, N)
+    assert spmm.SpMM_PlanLaunch(128 * 513, 64, 192, 1)["lds_bytes"] < 163840
+    for only in (None, [2]):
+        assert (2, 0, 3, tune_plans.ONE_PER_ROW) in tune_plans.candidate_plans(64, 7, only)
+        assert (2, 0, 3, tune_plans.TWO_PER_ROW) in tune_plans.candidate_plans(64, 6, only)
+    assert tune_plans.planned_args((2, 0, 3, tune_plans.ONE_PER_ROW)) == (2, 0, 3, 0, 0)
+    assert tune_plans.planned_args((2, 0, 3, tune_plans.TWO_PER_ROW))[:4] == (2, 0, 3, 4)
+    results = [(9.0, (2, 0, 3, tune_plans.ONE_PER_ROW)), (9.5, (2, 0, 3, 0))]
+    assert tune_plans.best_row(49152, 12288, 64, results).lstrip().startswith("{49152, 12288, 64, 2, 0, 3, 0},  // 9.5 us")
+
+
 def test_planner_uses_every_compute_unit_on_the_headline_shapes(spmm):
     # one round of workgroups, at least 200 of them, for the big OPT layers at N = 16
     for (M, K) in [(28672, 7168), (7168, 28672), (36864, 9216), (9216, 36864)]:
