@@ -272,7 +272,7 @@ constexpr long kManyFrom = 16384;
 //
 // For a list of at most four rounds a word's place in code is one byte, (room - 1) * 4 + (3 - round); for longer
 // lists the place is written as two bytes.  (Three more bytes: what a lap writes beyond its own words.)
-__device__ __forceinline__ int place_bytes(int n)
+__device__ __forceinline__ constexpr int place_bytes(int n)
 {
     return n <= 256 ? n + 3 : 2 * n;
 }
@@ -391,8 +391,8 @@ __global__ __launch_bounds__(kEmitWaves * 64, 8) void a24_residual_emit_kernel(c
                                                                                uint32_t* __restrict__ words)
 {
     constexpr int kListsPerWave = kEmitLists / kEmitWaves;
-    constexpr int kPlaces = kEmitLists * 256 > 2 * kMaxListWords ? kEmitLists * 256 : 2 * kMaxListWords;  // bytes: lists of 256 words (an ordinary residual has up to 200) are dealt in one pass
-    static_assert(kPlaces >= 2 * kMaxListWords, "the longest list has to fit");
+    constexpr int kPlaces = kEmitLists * place_bytes(256);  // lists of 256 words (an ordinary residual has up to 200) are dealt in one pass
+    static_assert(kPlaces >= place_bytes(kMaxListWords), "the longest list has to fit");
     __shared__ unsigned images[kEmitWaves][16 * 64];  // per wave: a list's block, [row][bank] column pairs
     __shared__ unsigned sorted[kEmitLists][17];      // counts of a list's banks, one byte each, largest first
     __shared__ int length[kEmitLists];
