@@ -257,7 +257,8 @@ __global__ __launch_bounds__(offscan::kThreads) void a24_residual_scan_kernel(in
 // lane at its own bank, 110; with 16 lists 99).  A list of at most 64 words stays in row-major order, as the host leaves it.
 //
 // The residual is read a second time for the writing (from the last-level cache) instead of kept in
-// registers: more workgroups per compute unit, whose dealing waves hide each other.
+// registers: more workgroups per compute unit, whose dealing waves hide each other.  Seven of 16 lists: 64 vector registers and
+// 96 scalar ones are the most a wave may have (with 97, six: 7168 x 7168, 70 words a list, 34 us -> 43).
 constexpr int kEmitWaves = 4;
 // Lists per workgroup: the lists of a wave follow one another and the others wait while one wave deals, so few lists
 // are better spread over more waves, and many are better dealt 16 at a time (whole calls at 50 / 60 / 95 %:
@@ -391,33 +392,37 @@ __global__ __launch_bounds__(kEmitWaves * 64, 8) void a24_residual_emit_kernel(c
                                                                                uint32_t* __restrict__ words)
 {
     constexpr int kListsPerWave = kEmitLists / kEmitWaves;
-    constexpr int kPlaces = kEmitLists * place_bytes(256);  // lists of 256 words (an ordinary residual has up to 200) are dealt in one pass
+    constexpr int kPlaces = kEmitLists * place_bytes(256);  // bytes: lists of 256 words (an ordinary residual has up to 200) are dealt in one pass
+    constexpr int kImages = kEmitWaves * 16 * 64 * 4;  // bytes, per wave: a list's block, [row][bank] column pairs
     static_assert(kPlaces >= place_bytes(kMaxListWords), "the longest list has to fit");
-    __shared__ unsigned images[kEmitWaves][16 * 64];  // per wave: a list's block, [row][bank] column pairs
+    __shared__ __attribute__((aligned(16))) uint8_t room[kImages + kPlaces];  // the places, then the images
     __shared__ unsigned sorted[kEmitLists][17];      // counts of a list's banks, one byte each, largest first
     __shared__ int length[kEmitLists];
-    __shared__ uint8_t places[kPlaces];
     const int L = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int total = offsets[lists];
     if (total < 0)  // the word count did not fit an int: no offset of this table means anything, nothing is written
         return;
     if (blockIdx.x == 0 && w == 0)  // the padding behind the last list
         words[(size_t)total + L] = 0;
-    unsigned* const image = images[w];
+    uint8_t* const places = room;
+    unsigned* const image = reinterpret_cast<unsigned*>(room + kPlaces) + w * (16 * 64);
 
     // wave w takes the workgroup's lists w, w + 4, ...
     auto list_of = [&](int i) { return (long)blockIdx.x * kEmitLists + i * kEmitWaves + w; };
-    auto load_list = [&](long list, unsigned (&pairs)[16]) {
+    auto block_of = [&](long list) {
         const unsigned unit_row = static_cast<unsigned>(list / kGroupBlocks);  // (128-row group, unit)
         const unsigned group = unit_row / units, u = unit_row % units;
-        size_t block = ((size_t)group * kGroupBlocks + list % kGroupBlocks) * 16 * K + (size_t)u * 128;
+        return A2 + (((size_t)group * kGroupBlocks + list % kGroupBlocks) * 16 * K + (size_t)u * 128);
+    };
+    // (in the global address space by name: the compiler does not see that through the asm below)
+    auto load_list = [&](long list, unsigned (&pairs)[16]) {
+        auto* src = (const __attribute__((address_space(1))) uint16_t*)block_of(list);
         int lane = L;
         // (opaque: else the compiler issues the loads of all lists ahead of the first one's use, 300 registers)
-        asm volatile("" : "+s"(block), "+v"(lane)::"memory");
-        const uint16_t* src = A2 + block;
+        asm volatile("" : "+s"(src), "+v"(lane)::"memory");
 #pragma unroll
         for (int r = 0; r < 16; r++)
-            pairs[r] = *reinterpret_cast<const unsigned*>(src + (size_t)r * K + 2 * (lane ^ (r << 2)));
+            pairs[r] = *(const __attribute__((address_space(1))) unsigned*)(src + (size_t)r * K + 2 * (lane ^ (r << 2)));
     };
     unsigned kept[kListsPerWave];  // bit 2 r + h: element h of row r's pair
     int start[kListsPerWave];      // where the bank's words begin in the bank-sorted sequence
@@ -495,11 +500,15 @@ __global__ __launch_bounds__(kEmitWaves * 64, 8) void a24_residual_emit_kernel(c
     }
     __syncthreads();
 
-    // 2. deal as many of the lists as there is room for (all of them, but for very dense ones), 3. write them
+    // 2. deal as many of the lists as there is room for (all of them, but for very dense ones), 3. write them.  With a list of
+    // more than 256 words among them the images' room is the places' as well (ten lists of 1024 words), and values come from
+    // memory one by one: a pass costs as much as its longest list, so what counts is how few there are (21504 x 7168, 300 / 700
+    // words a list: 921 / 4834 us with the places' own room, 357 / 1265 with both; with 32 lists to a workgroup 660 / 3030).
     const int mine = L < kEmitLists ? length[L] : 0;
     const int through = offscan::wave_inclusive_sum(mine > 0 ? place_bytes(mine) : 0);  // room for lists 0 .. L
+    const int more = __any(mine > 256) ? kImages : 0;  // bytes of the images' room that are the places'
     for (int first = 0, dealt = 0; first < kEmitLists;) {
-        const uint64_t fit = __ballot(L < kEmitLists && through - dealt <= kPlaces);  // 0 .. last - 1: totals only grow
+        const uint64_t fit = __ballot(L < kEmitLists && through - dealt <= kPlaces + more);  // 0 .. last - 1: totals only grow
         const int last = __popcll(fit);
         const int at = through - place_bytes(mine) - dealt;
         if (w == 0 && L >= first && L < last && mine > 0) {
@@ -520,16 +529,27 @@ __global__ __launch_bounds__(kEmitWaves * 64, 8) void a24_residual_emit_kernel(c
             const int n = __builtin_amdgcn_readlane(mine, li);
             if (li < first || li >= last || n == 0)
                 continue;
-            unsigned pairs[16];
-            load_list(list_of(i), pairs);
             const uint8_t* const list_places = places + __builtin_amdgcn_readlane(at, li);
             uint32_t* const out = words + (size_t)offsets[list_of(i)];
             const unsigned ends = round_ends(n);
+            int p = start[i];
+            if (more) {
+                const uint16_t* const src = block_of(list_of(i));
+                unsigned lane = L;
+                asm volatile("" : "+v"(lane));  // (or what is made of it is kept in registers from list to list)
+                for (unsigned mask = kept[i]; mask; mask &= mask - 1, p++) {
+                    const unsigned e = __builtin_ctz(mask), r = e / 2;
+                    const unsigned value = src[(size_t)r * K + 2 * (lane ^ (r << 2)) + e % 2];
+                    out[static_cast<unsigned>(place_of(list_places, p, n, ends))] = value | (e * 130u & 0xf02u) << 16 | lane << 18;
+                }
+                continue;
+            }
+            unsigned pairs[16];
+            load_list(list_of(i), pairs);
 #pragma unroll
             for (int r = 0; r < 16; r++)
                 image[r * 64 + L] = pairs[r];
             asm volatile("" ::: "memory");
-            int p = start[i];
             for (unsigned mask = kept[i]; mask; mask &= mask - 1, p++) {
                 const unsigned e = __builtin_ctz(mask);
                 const unsigned address = (e * 130u & 0xf02u) | L * 4;  // (e / 2) * 256 + (e % 2) * 2: here as in the product's own image

@@ -1066,3 +1066,29 @@ def test_device_residual_lists_of_uneven_banks(spmm, oracle, M, K):
     assert longest == want_longest
     assert np.array_equal(offs.cpu().numpy(), want_offs)
     assert np.array_equal(words.cpu().numpy().view(np.uint32), want_words)
+
+
+@pytest.mark.parametrize("M,K", [(256, 1280), (4224, 8192)])  # eight lists to a workgroup, and 16
+@pytest.mark.parametrize("lengths", [(257,), (700,), (1024,), (1024, 1024, 40, 256, 1024, 0, 1023, 257, 65), (512, 200, 129)])
+def test_device_residual_lists_of_many_words(spmm, M, K, lengths):
+    """Workgroups with lists of more than 256 words: more of them than their places have room for at once, and beside
+    lists of every other kind; the host's words, bit for bit."""
+    torch = _torch()
+    rng = np.random.default_rng(sum(lengths))
+    lists = M // 16 * (K // 128)
+    most = np.flatnonzero(np.arange(2048) % 4 >= 2)  # what a split leaves: at most two of every four
+    blocks = np.zeros((lists, 2048), dtype=np.uint16)
+    for i in range(lists):
+        n = lengths[i % len(lengths)]
+        blocks[i, rng.permutation(most)[:n] if n < 1024 else most] = rng.integers(1, 0x7C00, size=n)
+    # lists are numbered ((16-row block / 8) * units + unit) * 8 + block % 8
+    A2 = blocks.reshape(M // 128, K // 128, 8, 16, 128).transpose(0, 2, 3, 1, 4).reshape(M, K)
+    A2 = np.ascontiguousarray(A2).view(np.float16)
+    want_words, want_offs, want_longest = spmm.HeteroSparse_PackA2(A2)
+    assert np.array_equal(np.diff(want_offs), np.resize(lengths, lists))
+    d_A2 = torch.from_numpy(A2.view(np.int16).copy()).to("cuda:0").view(torch.float16)
+    print(f"[gpu case] residual lists of many words M={M} K={K} lengths={lengths}", flush=True)
+    words, offs, longest = spmm.pack_residual_on_device(d_A2)
+    torch.cuda.synchronize()
+    assert longest == want_longest and np.array_equal(offs.cpu().numpy(), want_offs)
+    assert np.array_equal(words.cpu().numpy().view(np.uint32), want_words)
