@@ -402,11 +402,17 @@ __device__ __forceinline__ void shared_b_product(const uint8_t* __restrict__ pac
     // rounds of such a list are fetched when the unit's turn comes, ahead of the loads that the
     // same phase issues for the unit two further on, and awaited with the count of just those
     // loads; whatever a list holds beyond that comes through ordinary loads inside the
-    // multiplication, which wait for everything in flight.  Extra loads never invalidate the
-    // constant waits elsewhere: a wait that allows N loads to stay outstanding covers the loads it
-    // is meant for however many younger ones there are.
+    // multiplication, three rounds at a time, which wait for everything in flight.  Extra loads never
+    // invalidate the constant waits elsewhere: a wait that allows N loads to stay outstanding covers the
+    // loads it is meant for however many younger ones there are.
+    // One wave with longer lists than the others holds all of them up at the next barrier, so up to 32 tokens, where a unit
+    // has little else to do, EX covers 640 words (the longest lists of a 50 % sparse weight with uneven rows), and the other
+    // waves do not send their next unit's loads ahead of it (the pipeline below, STRAIGHT).  1664 x 37760 at 50 %, uneven rows,
+    // 16 tokens: 60.8 us, now 50.8, through registers before either 56.3; 28672 x 7168 at 60 % 69.2, 66.1, 75.0.  At 64 tokens
+    // neither pays (21504 x 7168 at 50 %: 60.9 us, 65.8 with both).
     constexpr bool kLong = RL == 5;
-    constexpr int EX = 3;
+    constexpr int EX = NT <= 2 ? 5 : 3;
+    constexpr bool kBarrierFirst = kLong && NT <= 2;
     constexpr int kLoadsUnit = kLoadsHead + CH + kLoadsA;  // what issue_unit puts in flight
     unsigned ex[RB][EX] = {};
     auto any_longer = [&](const UnitRegs& x) __attribute__((always_inline)) {
@@ -539,8 +545,7 @@ __device__ __forceinline__ void shared_b_product(const uint8_t* __restrict__ pac
                             *reinterpret_cast<unsigned short*>(image + (x.w[r][i] >> 16)) = static_cast<unsigned short>(x.w[r][i]);
                     // A list longer than the RL rounds that travel with the unit: EX more rounds
                     // have just landed (above); the rest is fetched here, with ordinary loads,
-                    // which wait for everything this wave has in flight (a stall per round, for
-                    // lists of more than 512 words only).
+                    // which wait for everything this wave has in flight (a stall per three rounds).
                     const bool longer = kLong && n > RL * kWave;
                     if constexpr (kLong) {
                         if (longer) {
@@ -555,10 +560,17 @@ __device__ __forceinline__ void shared_b_product(const uint8_t* __restrict__ pac
                             for (int i = 0; i < EX; i++)
                                 if (n > (RL + i) * kWave)
                                     *reinterpret_cast<unsigned short*>(image + (ex[r][i] >> 16)) = static_cast<unsigned short>(ex[r][i]);
-                            for (int at0 = (RL + EX) * kWave; at0 < n; at0 += kWave) {
-                                const int at = at0 + lane;
-                                const unsigned w = words[x.start[r] + (at < n ? at : n - 1)];
-                                *reinterpret_cast<unsigned short*>(image + (w >> 16)) = static_cast<unsigned short>(w);
+#pragma unroll 1
+                            for (int at0 = (RL + EX) * kWave; at0 < n; at0 += 3 * kWave) {
+                                unsigned rest[3];
+#pragma unroll
+                                for (int i = 0; i < 3; i++) {
+                                    const int at = at0 + i * kWave + lane;
+                                    rest[i] = words[x.start[r] + (at < n ? at : n - 1)];
+                                }
+#pragma unroll
+                                for (int i = 0; i < 3; i++)
+                                    *reinterpret_cast<unsigned short*>(image + (rest[i] >> 16)) = static_cast<unsigned short>(rest[i]);
                             }
                         }
                     }
@@ -626,7 +638,7 @@ __device__ __forceinline__ void shared_b_product(const uint8_t* __restrict__ pac
     // STRAIGHT: a unit's tile loads come last, two units ahead like its records, but behind the phase's barrier:
     //   in flight at the top        records(u), tile(u), [offsets(u+2),] records(u+1), tile(u+1)
     //   wait until kLoadsA + CH stay   -> records(u), offsets(u+2) and this wave's share of tile(u) have landed
-    //   issue [offsets(u+3),] records(u+2); barrier; issue tile(u+2); multiply unit u
+    //   issue [offsets(u+3),] records(u+2); barrier (kBarrierFirst: ahead of those loads); issue tile(u+2); multiply unit u
     // Behind the barrier every wave's share of tile(u) is there and nobody reads tile(u-1) any more, whose buffer
     // tile(u+2) goes to.  (The first phase's queue has tile(u) and tile(u+1) ahead of both units' words.)
     UnitRegs x[3];
@@ -682,9 +694,12 @@ __device__ __forceinline__ void shared_b_product(const uint8_t* __restrict__ pac
             store_b(x[(k + 1) % 3], buf ^ 1);
             int o2[RB + 1] = {};
             offsets_from(x[(k + 1) % 3], o2);  // unit u + 1 brought the offsets of unit u + 2
+            if constexpr (STRAIGHT && kBarrierFirst)
+                __syncthreads();
             issue_unit(x[(k + 2) % 3], ahead(2), ahead(3), o2);
             if constexpr (STRAIGHT) {
-                __syncthreads();
+                if constexpr (!kBarrierFirst)
+                    __syncthreads();
                 issue_tile(ahead(2), (k + 2) % 3);
             }
             multiply_from(x[k], buf);

@@ -956,6 +956,7 @@ def test_device_residual_lists_with_offsets_of_another_matrix(spmm, M, K):
 @pytest.mark.parametrize("M,K,split_k,sparsity", [
     (128, 128, 1, 0.5), (128, 256, 1, 0.95), (256, 384, 1, 0.3), (384, 512, 1, 0.6),  # one to four units: the pipeline's ends
     (256, 640, 2, 0.7), (128, 1792, 3, 0.55),                                         # batches of unequal length
+    (256, 1152, 2, 0.2), (384, 768, 1, 0.0), (256, 1408, 1, "uneven"),                # lists beyond what travels with a unit
     (5632, 1024, 8, 0.5), (10752, 512, 4, 0.45), (10752, 896, 7, 0.8),                # eight waves; four where eight do not run at once
 ])
 def test_activations_straight_into_lds(spmm, oracle, N, M, K, split_k, sparsity):
@@ -966,9 +967,17 @@ def test_activations_straight_into_lds(spmm, oracle, N, M, K, split_k, sparsity)
     gen = torch.Generator(device="cuda:0")
     gen.manual_seed(M + K + N)
     W = torch.randn((M, K), generator=gen, device="cuda:0") * 0.02
-    W = (W * (torch.rand((M, K), generator=gen, device="cuda:0") >= sparsity)).half()
+    keep = torch.rand((M, K), generator=gen, device="cuda:0")
+    if sparsity == "uneven":  # each 16 x 128 block of a density of its own, one of 32 dense: a wave at a time has a long list
+        density = torch.rand((M // 16, K // 128), generator=gen, device="cuda:0")
+        density = torch.where(torch.rand(density.shape, generator=gen, device="cuda:0") < 1 / 32, torch.ones_like(density), density)
+        keep = keep >= 1 - density.repeat_interleave(16, 0).repeat_interleave(128, 1)
+    else:
+        keep = keep >= sparsity
+    W = (W * keep).half()
     packed, residual = spmm.split_pack_on_device(W)
     words, offsets, longest = spmm.pack_residual_on_device(residual)
+    assert longest > 640 or sparsity not in (0.2, 0.0, "uneven")
     ldb = K + 72
     B = torch.randn((N, ldb), generator=gen, device="cuda:0").half()
     odd = torch.empty(N * ldb + 8, dtype=torch.float16, device="cuda:0")[1:1 + N * ldb].view(N, ldb)
