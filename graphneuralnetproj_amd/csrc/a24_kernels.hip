@@ -275,7 +275,7 @@ constexpr int kImageBytes = 4096;
 // hands lane i of a group of sixteen the i-th column of a 4 x 16 block whose rows the sixteen lanes
 // address four to a row: two such reads give a lane the eight consecutive k of its token that the
 // matrix instructions want.
-template<int NT, int RB, int W, int RL, bool RM, bool STRAIGHT>
+template<int NT, int RB, int W, int RL, bool RM, bool STRAIGHT, int EX = 3>
 __device__ __forceinline__ void shared_b_product(const uint8_t* __restrict__ packed, const _Float16* __restrict__ B,
                                                  _Float16* __restrict__ out, int units, int units_per_batch, long ldb, long ldo,
                                                  long slab, int n_tokens, const unsigned* __restrict__ words,
@@ -402,17 +402,17 @@ __device__ __forceinline__ void shared_b_product(const uint8_t* __restrict__ pac
     // rounds of such a list are fetched when the unit's turn comes, ahead of the loads that the
     // same phase issues for the unit two further on, and awaited with the count of just those
     // loads; whatever a list holds beyond that comes through ordinary loads inside the
-    // multiplication, three rounds at a time, which wait for everything in flight.  Extra loads never
+    // multiplication, which wait for everything in flight (STRAIGHT: three rounds at a time).  Extra loads never
     // invalidate the constant waits elsewhere: a wait that allows N loads to stay outstanding covers the
     // loads it is meant for however many younger ones there are.
-    // One wave with longer lists than the others holds all of them up at the next barrier, so up to 32 tokens, where a unit
-    // has little else to do, EX covers 640 words (the longest lists of a 50 % sparse weight with uneven rows), and the other
-    // waves do not send their next unit's loads ahead of it (the pipeline below, STRAIGHT).  1664 x 37760 at 50 %, uneven rows,
-    // 16 tokens: 60.8 us, now 50.8, through registers before either 56.3; 28672 x 7168 at 60 % 69.2, 66.1, 75.0.  At 64 tokens
-    // neither pays (21504 x 7168 at 50 %: 60.9 us, 65.8 with both).
+    // STRAIGHT: one wave with longer lists than the others holds all of them up at the next barrier, so up to 32 tokens, where a
+    // unit has little else to do, the other waves do not send their next unit's loads ahead of it (kBarrierFirst), and EX is
+    // five where lists exceed 512 words (launch_shared_b_nt).  1664 x 37760 at 50 %, uneven rows, 16 tokens: 60.8 us, now 50.8,
+    // through registers 56.3; 28672 x 7168 at 60 %, uneven rows (up to 427 words): 69.2, 64.9, 75.0.  At 64 tokens neither pays
+    // (21504 x 7168 at 50 %: 60.9 us, 65.8 with both), nor more rounds through registers (7296 x 15488 at 40 %, 8 tokens, up
+    // to 374 words: 45.8, with five 50.6).
     constexpr bool kLong = RL == 5;
-    constexpr int EX = NT <= 2 ? 5 : 3;
-    constexpr bool kBarrierFirst = kLong && NT <= 2;
+    constexpr bool kBarrierFirst = STRAIGHT && kLong && NT <= 2;
     constexpr int kLoadsUnit = kLoadsHead + CH + kLoadsA;  // what issue_unit puts in flight
     unsigned ex[RB][EX] = {};
     auto any_longer = [&](const UnitRegs& x) __attribute__((always_inline)) {
@@ -545,7 +545,7 @@ __device__ __forceinline__ void shared_b_product(const uint8_t* __restrict__ pac
                             *reinterpret_cast<unsigned short*>(image + (x.w[r][i] >> 16)) = static_cast<unsigned short>(x.w[r][i]);
                     // A list longer than the RL rounds that travel with the unit: EX more rounds
                     // have just landed (above); the rest is fetched here, with ordinary loads,
-                    // which wait for everything this wave has in flight (a stall per three rounds).
+                    // which wait for everything this wave has in flight (a stall per trip).
                     const bool longer = kLong && n > RL * kWave;
                     if constexpr (kLong) {
                         if (longer) {
@@ -560,17 +560,24 @@ __device__ __forceinline__ void shared_b_product(const uint8_t* __restrict__ pac
                             for (int i = 0; i < EX; i++)
                                 if (n > (RL + i) * kWave)
                                     *reinterpret_cast<unsigned short*>(image + (ex[r][i] >> 16)) = static_cast<unsigned short>(ex[r][i]);
-#pragma unroll 1
-                            for (int at0 = (RL + EX) * kWave; at0 < n; at0 += 3 * kWave) {
-                                unsigned rest[3];
+                            auto fetch = [&](int at0, auto rounds) __attribute__((always_inline)) {
+                                unsigned rest[decltype(rounds)::value];
 #pragma unroll
-                                for (int i = 0; i < 3; i++) {
+                                for (int i = 0; i < decltype(rounds)::value; i++) {
                                     const int at = at0 + i * kWave + lane;
                                     rest[i] = words[x.start[r] + (at < n ? at : n - 1)];
                                 }
 #pragma unroll
-                                for (int i = 0; i < 3; i++)
+                                for (int i = 0; i < decltype(rounds)::value; i++)
                                     *reinterpret_cast<unsigned short*>(image + (rest[i] >> 16)) = static_cast<unsigned short>(rest[i]);
+                            };
+                            if constexpr (STRAIGHT) {
+#pragma unroll 1
+                                for (int at0 = (RL + EX) * kWave; at0 < n; at0 += 3 * kWave)
+                                    fetch(at0, std::integral_constant<int, 3>{});
+                            } else {
+                                for (int at0 = (RL + EX) * kWave; at0 < n; at0 += kWave)
+                                    fetch(at0, std::integral_constant<int, 1>{});
                             }
                         }
                     }
@@ -694,7 +701,7 @@ __device__ __forceinline__ void shared_b_product(const uint8_t* __restrict__ pac
             store_b(x[(k + 1) % 3], buf ^ 1);
             int o2[RB + 1] = {};
             offsets_from(x[(k + 1) % 3], o2);  // unit u + 1 brought the offsets of unit u + 2
-            if constexpr (STRAIGHT && kBarrierFirst)
+            if constexpr (kBarrierFirst)
                 __syncthreads();
             issue_unit(x[(k + 2) % 3], ahead(2), ahead(3), o2);
             if constexpr (STRAIGHT) {
@@ -802,10 +809,15 @@ __global__ __launch_bounds__(W* kWave) void a24_spmm_straight_b_kernel(A24_PARAM
 {
     shared_b_product<NT, RB, W, RL, RM, true>(A24_ARGS);
 }
+template<int NT, int RB, int W, bool RM>  // lists of more than 512 words
+__global__ __launch_bounds__(W* kWave) void a24_spmm_straight_long_kernel(A24_PARAMS)
+{
+    shared_b_product<NT, RB, W, 5, RM, true, 5>(A24_ARGS);
+}
 #undef A24_ARGS
 #undef A24_PARAMS
 
-template<int NT, int RB, int W, int RL, bool RM, bool STRAIGHT = false>
+template<int NT, int RB, int W, int RL, bool RM, bool STRAIGHT = false, bool LONG = false>
 int launch_shared_b(hipStream_t stream, const void* packed, const void* B, void* out, int M, int N, int K, int split_k,
                     long ldb, long ldo, long slab, const void* words, const void* offsets, int relu, void* fused_out,
                     unsigned int* arrivals, long ldc)
@@ -816,7 +828,9 @@ int launch_shared_b(hipStream_t stream, const void* packed, const void* B, void*
         return static_cast<int>(hipErrorInvalidValue);
     const unsigned lds = (STRAIGHT ? 3 * NT * 16 * 256 : 2 * NT * 16 * kRowBytes) + (RL > 0 ? W * kImageBytes : 0);
     auto* const kern = [] {
-        if constexpr (STRAIGHT)
+        if constexpr (LONG)
+            return a24_spmm_straight_long_kernel<NT, RB, W, RM>;
+        else if constexpr (STRAIGHT)
             return a24_spmm_straight_b_kernel<NT, RB, W, RL, RM>;
         else
             return a24_spmm_shared_b_kernel<NT, RB, W, RL, RM>;
@@ -833,8 +847,8 @@ int launch_shared_b(hipStream_t stream, const void* packed, const void* B, void*
     return static_cast<int>(hipGetLastError());
 }
 
-// rl: loads per residual list (0 = no residual).  The fused form has the library's own launch
-// shapes only: two row blocks per wave, four or eight waves.
+// rl: loads per residual list (0 = no residual; five and more: five, of the rounds of the longest list).  The fused form has
+// the library's own launch shapes only: two row blocks per wave, four or eight waves.
 template<int NT>
 int launch_shared_b_nt(hipStream_t s, const void* packed, const void* B, void* out, int M, int N, int K, int split_k, int rb,
                        int waves, long ldb, long ldo, long slab, int rl, const void* words, const void* offsets, int relu,
@@ -846,6 +860,16 @@ int launch_shared_b_nt(hipStream_t s, const void* packed, const void* B, void* o
     // straight into LDS where their granules are aligned; up to 16 tokens only with four waves (28672 x 7168 in
     // two batches, eight waves: 46.0 us through registers, 46.6 straight; four waves, one batch: 43.5, 43.1).
     const bool aligned = (reinterpret_cast<uintptr_t>(B) & 15) == 0 && (row_major || ldb % 8 == 0);
+    // (beyond five rounds and the three that are fetched in time: five, up to 32 tokens)
+    if constexpr (NT <= 2) {
+        if (aligned && rb == 2 && waves == 4 && rl > 8)
+            return row_major ? A24_GO(2, 4, 5, true, true, true) : A24_GO(2, 4, 5, false, true, true);
+        if constexpr (NT > 1) {
+            if (aligned && rb == 2 && waves == 8 && rl > 8)
+                return row_major ? A24_GO(2, 8, 5, true, true, true) : A24_GO(2, 8, 5, false, true, true);
+        }
+    }
+    rl = rl < 5 ? rl : 5;
 #define A24_STRAIGHT(W_, RL_)                             \
     if (aligned && rb == 2 && waves == W_ && rl == RL_) \
         return row_major ? A24_GO(2, W_, RL_, true, true) : A24_GO(2, W_, RL_, false, true);
@@ -917,8 +941,8 @@ int launch_nt(hipStream_t s, const void* packed, const void* B, void* out, int M
 // Batch b of ceil((K/128)/split_k) units writes fp16 [N][ldo] to out + b * slab.  The caller has
 // checked: M % (16 * rb) == 0 (share_b: M % (16 * rb * waves) == 0), K % 128 == 0, N in {8, 16, 32, 64}, no batch empty, pointers set.
 // residual_loads > 0 (share_b with rb == 2 only): the launch also multiplies the residual lists
-// words / offsets; residual_loads rounds of 64 words travel with the records, a longer list's rest is
-// fetched where it is needed.  relu (share_b only): negative
+// words / offsets, residual_loads rounds of 64 words the longest: up to five rounds travel with the records, a longer list's
+// rest is fetched where it is needed.  relu (share_b only): negative
 // results are written as zero (for a launch that writes the finished result).
 // fuse_page >= 0 (share_b, split_k > 1, ldo == M, slab == M * N): the launch adds its slabs up into
 // fused_out (token stride ldc) itself, counting arrivals on that page of the library's counters.

@@ -816,8 +816,7 @@ int fused_call(const char* who, void* stream, const void* Packed_A1, const void*
     // up to five rounds of 64 words travel with a unit's records; what a longer list holds beyond them
     // is fetched where it is needed (a24_kernels.hip)
     const int rounds = (LongestList + 63) / 64;
-    const int loads = rounds < HETERO_FUSED_PIPELINED_ROUNDS ? rounds : HETERO_FUSED_PIPELINED_ROUNDS;
-    const int waves = a24_waves(B, M > 0 ? M : 128, N, Split_K, loads, row_major);
+    const int waves = a24_waves(B, M > 0 ? M : 128, N, Split_K, rounds, row_major);
     if (!Packed_A1 || !A2_Words || !A2_Offsets || !B || !C || LongestList < 0 || LongestList > HETERO_FUSED_MAX_LIST
         || !a24_shape_ok(M, N, K, Split_K, 2, waves, 1) || (Split_K > 1 && !Reduction_Workspace) || ldb < K || ldc < M
         || ldb % 8 != 0 || ldc % 8 != 0 || (Flags & ~(SPMM_FLAG_RELU | SPMM_FLAG_SEPARATE_REDUCTION))) {
@@ -828,9 +827,9 @@ int fused_call(const char* who, void* stream, const void* Packed_A1, const void*
     const int relu = (Flags & SPMM_FLAG_RELU) ? 1 : 0;
     const long mn = static_cast<long>(M) * N;
     if (Split_K == 1)
-        return a24_launch_spmm(stream, Packed_A1, B, C, M, N, K, 1, 2, waves, 1, ldb, ldc, mn, loads, A2_Words, A2_Offsets, relu, -1,
+        return a24_launch_spmm(stream, Packed_A1, B, C, M, N, K, 1, 2, waves, 1, ldb, ldc, mn, rounds, A2_Words, A2_Offsets, relu, -1,
                                nullptr, 0, row_major ? 1 : 0);
-    return a24_split_call(stream, Packed_A1, B, ldb, C, ldc, M, N, K, Reduction_Workspace, Split_K, 2, waves, loads, A2_Words,
+    return a24_split_call(stream, Packed_A1, B, ldb, C, ldc, M, N, K, Reduction_Workspace, Split_K, 2, waves, rounds, A2_Words,
                           A2_Offsets, relu, (Flags & SPMM_FLAG_SEPARATE_REDUCTION) != 0, row_major);
 }
 

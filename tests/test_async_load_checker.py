@@ -200,3 +200,5 @@ def test_built_sparse_mfma_kernels_without_registers_for_the_tile_pass():
     r = subprocess.run([sys.executable, CHECKER, asm, "a24_spmm_straight_b_kernel"], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
     assert r.stdout.count("ok ") == (3 + 2) * 6 * 2
+    r = subprocess.run([sys.executable, CHECKER, asm, "a24_spmm_straight_long_kernel"], capture_output=True, text=True)
+    assert r.returncode == 0 and r.stdout.count("ok ") == 3 * 2, r.stdout  # lists beyond 512 words, up to 32 tokens
