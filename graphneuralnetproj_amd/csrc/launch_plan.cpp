@@ -162,11 +162,12 @@ bool complete_plan(int N, int K, int split_k, bool row_major, LaunchPlan& p)
 }
 
 // Two waves to a tile row where the row-sharing layout has three or four tile rows to a workgroup and a batch is long enough
-// to pay for the second barrier and the sum of the halves.  Measured on 60 calls, one wave to a row -> two: three rows,
-// column-major, 1.02 to 1.16 times as fast from four tiles a batch on (49152 x 12288 at 80 % 130 -> 119 us, at 60 % 216 ->
-// 177, at 90 % 106 -> 92; 0.97 to 0.99 with one or two tiles), row-major 1.05 to 1.4 (149 -> 119, 219 -> 175, 129 -> 93);
-// four rows, row-major, 1.01 to 1.33 from 20 tiles on (36864 x 9216 in three batches 82 -> 74), 0.97 to 1.08 below; four
-// rows, column-major, 0.98 to 1.04 at 60 to 80 %: left to one wave.
+// to pay for the second barrier and the sum of the halves.  One wave to a row -> two, on 177 calls
+// (profiles/two_waves_per_tile_row_64_tokens.txt): three rows, column-major, 1.01 to 1.25 times as fast from four tiles a batch
+// on (49152 x 12288 at 80 % 129 -> 115 us, at 60 % 215 -> 173, at 90 % 105 -> 91; 0.96 to 1.06 with one to three), row-major
+// 1.05 to 1.40 (146 -> 116, 217 -> 173, 128 -> 93; 0.95 to 1.03); four rows, row-major, 1.00 to 1.33 from 20 tiles on
+// (36864 x 9216 in three batches 80 -> 72), below 0.97 (70 % sparse in 11 or 18 tiles) to 1.27 (95 % in 15); four rows,
+// column-major, 0.98 to 1.04 at 60 to 80 % when it was tried: left to one wave.
 LaunchPlan with_two_waves(int N, int K, int split_k, bool row_major, const LaunchPlan& p)
 {
     const long tiles = (K / kTileCols - 1) / split_k + 1;

@@ -542,7 +542,9 @@ int a24_waves_for(int M, int split_k)
 // ... and for a call: B, the residual's rounds.  Where the activations go straight into LDS (aligned: a24_kernels.hip),
 // eight waves are better by 1 to 3 % as long as their workgroups run all at once, and four, two workgroups to a
 // compute unit, beyond (27648 x 9216 at 60 %, 64 tokens: two batches 74.2 us with eight, 75.6 with four; three batches
-// 97.9 and 82.6; seven 95.7 and 93.3) and for the longest lists at 64 tokens (50 %, two batches: 93.3 and 90.6).
+// 97.9 and 82.6; seven 95.7 and 93.3) and for the longest lists at 64 tokens (50 %, two batches: 93.3 and 90.6).  So at any
+// number of tokens: 312 calls at 8 to 64, 13 shapes, 50 to 70 %, both layouts, are 0.97 to 1.32 times as fast with four, 1.17
+// in the mean (profiles/a24_four_and_eight_waves.txt).
 // Where they come through registers, four waves for the longest lists at 64 tokens: what fits.
 int a24_waves(const void* B, int M, int N, int split_k, int rounds, bool row_major)
 {
@@ -563,7 +565,8 @@ A24Plan a24_default_plan(int M, int N, int K)
     // workgroups of eight waves or as many of four with half the slabs (FFN1 28672x7168, N = 16:
     // four waves, one batch, no reduction: 36.0 us against 35.2 + 3 us), else e.g. 432 rather than
     // 144 or 288.  With 64 tokens eight waves hide the matrix cores' and the LDS's latencies better
-    // (FFN1: 41 us + reduction against 46).
+    // (FFN1: 41 us + reduction against 46).  (A call with more workgroups of eight than run at once launches four where its
+    // activations are aligned, a24_waves: the estimate, of eight, is then too long by up to a quarter.)
     // Small matrices would run faster from more batches (256 x 1024 at 64 tokens, eight instead of one: 1.75
     // times), but a batch's partial sums are rounded to fp16: the error against 64 bits goes from 2.1e-4 to
     // 3.1e-4, which is the caller's to choose (any Split_K is taken), not this suggestion's.

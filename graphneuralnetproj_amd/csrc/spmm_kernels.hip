@@ -1173,19 +1173,20 @@ __global__ __launch_bounds__(2 * kWave, 2) void tcsl_spmm_pair_kernel(const int*
 // 64 tokens, ROWS tile rows to a workgroup and two waves to each: a wave takes all 128 rows and all tokens of one half of the
 // batch's tiles, and the two sums meet in LDS at the end.
 //
-// What bounds 64 tokens in the first kernel is the instruction issue of one wave to a SIMD (1744 of 2953 cycles a tile: 74 LDS
-// instructions, 64 MFMAs, the rest) with nothing beside it, and the activation fragments, a quarter of a line per lane and
-// load (512 of 614 accesses to the vector L1 a tile).  Multiplying a tile between the scatter instructions of the next one, in
-// one wave, gained nothing for the first reason (49152 x 12288 131 -> 142 us).  Two waves fit a SIMD at 256 registers: one set
+// What bounds 64 tokens in the first kernel is one wave to a SIMD with nothing beside it: 2828 cycles a tile, 1383 of them
+// issuing (72 LDS instructions 519, 115 of the vector unit with the 64 MFMAs 467), 649 waiting for data, 798 for the issue.
+// Here a compute unit spends 834 cycles on a tile instead of 943, and LDS instructions issue in 721 of them instead of 519:
+// that is the bound now (counters in profiles/two_waves_per_tile_row_counters.txt).  Multiplying a tile between the scatter
+// instructions of the next one, in one wave, made it slower.  Two waves fit a SIMD at 256 registers: one set
 // of words, fetched while the tile before it is multiplied, instead of a ring of two; no fragments in flight, because the ROWS
 // waves of a half share each activation tile through LDS, where it goes straight from memory in whole lines; and no addresses
 // kept to undo the scatter, except for small tiles: larger ones are cleared in whole lines.
 //
 // A barrier per kTiles tiles: in front of it each wave has waited for its share of the activations that its half reads next,
 // behind it nobody reads the ones before, and the next are fetched into their place.  Two tiles between barriers, where LDS has
-// the room, let the waves' memory latencies even out (126 -> 120 us).  Every wave of the workgroup takes the same number of steps;
+// the room, let the waves' memory latencies even out (5 % on the largest product).  Every wave of the workgroup takes the same number of steps;
 // an empty tile (or one past a half's end) is not multiplied.
-// Measured, and where it is used: launch_plan.cpp, with_two_waves.  The images are ROWS * 32 KiB of LDS, the activations kTiles * 32 KiB.
+// Where it is used, with times: launch_plan.cpp, with_two_waves.  The images are ROWS * 32 KiB of LDS, the activations kTiles * 32 KiB.
 constexpr int halves_tiles(int rows)  // tiles between two barriers
 {
     return rows < 4 ? 2 : 1;

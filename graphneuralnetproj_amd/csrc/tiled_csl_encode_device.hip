@@ -128,7 +128,7 @@ __device__ __forceinline__ int half_wave_reduce(int x, int neutral, Op op)
 //   * The words are stored past the caches (nt): whole lines that nothing here reads again (21504 x 7168 at 60 %: 111 us,
 //     now 97; the count kernel of the next weight 72 us, now 63).
 // (Bank lists staged in LDS, level sums by one thread over 260 levels, words stored one by one:
-// 303 us for a 28672 x 7168 weight at 80 %; 766 instructions per wave and tile: 124; now 109, 5.3 TB/s.  Alone, 21504 x 7168
+// 303 us for a 28672 x 7168 weight at 80 %; 766 instructions per wave and tile: 124; now 99 to 107 by the run.  Alone, 21504 x 7168
 // at 50 / 80 / 95 %: 157 / 97 / 88 us, now 132 / 77 / 70; 1024 x 1024 at 80 %: 5.3, now 4.9.)
 constexpr int kSeqWords = 4096, kPassWords = kSeqWords - 128;  // the first pass takes the tail's up to 124 pops as well
 
